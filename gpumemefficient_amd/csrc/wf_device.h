@@ -182,11 +182,10 @@ struct WfServeArgs {
     int32_t *pair_done;         // strips finished, per slot
 };
 
-// In-place table stencils swept with the same strip schedule (wf_stencil.hip):
-// the reference's summed-area table and one Gauss-Seidel SOR sweep.
-enum { WFS_SAT = 0, WFS_SOR = 1 };
+// In-place table stencils: one Gauss-Seidel SOR sweep with the same strip
+// schedule (wf_stencil.hip) and the summed-area table (wf_sat.hip).
 
-// Kernel argument block of a stencil sweep.  The table is row-major with
+// Kernel argument block of an SOR sweep.  The table is row-major with
 // pitch `ld` int32 (ld >= n1 + 3, ld % 4 == 0, 16-byte aligned base); rows
 // 0 and n2 + 1 and columns 0, n1 + 1, n1 + 2 are fixed boundary values and
 // the interior 1 <= y <= n2, 1 <= x <= n1 is updated in place.
@@ -195,9 +194,24 @@ struct WfStencilArgs {
     int64_t ld;
     int32_t n1, n2;
     int32_t nstrips;         // strips of 64 * waves rows
-    int32_t op;              // WFS_SAT / WFS_SOR
     uint64_t *bnd;           // (nstrips - 1) rows of n1 + 1 words: (epoch << 32) | value
     int32_t *counter;        // strip claim counter (zeroed by the reset kernel)
+    WfResultDev *res;        // res[0].status: timeout flag
+    const uint32_t *epoch;
+    int64_t timeout_ticks;
+};
+
+// Kernel argument block of a summed-area table (wf_sat.hip): the table as
+// above, in ntr x ntc tiles.
+enum { WFS_SAT_TILE_ROWS = 128, WFS_SAT_TILE_COLS = 512 };
+struct WfSatArgs {
+    int32_t *t;
+    int64_t ld;
+    int32_t n1, n2;
+    int32_t ntr, ntc;
+    uint64_t *rowsum;        // [ntr][ntc][WFS_SAT_TILE_ROWS] words (epoch << 32) | value: row sums of each tile
+    uint64_t *bottom;        // [ntr][ntc][WFS_SAT_TILE_COLS] words: each tile's finished bottom row
+    int32_t *counter;        // tile claim counter (zeroed by the reset kernel)
     WfResultDev *res;        // res[0].status: timeout flag
     const uint32_t *epoch;
     int64_t timeout_ticks;

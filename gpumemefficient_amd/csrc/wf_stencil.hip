@@ -1,10 +1,9 @@
-// wf_stencil.hip -- gfx950 wavefront engine for the reference's other users of
-// the hyperlane schedule: in-place sweeps over a whole int32 table whose cell
-// depends on its left and upper neighbours after they were updated.
+// wf_stencil.hip -- gfx950 wavefront engine for the reference's 2D-SOR
+// program: an in-place sweep over a whole int32 table whose cell depends on
+// its left and upper neighbours after they were updated.  (The reference's
+// other user of the hyperlane schedule, the summed-area table, is a prefix
+// sum and needs no wavefront: wf_sat.hip.)
 //
-//   SAT  summed-area table:
-//          T(y,x) = T(y,x-1) + T(y-1,x) + T(y,x) - T(y-1,x-1)
-//        (SAT/GPU_Hyperlane_Share.cu:169, :196, :233), int32 wrap-around.
 //   SOR  one Gauss-Seidel sweep of the 5-point stencil:
 //          T(y,x) = (T(y,x-1) + T(y-1,x) + T(y,x) + T(y,x+1) + T(y+1,x)) / 5
 //        with left and up already updated and right and down not
@@ -189,8 +188,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t interior_rsrc(const WfStencilA
 }
 
 // One chunk of kK steps from s0 for one wave.  `h` is the lane's last updated
-// value (its left neighbour), `dg` the upper neighbour of the previous step
-// (SAT's diagonal).  MASKED: some lane is outside its columns 1..n1 or holds
+// value (its left neighbour).  MASKED: some lane is outside its columns 1..n1 or holds
 // no interior row; those lanes keep their state and write nothing.
 //
 // The old values a group of 4 steps needs (own row: columns x..x+4; row
@@ -200,12 +198,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t interior_rsrc(const WfStencilA
 // LDS latency overlaps a group of arithmetic.  Reads may run past slot 127
 // into the mirror of slots 0..3 (old values, which is what they need);
 // writes always go to the slot itself.
-template <int OP, bool MASKED>
-__device__ __forceinline__ void st_chunk(int s0, int lane, int n1, bool rowok, int &h, int &dg, int *wrow,
+template <bool MASKED>
+__device__ __forceinline__ void st_chunk(int s0, int lane, int n1, bool rowok, int &h, int *wrow,
                                          const int *ring_prev, int *ring_cur, int *dummy)
 {
-    constexpr int NO = (OP == WFS_SOR) ? 5 : 4;  // own-row values per group
-    constexpr int ND = (OP == WFS_SOR) ? 4 : 1;  // row-below values per group (SAT: none)
+    constexpr int NO = 5;  // own-row values per group
+    constexpr int ND = 4;  // row-below values per group
     const int *__restrict__ inj_base = ring_prev + ((s0 + 64) & (kRS - 1));
     int *cap = (lane == 63) ? ring_cur + ((s0 + 1) & (kRS - 1)) : dummy + lane;
     int *cap_last = (lane == 63) ? ring_cur + ((s0 + kK) & (kRS - 1)) : dummy + lane + (kK - 1);
@@ -217,12 +215,8 @@ __device__ __forceinline__ void st_chunk(int s0, int lane, int n1, bool rowok, i
         const int p0 = (xb + q) & (kTW - 1);
 #pragma unroll
         for (int u = 0; u < NO; ++u) o[u] = wrow[p0 + u];
-        if (OP == WFS_SOR) {
 #pragma unroll
-            for (int u = 0; u < ND; ++u) d[u] = wrow[kTS + p0 + u];
-        } else {
-            d[0] = 0;
-        }
+        for (int u = 0; u < ND; ++u) d[u] = wrow[kTS + p0 + u];
     };
     load_ops(0, own, dn, inj4);
 #pragma unroll
@@ -238,21 +232,14 @@ __device__ __forceinline__ void st_chunk(int s0, int lane, int n1, bool rowok, i
             const int x = xb + j;
             const int self = own[u];
             const int up = __builtin_amdgcn_update_dpp(injv[u], h, kDppWaveShr1, 0xf, 0xf, false);
-            int nv;
-            if (OP == WFS_SAT) {
-                nv = (int)((uint32_t)h + (uint32_t)up + (uint32_t)self - (uint32_t)dg);
-            } else {
-                const int right = own[u + 1];
-                const int down = dn[u];
-                const int sum = (int)((uint32_t)h + (uint32_t)up + (uint32_t)self + (uint32_t)right +
-                                      (uint32_t)down);
-                nv = sum / 5;
-            }
+            const int right = own[u + 1];
+            const int down = dn[u];
+            const int sum = (int)((uint32_t)h + (uint32_t)up + (uint32_t)self + (uint32_t)right + (uint32_t)down);
+            const int nv = sum / 5;
             bool valid = true;
             if (MASKED) valid = rowok && (unsigned)(x - 1) < (unsigned)n1;
             if (valid) wrow[x & (kTW - 1)] = nv;
             h = valid ? nv : h;
-            dg = up;
             capv[u] = h;
         }
         // The group's ring captures together (adjacent slots: paired writes).
@@ -274,7 +261,7 @@ __device__ __forceinline__ void st_chunk(int s0, int lane, int n1, bool rowok, i
     }
 }
 
-template <int OP, int W>
+template <int W>
 __device__ void stencil_strip(const WfStencilArgs &a, int g, StShared<W> &sh, int lane, int wave, uint32_t epoch)
 {
     const int n1 = a.n1;
@@ -347,7 +334,6 @@ __device__ void stencil_strip(const WfStencilArgs &a, int g, StShared<W> &sh, in
     __syncthreads();
 
     int h = active ? wrow[0] : 0;  // column 0: the left boundary
-    int dg = 0;
     int copied = 0;  // wave W-1: bottom-row columns stored to bnext
     auto copy_out = [&](int upto, bool from_ring) {
         while (copied < upto) {
@@ -386,12 +372,11 @@ __device__ void stencil_strip(const WfStencilArgs &a, int g, StShared<W> &sh, in
         // of the previous chunk.
         stage_store(sg, win, cj + 1, lane);
         stage_load(sg, rs, a.ld, cj + 3, lane);
-        if (cj == 0 && lane == 0) dg = sh.ring[wave][63];  // column 0 of the row above
         const bool steady = nrows == 64 && s0 >= 63 && s0 + kK - 1 <= n1 - 1;
         if (steady)
-            st_chunk<OP, false>(s0, lane, n1, rowok, h, dg, wrow, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave]);
+            st_chunk<false>(s0, lane, n1, rowok, h, wrow, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave]);
         else
-            st_chunk<OP, true>(s0, lane, n1, rowok, h, dg, wrow, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave]);
+            st_chunk<true>(s0, lane, n1, rowok, h, wrow, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave]);
         // Steps < s0 + kK are done: lane 63 has finished columns < s0 + kK - 62,
         // so every lane has finished block cj-2.
         if (wave == W - 1 && has_next) copy_out(min(n1 + 1, s0 + kK - 62), true);
@@ -429,7 +414,7 @@ __device__ void stencil_strip(const WfStencilArgs &a, int g, StShared<W> &sh, in
         for (int b = max(0, nch - 2); 32 * b <= n1; ++b) flush_block(a, win, b, nrows, lane, outr);
 }
 
-template <int OP, int W>
+template <int W>
 __global__ __launch_bounds__(64 * W) void wf_stencil_kernel(WfStencilArgs a)
 {
     __shared__ StShared<W> sh;
@@ -445,30 +430,24 @@ __global__ __launch_bounds__(64 * W) void wf_stencil_kernel(WfStencilArgs a)
         const int g = __builtin_amdgcn_readfirstlane(sh.task);
         __syncthreads();
         if (g >= a.nstrips) break;
-        stencil_strip<OP, W>(a, g, sh, lane, wave, epoch);
+        stencil_strip<W>(a, g, sh, lane, wave, epoch);
         __syncthreads();
     }
 }
 
 }  // namespace wfs
 
-static const void *stencil_fn(int op, int waves)
+static const void *stencil_fn(int waves)
 {
-    if (op == WFS_SAT) {
-        if (waves == 1) return reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<WFS_SAT, 1>);
-        if (waves == 2) return reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<WFS_SAT, 2>);
-        if (waves == 4) return reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<WFS_SAT, 4>);
-    } else if (op == WFS_SOR) {
-        if (waves == 1) return reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<WFS_SOR, 1>);
-        if (waves == 2) return reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<WFS_SOR, 2>);
-        if (waves == 4) return reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<WFS_SOR, 4>);
-    }
-    return nullptr;
+    return waves == 1   ? reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<1>)
+           : waves == 2 ? reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<2>)
+           : waves == 4 ? reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<4>)
+                        : nullptr;
 }
 
-extern "C" int wf_stencil_resident(int op, int waves, int cus)
+extern "C" int wf_stencil_resident(int waves, int cus)
 {
-    const void *fn = stencil_fn(op, waves);
+    const void *fn = stencil_fn(waves);
     if (!fn) return 0;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * waves, 0) != hipSuccess || per_cu < 1) {
@@ -478,9 +457,9 @@ extern "C" int wf_stencil_resident(int op, int waves, int cus)
     return per_cu * cus;
 }
 
-extern "C" hipError_t wf_launch_stencil(int op, int waves, int grid, const WfStencilArgs *a, hipStream_t stream)
+extern "C" hipError_t wf_launch_stencil(int waves, int grid, const WfStencilArgs *a, hipStream_t stream)
 {
-    const void *fn = stencil_fn(op, waves);
+    const void *fn = stencil_fn(waves);
     if (!fn || grid <= 0) return hipErrorInvalidValue;
     void *args[] = {const_cast<WfStencilArgs *>(a)};
     return hipLaunchKernel(fn, dim3(grid), dim3(64 * waves), args, 0, stream);

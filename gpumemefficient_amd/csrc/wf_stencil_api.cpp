@@ -1,5 +1,6 @@
-// wf_stencil_api.cpp -- C ABI of the in-place table stencils (wf_stencil.hip):
-// the reference's summed-area table and 2D-SOR sweeps behind
+// wf_stencil_api.cpp -- C ABI of the in-place table stencils: the
+// reference's summed-area table (wf_sat.hip) and 2D-SOR sweep (wf_stencil.hip)
+// behind
 // void SOR(int n1, int n2, int *table[, int tX, int tY])
 // (SAT/GPU_Hyperlane_Share.h:5, 2D-SOR/nested_loop/GPU_Hyperlane_Share.h:5 and
 // the Cache headers).
@@ -22,9 +23,8 @@ int pick_waves(wf_ctx *ctx, const wf_tile *tile, int64_t n2, int *waves)
         // Four waves per strip: the sweep is bound by the chain of waves down
         // the table, and a hop between waves of one strip (three 32-step
         // chunks through LDS) is shorter than one between strips (through
-        // HBM), so taller strips win even with CUs left idle (2^15: 7.15 ms
-        // SAT / 7.69 ms SOR against 7.22 / 7.95 ms with 128-row strips;
-        // 2^14: 3.41 / 3.77 against 3.57 / 3.93).  Shorter strips only for
+        // HBM), so taller strips win even with CUs left idle (2^15: 7.69 ms
+        // against 7.95 ms with 128-row strips; 2^14: 3.77 against 3.93).  Shorter strips only for
         // tables of fewer than four strips.
         (void)ctx;
         w = 4;
@@ -34,11 +34,60 @@ int pick_waves(wf_ctx *ctx, const wf_tile *tile, int64_t n2, int *waves)
     return WF_OK;
 }
 
+// Reset, one launch and the wait of a sweep, timed with HIP events.
+template <class Launch>
+int run_timed(wf_ctx *ctx, WfArenas *ar, double *ms, Launch &&launch)
+{
+    if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
+    if (wf_launch_reset((WfResultDev *)ar->res.ptr, 1, (int32_t *)ar->counters.ptr, 2, (uint32_t *)ar->epoch.ptr,
+                        ctx->stream) != hipSuccess)
+        return WF_ERR_DEVICE;
+    if (launch() != hipSuccess) return WF_ERR_DEVICE;
+    if (hipEventRecord(ctx->ev1, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
+    if (hipEventSynchronize(ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
+    float f = 0.f;
+    if (hipEventElapsedTime(&f, ctx->ev0, ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
+    *ms = f;
+    WfResultDev r{};
+    if (hipMemcpy(&r, ar->res.ptr, sizeof(r), hipMemcpyDeviceToHost) != hipSuccess) return WF_ERR_DEVICE;
+    return r.status ? WF_ERR_TIMEOUT : WF_OK;
+}
+
+// The summed-area table: tiles instead of strips (wf_sat.hip).
+int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double *ms)
+{
+    WfArenas *ar = &ctx->scratch;
+    const int cus = ctx->prop.multiProcessorCount;
+    const int64_t ntc = (n1 + 1 + WFS_SAT_TILE_COLS - 1) / WFS_SAT_TILE_COLS;  // columns 0..n1
+    const int64_t tr = WFS_SAT_TILE_ROWS, ntr = (n2 + tr - 1) / tr;
+    int st;
+    if ((st = ar->bnd.ensure((size_t)(ntr * ntc * (tr + WFS_SAT_TILE_COLS)) * sizeof(uint64_t), true)) != WF_OK) return st;
+    if ((st = ar->res.ensure(sizeof(WfResultDev))) != WF_OK) return st;
+    if ((st = ar->counters.ensure(2 * sizeof(int32_t))) != WF_OK) return st;
+    if ((st = ar->epoch.ensure(sizeof(uint32_t), true)) != WF_OK) return st;
+    WfSatArgs a{};
+    a.t = dt;
+    a.ld = ld;
+    a.n1 = (int32_t)n1;
+    a.n2 = (int32_t)n2;
+    a.ntr = (int32_t)ntr;
+    a.ntc = (int32_t)ntc;
+    a.rowsum = (uint64_t *)ar->bnd.ptr;
+    a.bottom = a.rowsum + ntr * ntc * tr;
+    a.counter = (int32_t *)ar->counters.ptr;
+    a.res = (WfResultDev *)ar->res.ptr;
+    a.epoch = (const uint32_t *)ar->epoch.ptr;
+    a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
+    const int grid = (int)std::min<int64_t>(ntr * ntc, std::max(1, wf_sat_resident(cus)));
+    return run_timed(ctx, ar, ms, [&] { return wf_launch_sat(grid, &a, ctx->stream); });
+}
+
 // The sweep on a device table (pitch ld, ld % 4 == 0, 16-byte aligned).
 int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, int waves, double *ms)
 {
     *ms = 0.0;
     if (n1 == 0 || n2 == 0) return WF_OK;
+    if (op == WF_SAT) return run_sat(ctx, n1, n2, dt, ld, ms);
     WfArenas *ar = &ctx->scratch;
     const int64_t strips = (n2 + 64 * waves - 1) / (64 * waves);
     int st;
@@ -54,26 +103,14 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     a.n1 = (int32_t)n1;
     a.n2 = (int32_t)n2;
     a.nstrips = (int32_t)strips;
-    a.op = op;
     a.bnd = (uint64_t *)ar->bnd.ptr;
     a.counter = (int32_t *)ar->counters.ptr;
     a.res = (WfResultDev *)ar->res.ptr;
     a.epoch = (const uint32_t *)ar->epoch.ptr;
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
-    const int lim = wf_stencil_resident(op, waves, ctx->prop.multiProcessorCount);
+    const int lim = wf_stencil_resident(waves, ctx->prop.multiProcessorCount);
     const int grid = (int)std::min<int64_t>(strips, std::max(1, lim));
-    if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
-    if (wf_launch_reset(a.res, 1, a.counter, 2, (uint32_t *)ar->epoch.ptr, ctx->stream) != hipSuccess)
-        return WF_ERR_DEVICE;
-    if (wf_launch_stencil(op, waves, grid, &a, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
-    if (hipEventRecord(ctx->ev1, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
-    if (hipEventSynchronize(ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
-    float f = 0.f;
-    if (hipEventElapsedTime(&f, ctx->ev0, ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
-    *ms = f;
-    WfResultDev r{};
-    if (hipMemcpy(&r, ar->res.ptr, sizeof(r), hipMemcpyDeviceToHost) != hipSuccess) return WF_ERR_DEVICE;
-    return r.status ? WF_ERR_TIMEOUT : WF_OK;
+    return run_timed(ctx, ar, ms, [&] { return wf_launch_stencil(waves, grid, &a, ctx->stream); });
 }
 
 // Host table -> device copy of pitch ldd -> sweep -> host table (or only the
