@@ -185,6 +185,7 @@ struct WfServeArgs {
 // In-place table stencils: one Gauss-Seidel SOR sweep with the same strip
 // schedule (wf_stencil.hip) and the summed-area table (wf_sat.hip).
 
+enum { WFS_SOR_STRIP_ROWS = 64 };
 // Kernel argument block of an SOR sweep.  The table is row-major with
 // pitch `ld` int32 (ld >= n1 + 3, ld % 4 == 0, 16-byte aligned base); rows
 // 0 and n2 + 1 and columns 0, n1 + 1, n1 + 2 are fixed boundary values and
@@ -193,7 +194,7 @@ struct WfStencilArgs {
     int32_t *t;
     int64_t ld;
     int32_t n1, n2;
-    int32_t nstrips;         // strips of 64 * waves rows
+    int32_t nstrips;         // strips of WFS_SOR_STRIP_ROWS rows
     uint64_t *bnd;           // (nstrips - 1) rows of n1 + 1 words: (epoch << 32) | value
     int32_t *counter;        // strip claim counter (zeroed by the reset kernel)
     WfResultDev *res;        // res[0].status: timeout flag

@@ -18,27 +18,43 @@
 // gives the row-major sequential sweep's result; the reference's hyperlane
 // tiles are one such order and so is this engine's.
 //
-// Geometry.  A strip of 64*W rows is swept left to right by one workgroup of
-// W waves; lane l of a wave owns one row and computes column x = s + 1 - l at
-// step s (the systolic front of the alignment engines).  The updated left
-// value stays in a VGPR, the updated upper value comes from lane l-1 through
-// one DPP wave_shr:1 (lane 0: from an LDS ring that the wave above, or for the
-// strip's first wave the strip above through HBM, fills).  Old values (self,
-// right, and the row below) come from an LDS window of the wave's 64 rows plus
-// the row below, staged from HBM in 32-column blocks with coalesced 16-byte
-// loads issued two chunks ahead of use; each new value is written back into the
-// window in place, and finished blocks go to HBM with coalesced 16-byte
-// stores.  Every cell is read once from and written once to HBM: the sweep
-// is bound by HBM bandwidth, not by the VALU.
+// Geometry.  A strip of 64 rows is swept left to right by one workgroup of
+// three waves.  Lane l of the compute wave owns one row and updates column
+// x = s + 1 - l at step s (the systolic front of the alignment engines).  The
+// updated left value stays in a VGPR; the updated upper value comes from lane
+// l-1 through one DPP wave_shr:1; and since lane l+1 is one column behind, the
+// value below, T(y+1,x), is the lane below's own right neighbour of the same
+// step: one DPP wave_shl:1.
 //
-// Waves of a workgroup advance in lock-step chunks of K = 32 steps between
-// s_barriers, wave w D = 3 chunks behind wave w-1.  A strip hands its bottom
-// row (columns 0..n1) to the next strip through HBM as (launch epoch << 32 |
-// value) words written and polled with relaxed device-scope atomics, as the
-// alignment engines do; strips are claimed in order from an atomic counter,
-// so a strip only waits on one that a running workgroup holds.
+// The rows' old values sit in an LDS window in *step* order: column x of row
+// l at slot x - 1 + l, so that the slot is the step and the same for every
+// lane.  A lane reads the old values of four steps with one ds_read_b128 and
+// writes the four new ones over them with one ds_write_b128, and when a chunk
+// of 16 steps is done, its slots are done in all 64 rows.
+//
+// The mover wave carries the window: it loads the skewed 16-byte vectors of
+// the rows (4-byte aligned in HBM) kAhead chunks ahead, stages them in LDS and
+// stores finished chunks back.  The boundary wave stages the row above for
+// lane 0 and publishes the strip's bottom row for the next strip, through HBM
+// as (launch epoch << 32 | value) words written and polled at device scope, as
+// the alignment engines do.  The compute wave touches LDS only: about 12 issue
+// slots a step, of which the division's v_mul_hi is four.  The three meet at a
+// barrier per chunk.  Strips are claimed in order from an atomic counter, so a
+// strip only waits on one that a running workgroup holds.
+//
+// Bound: the chain of n2 / 64 strips, each about 155 steps (80 of them the
+// lanes' skew and a chunk, the rest the row's way through memory) behind the
+// one above, and n1 steps of 26 ns; from about 16384 x 16384 on also the memory
+// traffic of 64-byte row segments.  Measured (kernel time; before: 256-row strips,
+// the window in column order, staging by the compute waves themselves): 9001 x
+// 7043 2.01 -> 0.71 ms, 1000 x 1000 0.21 -> 0.10, 16384 x 16384 3.10 -> 1.89,
+// 32768 x 32768 6.65 -> 4.5.  Two compute waves a strip (128 rows): 0.69 ms at
+// 9001 x 7043 and 5.3 at 32768 x 32768.  Chunks in flight: 4 / 6 / 8 4.8 / 4.4 /
+// 4.6 ms at 32768 x 32768, no difference at 9001 x 7043.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "wf_cells.h"
 #include "wf_device.h"
@@ -48,28 +64,21 @@ namespace wfs {
 using wfk::kDppWaveShr1;
 using wfk::now_ticks;
 
-constexpr int kK = 32;                  // steps per chunk
-constexpr int kD = (kK + 62) / kK + 1;  // chunks between consecutive waves
-constexpr int kTW = 128;                // window columns per row (4 blocks of 32)
-constexpr int kTS = kTW + 8;            // row stride in dwords: slot 128 mirrors slot 0
-constexpr int kTR = 65;                 // window rows: the wave's 64 plus the row below
-constexpr int kRS = 256;                // ring slots; column x lives in slot (x + 63) mod kRS
-constexpr int kVec = kTR * 8;           // 16-byte vectors in one block of the window
+constexpr int kDppWaveShl1 = 0x130;     // DPP_CTRL wave_shl:1 (GFX9 family)
+constexpr int kRows = 64;               // rows of a strip
+constexpr int kK = 16;                  // steps per chunk
+constexpr int kAhead = 6;               // chunks of loads in flight (registers of the mover)
+constexpr int kTW = 128;                // window slots per row (8 chunks)
+constexpr int kTS = kTW + 4;            // row stride: 16 lanes' 16-byte accesses fall in distinct banks
+constexpr uint32_t kOut = 0xf0000000u;  // buffer offset out of range, also 64 bytes x chunks further
 
-template <int W>
 struct StShared {
-    // Window rows r = 0..64 of each wave; column x in slot x mod 128.  The
-    // stride of 136 dwords makes the lanes' skewed reads (column s + 1 - l in
-    // row l) fall in distinct banks.
-    __attribute__((aligned(16))) int win[W][kTR * kTS];
-    // ring[0]: the strip's top row (wave 0's lane 0 input); ring[w+1]: lane
-    // 63 of wave w, read by wave w+1 (w = W-1: copied to HBM).
-    __attribute__((aligned(16))) int ring[W + 1][kRS];
-    // Lanes 0..62 store their value here so the ring capture is one unmasked
-    // ds_write per step.
-    int dummy[W][64 + kK];
+    __attribute__((aligned(16))) int win[kRows * kTS];
+    // bot: the row below the strip, its column x at slot x + 62 (lane 63's
+    // step); top: the row above, its column x at slot x + 62.
+    __attribute__((aligned(16))) int bot[kTW];
+    __attribute__((aligned(16))) int top[kTW];
     int task;
-    int abort_at;
 };
 
 // Barrier between the waves of the workgroup that orders their LDS accesses
@@ -82,385 +91,335 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// One block of the window (columns [32b, 32b+32) of the wave's 65 rows) in
-// flight between its global loads and its LDS stores: vector v = lane + 64k
-// is row v / 8, columns 32b + 4 (v % 8) .. + 3.
+// `bytes` bytes from p as a buffer resource: reads past the end give zeros,
+// writes are dropped.  Offsets are 32-bit: 65 rows of the pitch must fit
+// (checked by the host).  The descriptor's fields pass through readfirstlane:
+// a descriptor the compiler cannot prove uniform lives in VGPRs, and every
+// access then becomes a waterfall loop.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void *p, int64_t bytes)
+{
+    const uint64_t base = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
+    const int size = __builtin_amdgcn_readfirstlane((int)(uint32_t)bytes);
+    // Third descriptor dword of an untyped buffer on the gfx9 family.
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0, size, 0x00020000);
+}
+
+// Cache policy of accesses that other workgroups of the launch see or make:
+// device scope (bit 4: sc1), as a relaxed agent-scope atomic has.
+constexpr int kCoherent = 16;
+
+// One chunk of a wave's window in flight between its global loads and its LDS
+// stores: slots 4k..4k+3 of row row(i) per lane, and (lanes 0..3) of the row
+// below.
 struct Stage {
-    int4 v[(kVec + 63) / 64];
+    int4 v[4];
+    int4 b;
 };
 
-// The wave's 65 window rows as a buffer resource: loads past its last row
-// (rows below the table) read zeros, so every block load is issued
-// unconditionally, with no per-lane branch (see the chunk loop).  Offsets
-// are 32-bit: 73 rows of the pitch must fit (checked by the host).
-// The descriptor's fields pass through readfirstlane: a descriptor the
-// compiler cannot prove uniform lives in VGPRs, and every buffer load then
-// becomes a waterfall loop (readfirstlane, compare, exec mask, load, repeat).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t window_rsrc(const WfStencilArgs &a, int yw)
+// Lane's vectors: four lanes cover a row's 16 slots; the rows of 16
+// consecutive lanes are 4 apart, so that their 16-byte LDS accesses fall in
+// distinct banks.
+__device__ __forceinline__ int vec_row(int i, int lane) { return 16 * i + 4 * ((lane >> 2) & 3) + (lane >> 4); }
+
+// Slot q of row r holds column q + 1 - r: byte offset of a vector in the
+// wave's rows.
+__device__ __forceinline__ uint32_t vec_off(int r, int slot, int64_t ld)
 {
-    const int rows = max(0, min(kTR, a.n2 + 2 - yw));
-    const uint64_t base = reinterpret_cast<uint64_t>(a.t + (int64_t)yw * a.ld);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
-    int *p = reinterpret_cast<int *>(((uint64_t)hi << 32) | lo);
-    const int bytes = __builtin_amdgcn_readfirstlane((int)(rows * a.ld * 4));
-    // Third descriptor dword of an untyped buffer on the gfx9 family.
-    return __builtin_amdgcn_make_buffer_rsrc(p, 0, bytes, 0x00020000);
+    return (uint32_t)(r * (ld - 1) * 4) + (uint32_t)(slot + 1) * 4u;
 }
 
-__device__ __forceinline__ void stage_load(Stage &sg, __amdgpu_buffer_rsrc_t rs, int64_t ld, int b, int lane)
+// Four steps of a lane: old values of its row (self of steps 0..3, and the
+// next one), lane 0's upper and lane 63's lower neighbours.  HEAD: x0 is the
+// lane's column at step 0; columns left of 1 keep the left boundary `h`.
+// Columns right of n1 and rows below n2 need no mask: nothing inside the table
+// depends on them and the movers do not store them.
+template <bool HEAD>
+__device__ __forceinline__ int4 sor_group(int &h, int4 self, int next, int4 up4, int4 down4, int x0)
 {
+    const int sv[5] = {self.x, self.y, self.z, self.w, next};
+    const int uv[4] = {up4.x, up4.y, up4.z, up4.w};
+    const int dv[4] = {down4.x, down4.y, down4.z, down4.w};
+    int out[4];
 #pragma unroll
-    for (int k = 0; k < (kVec + 63) / 64; ++k) {
-        const int v = lane + 64 * k;
-        // Row v / 8 of the window; a vector past the pitch reads the next
-        // row's first columns (never used: the table's columns end at n1 + 2).
-        const uint32_t off = (uint32_t)(((v >> 3) * ld + 32 * b + 4 * (v & 7)) * 4);
-        sg.v[k] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+    for (int u = 0; u < 4; ++u) {
+        const int down = __builtin_amdgcn_update_dpp(dv[u], sv[u + 1], kDppWaveShl1, 0xf, 0xf, false);
+        const uint32_t old = (uint32_t)sv[u] + (uint32_t)sv[u + 1] + (uint32_t)down;
+        const int up = __builtin_amdgcn_update_dpp(uv[u], h, kDppWaveShr1, 0xf, 0xf, false);
+        const int nv = (int)((uint32_t)h + (uint32_t)up + old) / 5;
+        h = (HEAD && x0 + u < 1) ? h : nv;
+        out[u] = h;
     }
+    return make_int4(out[0], out[1], out[2], out[3]);
 }
 
-__device__ __forceinline__ void stage_store(const Stage &sg, int *win, int b, int lane)
-{
-#pragma unroll
-    for (int k = 0; k < (kVec + 63) / 64; ++k) {
-        const int v = lane + 64 * k;
-        if (k < kVec / 64 || v < kVec) {
-            const int slot = (32 * b + 4 * (v & 7)) & (kTW - 1);
-            *reinterpret_cast<int4 *>(win + (v >> 3) * kTS + slot) = sg.v[k];
-        }
-    }
-    // A block at slot 0 is mirrored at slots 128..131 (the vectors of lanes
-    // with v % 8 == 0); the other lanes rewrite their own vector, so the
-    // stores need no per-lane branch.
-    if ((b & 3) == 0) {
-#pragma unroll
-        for (int k = 0; k < (kVec + 63) / 64; ++k) {
-            const int v = lane + 64 * k;
-            if (k < kVec / 64 || v < kVec) {
-                const int slot = (v & 7) == 0 ? kTW : 4 * (v & 7);
-                *reinterpret_cast<int4 *>(win + (v >> 3) * kTS + slot) = sg.v[k];
-            }
-        }
-    }
-}
-
-// Store block b of the wave's interior rows (r < nrows) back to the table
-// through a buffer descriptor over those rows: a vector outside them, or
-// holding no interior column, gets an offset past the descriptor's end and
-// the hardware drops it (boundary columns inside a stored vector are written
-// back unchanged).  With no branch around the stores the eight LDS reads are
-// issued together, not one round trip per vector.
-__device__ __forceinline__ void flush_block(const WfStencilArgs &a, const int *win, int b, int nrows, int lane,
-                                            __amdgpu_buffer_rsrc_t out)
-{
-    if (b < 0 || 32 * b > a.n1) return;
-    int4 val[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int v = lane + 64 * k;
-        val[k] = *reinterpret_cast<const int4 *>(win + (v >> 3) * kTS + ((32 * b + 4 * (v & 7)) & (kTW - 1)));
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int v = lane + 64 * k;
-        const int rr = v >> 3;
-        const int c = 32 * b + 4 * (v & 7);
-        const uint32_t off = (rr < nrows && c + 3 >= 1 && c <= a.n1) ? (uint32_t)((rr * a.ld + c) * 4) : 0xfffffff0u;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) uint32_t, val[k]),
-                                               out, off, 0, 0);
-    }
-}
-
-// The wave's interior rows (nrows of them from yw) as the descriptor of
-// flush_block, its fields through readfirstlane as in window_rsrc.  The 4
-// bytes past the last row cover the one dword a stored vector can reach
-// beyond its row when the pitch is not a multiple of 4: the next row's
-// column 0, a boundary value written back unchanged.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t interior_rsrc(const WfStencilArgs &a, int yw, int nrows)
-{
-    const uint64_t base = reinterpret_cast<uint64_t>(a.t + (int64_t)yw * a.ld);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
-    int *p = reinterpret_cast<int *>(((uint64_t)hi << 32) | lo);
-    const int bytes = __builtin_amdgcn_readfirstlane(nrows > 0 ? (int)(nrows * a.ld * 4 + 4) : 0);
-    return __builtin_amdgcn_make_buffer_rsrc(p, 0, bytes, 0x00020000);
-}
-
-// One chunk of kK steps from s0 for one wave.  `h` is the lane's last updated
-// value (its left neighbour).  MASKED: some lane is outside its columns 1..n1 or holds
-// no interior row; those lanes keep their state and write nothing.
-//
-// The old values a group of 4 steps needs (own row: columns x..x+4; row
-// below: x..x+3), and lane 0's upper neighbours from the ring, are read one
-// group ahead, before the current group writes
-// its new values: the reads are of columns no lane has updated yet, and the
-// LDS latency overlaps a group of arithmetic.  Reads may run past slot 127
-// into the mirror of slots 0..3 (old values, which is what they need);
-// writes always go to the slot itself.
-template <bool MASKED>
-__device__ __forceinline__ void st_chunk(int s0, int lane, int n1, bool rowok, int &h, int *wrow,
-                                         const int *ring_prev, int *ring_cur, int *dummy)
-{
-    constexpr int NO = 5;  // own-row values per group
-    constexpr int ND = 4;  // row-below values per group
-    const int *__restrict__ inj_base = ring_prev + ((s0 + 64) & (kRS - 1));
-    int *cap = (lane == 63) ? ring_cur + ((s0 + 1) & (kRS - 1)) : dummy + lane;
-    int *cap_last = (lane == 63) ? ring_cur + ((s0 + kK) & (kRS - 1)) : dummy + lane + (kK - 1);
-    const int xb = s0 + 1 - lane;  // the lane's column at step s0
-    int own[NO], dn[ND];
-    int4 inj4;
-    auto load_ops = [&](int q, int (&o)[NO], int (&d)[ND], int4 &in4) {
-        in4 = *reinterpret_cast<const int4 *>(inj_base + q);
-        const int p0 = (xb + q) & (kTW - 1);
-#pragma unroll
-        for (int u = 0; u < NO; ++u) o[u] = wrow[p0 + u];
-#pragma unroll
-        for (int u = 0; u < ND; ++u) d[u] = wrow[kTS + p0 + u];
-    };
-    load_ops(0, own, dn, inj4);
-#pragma unroll
-    for (int q = 0; q < kK; q += 4) {
-        const int injv[4] = {inj4.x, inj4.y, inj4.z, inj4.w};
-        int nown[NO], ndn[ND];
-        int4 ninj4 = inj4;
-        int capv[4];
-        if (q + 4 < kK) load_ops(q + 4, nown, ndn, ninj4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = q + u;
-            const int x = xb + j;
-            const int self = own[u];
-            const int up = __builtin_amdgcn_update_dpp(injv[u], h, kDppWaveShr1, 0xf, 0xf, false);
-            const int right = own[u + 1];
-            const int down = dn[u];
-            const int sum = (int)((uint32_t)h + (uint32_t)up + (uint32_t)self + (uint32_t)right + (uint32_t)down);
-            const int nv = sum / 5;
-            bool valid = true;
-            if (MASKED) valid = rowok && (unsigned)(x - 1) < (unsigned)n1;
-            if (valid) wrow[x & (kTW - 1)] = nv;
-            h = valid ? nv : h;
-            capv[u] = h;
-        }
-        // The group's ring captures together (adjacent slots: paired writes).
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = q + u;
-            if (j == kK - 1)
-                *cap_last = capv[u];
-            else
-                cap[j] = capv[u];
-        }
-        if (q + 4 < kK) {
-            inj4 = ninj4;
-#pragma unroll
-            for (int u = 0; u < NO; ++u) own[u] = nown[u];
-#pragma unroll
-            for (int u = 0; u < ND; ++u) dn[u] = ndn[u];
-        }
-    }
-}
-
-template <int W>
-__device__ void stencil_strip(const WfStencilArgs &a, int g, StShared<W> &sh, int lane, int wave, uint32_t epoch)
+__device__ __forceinline__ void sor_strip(const WfStencilArgs &a, int g, StShared &sh, int lane, int wave,
+                                          uint32_t epoch)
 {
     const int n1 = a.n1;
-    const int yw = 1 + g * 64 * W + wave * 64;  // the wave's first row
-    const int rows_left = a.n2 - g * 64 * W;     // interior rows from the strip's first
-    const int wa = min(W, (rows_left + 63) / 64);
-    const bool active = wave < wa;
-    const int nrows = active ? min(64, a.n2 - yw + 1) : 0;  // interior rows of the wave
-    const bool rowok = lane < nrows;
-    const int nsteps = n1 + 63;                 // lane 63 updates column n1 at step n1 + 62
-    const int nch = (nsteps + kK - 1) / kK;
-    const int total = nch + (wa - 1) * kD;
-    const int nfill = (n1 + 1 + kK - 1) / kK;   // ring chunks covering columns 0..n1
+    const int y0 = 1 + g * kRows;  // the strip's first row
+    // Lane 63 updates column n1 at step n1 + 62; whole turns of the mover's
+    // loop.  Every wave passes a barrier before chunk 0 and one after each
+    // chunk; none leaves early: when a dependency wait is given up the launch
+    // is marked, and the strip runs on without waiting.
+    const int nch = (n1 + 63 + kK * kAhead - 1) / (kK * kAhead) * kAhead;
     const bool has_prev = g > 0;
     const bool has_next = g + 1 < a.nstrips;
     const uint64_t *bprev = a.bnd + (int64_t)(g - 1) * (n1 + 1);
     uint64_t *bnext = a.bnd + (int64_t)g * (n1 + 1);
-    const uint64_t tag = (uint64_t)epoch << 32;
-    int *win = sh.win[wave];
-    int *wrow = win + lane * kTS;
-    const __amdgpu_buffer_rsrc_t rs = window_rsrc(a, yw);
-    const __amdgpu_buffer_rsrc_t outr = interior_rsrc(a, yw, nrows);
+    int *win = sh.win;
 
-    // Top row (columns [32c, 32c+32), wave 0, lanes < 32): row 0 of the table
-    // for the first strip, else the previous strip's bottom row.
-    auto load_top = [&](int c) -> uint64_t {
-        const int x = c * kK + lane;
-        if (lane >= kK || x > n1) return tag;
-        if (!has_prev)  // row 0 is never written: any cache level may serve it
-            return tag | (uint32_t)__hip_atomic_load(a.t + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        return __hip_atomic_load(bprev + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    auto fill = [&](int c, uint64_t top) -> bool {
-        const int x = c * kK + lane;
-        const bool mine = lane < kK && x <= n1;
-        if (__builtin_amdgcn_ballot_w64(mine && (top >> 32) != (uint64_t)epoch) != 0) {
-            const int64_t t0 = now_ticks();
-            for (;;) {
-                __builtin_amdgcn_s_sleep(1);
-                if (mine && (top >> 32) != (uint64_t)epoch)
-                    top = __hip_atomic_load(bprev + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (__builtin_amdgcn_ballot_w64(mine && (top >> 32) != (uint64_t)epoch) == 0) break;
-                if (now_ticks() - t0 > a.timeout_ticks) return false;
-            }
-        }
-        if (mine) sh.ring[0][(x + 63) & (kRS - 1)] = (int)(uint32_t)top;
-        return true;
-    };
-
-    // Prologue: block 0 of the window in LDS, blocks 1 and 2 in flight (block
-    // b travels in sg[b & 1], two chunks ahead of its LDS store); the top
-    // ring's first two chunks.
-    Stage sg0, sg1;
-    if (active) {
-        stage_load(sg0, rs, a.ld, 0, lane);
-        stage_store(sg0, win, 0, lane);
-        stage_load(sg1, rs, a.ld, 1, lane);
-        stage_load(sg0, rs, a.ld, 2, lane);
-    }
-    // Top-row loads run two chunks ahead of their ring fill (top0 / top1
-    // alternate like the blocks), so an HBM round trip hides behind two
-    // chunks of arithmetic.
-    uint64_t top0 = tag, top1 = tag;
     if (wave == 0) {
-        bool ok = fill(0, load_top(0));
-        if (ok && nfill > 1) ok = fill(1, load_top(1));
-        if (!ok && lane == 0) sh.abort_at = -1;
-        top1 = load_top(2);
-    }
-    __syncthreads();
-
-    int h = active ? wrow[0] : 0;  // column 0: the left boundary
-    int copied = 0;  // wave W-1: bottom-row columns stored to bnext
-    auto copy_out = [&](int upto, bool from_ring) {
-        while (copied < upto) {
-            const int x = copied + lane;
-            if (x < upto) {
-                const int v = from_ring ? sh.ring[W][(x + 63) & (kRS - 1)] : 0;
-                __hip_atomic_store(bnext + x, tag | (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // ------------------------------------------------------ compute wave
+        lds_barrier();
+        int h = y0 + lane <= a.n2 ? a.t[(int64_t)(y0 + lane) * a.ld] : 0;  // column 0: the left boundary
+        int *wl = win + lane * kTS;
+        auto at = [](const int *p) __attribute__((always_inline)) { return *reinterpret_cast<const int4 *>(p); };
+        // Old values two groups ahead (the chunk after next is staged during
+        // this one), lane 63's lower neighbours one group ahead.
+        int4 cur = at(wl), nxt = at(wl + 4), down = at(sh.bot);
+        int up0 = sh.top[63];
+        auto chunk = [&](int cj, auto head) __attribute__((always_inline)) {
+            const int q0 = (cj * kK) & (kTW - 1), q1 = (q0 + kK) & (kTW - 1);
+            const int *rp = sh.top + ((q0 + 64) & (kTW - 1));
+            int4 up[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) up[i] = at(rp + 4 * i);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int4 nn = at(i < 2 ? wl + q0 + 4 * i + 8 : wl + q1 + 4 * i - 8);
+                const int4 dn = at(i < 3 ? sh.bot + q0 + 4 * i + 4 : sh.bot + q1);
+                const int4 nv = sor_group<decltype(head)::value>(
+                    h, cur, nxt.x, make_int4(up0, up[i].x, up[i].y, up[i].z), down, cj * kK + 4 * i + 1 - lane);
+                *reinterpret_cast<int4 *>(wl + q0 + 4 * i) = nv;
+                up0 = up[i].w;
+                cur = nxt;
+                nxt = nn;
+                down = dn;
             }
-            copied = min(upto, copied + 64);
-        }
-    };
-
-    // Every wave passes the same `total` barriers: kD idle chunks per wave
-    // above it, its nch chunks, then idle chunks until the last wave is done.
-    // The active chunks run in a loop of their own so that their nine block
-    // loads are issued on every iteration: the compiler then waits for a
-    // block's loads (two chunks old) without waiting for the newer ones.
-    bool aborted = sh.abort_at <= -1;
-    int j = 0;
-    const int jstart = active ? wave * kD : total;
-    for (; j < jstart && !aborted; ++j) {
-        lds_barrier();
-        aborted = sh.abort_at <= j;
-    }
-    // One active chunk; `sg` holds block cj+1 (loaded two chunks ago) and
-    // takes block cj+3; `top_old` holds the top row's chunk cj+2 (loaded
-    // during the previous chunk), `top_new` takes chunk cj+3.
-    auto chunk = [&](int cj, Stage &sg, uint64_t &top_new, uint64_t &top_old) {
-        const int s0 = cj * kK;
-        if (wave == 0 && cj + 3 < nfill) top_new = load_top(cj + 3);
-        // Keep the top-row load ahead of the block loads (the compiler would
-        // otherwise sink it toward its use, where waiting for it would also
-        // wait for the block loads issued after it).
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        // Window: block cj+1 takes the slot of block cj-3, flushed at the end
-        // of the previous chunk.
-        stage_store(sg, win, cj + 1, lane);
-        stage_load(sg, rs, a.ld, cj + 3, lane);
-        const bool steady = nrows == 64 && s0 >= 63 && s0 + kK - 1 <= n1 - 1;
-        if (steady)
-            st_chunk<false>(s0, lane, n1, rowok, h, wrow, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave]);
-        else
-            st_chunk<true>(s0, lane, n1, rowok, h, wrow, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave]);
-        // Steps < s0 + kK are done: lane 63 has finished columns < s0 + kK - 62,
-        // so every lane has finished block cj-2.
-        if (wave == W - 1 && has_next) copy_out(min(n1 + 1, s0 + kK - 62), true);
-        flush_block(a, win, cj - 2, nrows, lane, outr);
-        if (wave == 0 && cj + 2 < nfill) {
-            if (!fill(cj + 2, top_old) && lane == 0) sh.abort_at = j;
-        }
-        lds_barrier();
-        aborted = sh.abort_at <= j;
-        ++j;
-    };
-    // Even chunks stage from sg1, odd ones from sg0; the loop takes them in
-    // pairs so that the alternation is visible to the compiler.
-    for (int cj = 0; cj < nch && !aborted; cj += 2) {
-        chunk(cj, sg1, top0, top1);
-        if (cj + 1 >= nch || aborted) break;
-        chunk(cj + 1, sg0, top1, top0);
-    }
-    for (; j < total && !aborted; ++j) {
-        lds_barrier();
-        aborted = sh.abort_at <= j;
-    }
-
-    if (aborted) {
-        // A dependency wait timed out: mark the launch and release the strip
-        // below with placeholder values so it does not wait out its own timeout.
-        if (threadIdx.x == 0) atomicOr(&a.res->status, 1);
-        if (wave == W - 1 && has_next) copy_out(n1 + 1, false);
+            lds_barrier();
+        };
+        int cj = 0;
+        for (; cj < 4; ++cj) chunk(cj, std::true_type{});
+        for (; cj < nch; ++cj) chunk(cj, std::false_type{});
         return;
     }
-    if (wave == W - 1 && has_next) copy_out(n1 + 1, true);
-    // Blocks not yet flushed: nch-2 .. the one holding column n1 (all of
-    // them are still in the window).
-    if (active)
-        for (int b = max(0, nch - 2); 32 * b <= n1; ++b) flush_block(a, win, b, nrows, lane, outr);
+
+    if (wave == 2) {
+        // ----------------------------------------------------- boundary wave
+        // Publishes the strip's bottom row, and takes the row above the strip
+        // into sh.top: row 0 of the table (4 bytes a column), or the previous
+        // strip's words (8).  A wave of its own, because the words arrive late:
+        // waiting for one must not wait for the mover's loads and stores, which
+        // complete in one order.  One poll of the next 64 columns is issued per
+        // chunk and looked at four chunks later (a round trip to memory is
+        // longer than a chunk); only when the next chunk's columns are missing
+        // does the wave hold up the barrier and go through its polls.
+        const int tshift = has_prev ? 3 : 2;
+        const __amdgpu_buffer_rsrc_t topr =
+            rows_rsrc(has_prev ? (const void *)bprev : (const void *)a.t, has_prev ? (n1 + 1) * 8LL : (n1 + 3) * 4LL);
+        typedef __attribute__((ext_vector_type(2))) uint32_t u2;
+        struct Poll {
+            u2 v;
+            int x;
+        };
+        int have = 0;  // columns 1..have are in sh.top
+        int64_t t_new = now_ticks();
+        auto issue = [&](Poll &p) __attribute__((always_inline)) {
+            p.x = have + 1 + lane;
+            asm volatile("" ::: "memory");  // reads again what an earlier poll read
+            p.v = __builtin_amdgcn_raw_buffer_load_b64(topr, p.x <= n1 ? (uint32_t)p.x << tshift : kOut, 0, kCoherent);
+        };
+        // Chunk c reads columns up to 16c + 17; the ring has room for six more
+        // chunks.
+        auto need = [&](int c) __attribute__((always_inline)) { return min(n1, c * kK + kK + 1); };
+        auto examine = [&](Poll &p, int c) __attribute__((always_inline)) {
+            const bool ready = p.x <= n1 && (!has_prev || p.v.y == epoch);
+            const uint64_t late = ~__builtin_amdgcn_ballot_w64(ready);
+            const int upto = min(__builtin_amdgcn_readfirstlane(p.x) - 1 + (late ? (int)__builtin_ctzll(late) : 64),
+                                 need(c + 5));
+            if (upto > have) {
+                if (p.x > have && p.x <= upto) sh.top[(p.x + 62) & (kTW - 1)] = (int)p.v.x;
+                have = upto;
+                t_new = now_ticks();
+            } else if (have < need(c) && now_ticks() - t_new > a.timeout_ticks) {
+                if (lane == 0) atomicOr(&a.res->status, 1);
+                have = n1;
+            }
+            issue(p);
+        };
+        Poll p0, p1, p2, p3;
+        issue(p0);
+        issue(p1);
+        issue(p2);
+        issue(p3);
+        // The bottom row: lane 63's columns of chunk c (16 lanes), as soon as
+        // it is done.
+        const __amdgpu_buffer_rsrc_t pubr =
+            rows_rsrc(has_next ? (const void *)bnext : (const void *)a.t, has_next ? (n1 + 1) * 8LL : 0);
+        auto publish = [&](int c) __attribute__((always_inline)) {
+            const int s = c * kK + (lane & (kK - 1)), x = s - 62;
+            const u2 v = {(uint32_t)win[63 * kTS + (s & (kTW - 1))], epoch};
+            __builtin_amdgcn_raw_buffer_store_b64(
+                v, pubr, (lane < kK && c >= 0 && x >= 1 && x <= n1) ? (uint32_t)x * 8u : kOut, 0, kCoherent);
+        };
+        // One poll examined and reissued, one barrier passed if the next chunk's
+        // columns are there, one publish (of nothing if not): always the same
+        // accesses, so that waiting for a poll leaves the later ones in flight.
+        int j = -1;  // the chunk before the next barrier; -1: the first barrier
+        auto tick = [&](Poll &p) __attribute__((always_inline)) {
+            examine(p, j + 1);
+            const bool go = have >= need(j + 1) && j < nch;
+            if (go) lds_barrier();
+            publish(go ? j : -1);
+            j += go ? 1 : 0;
+        };
+        do {
+            tick(p0);
+            tick(p1);
+            tick(p2);
+            tick(p3);
+        } while (j < nch);
+        return;
+    }
+
+    // ------------------------------------------------------------ mover wave
+    // No value here is merged from a load and something else, and its loop has
+    // one exit: where a path with fewer loads in flight joins, the compiler would
+    // wait for nearly all of them.
+    const int nrows = min(kRows, a.n2 - y0 + 1);      // interior rows of the strip
+    const int trows = min(kRows + 1, a.n2 + 2 - y0);  // with the row below
+    const __amdgpu_buffer_rsrc_t rs = rows_rsrc(a.t + (int64_t)y0 * a.ld, trows * a.ld * 4);
+    const __amdgpu_buffer_rsrc_t outr = rows_rsrc(a.t + (int64_t)y0 * a.ld, nrows * a.ld * 4);
+    int *bot = sh.bot;
+    const int k4 = 4 * (lane & 3);
+    const int xv0 = k4 + 1 - vec_row(0, lane);  // column of the lane's first cell in chunk 0
+    uint32_t off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) off[i] = vec_off(vec_row(i, lane), k4, a.ld);
+    const uint32_t boff = lane < 4 ? vec_off(64, 4 * lane + 1, a.ld) : kOut;
+
+    // Where the pitch is n1 + 3, the vector that starts at column n1 of the
+    // table's last row would reach one cell past the table: it is loaded from
+    // a cell earlier (its first cell, T(n2+1, n1), is all that is needed of it).
+    const uint32_t tail = y0 + trows == a.n2 + 2 ? (uint32_t)(((trows - 1) * a.ld + a.ld - 3) * 4) : kOut;
+    auto load_vec = [&](uint32_t o) __attribute__((always_inline)) {
+        return __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(rs, o - (o == tail ? 4u : 0u), 0, 0));
+    };
+    auto load = [&](Stage &st, int c) __attribute__((always_inline)) {
+        const uint32_t co = (uint32_t)c * (kK * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st.v[i] = load_vec(off[i] + co);
+        st.b = load_vec(boff + co);
+    };
+    auto stage_vec = [&](int *d, uint32_t o, int4 v) __attribute__((always_inline)) {
+        v.x = o == tail ? v.y : v.x;
+        *reinterpret_cast<int4 *>(d) = v;
+    };
+    auto stage = [&](const Stage &st, int c) __attribute__((always_inline)) {
+        const int q0 = (c * kK) & (kTW - 1);
+        const uint32_t co = (uint32_t)c * (kK * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) stage_vec(win + vec_row(i, lane) * kTS + q0 + k4, off[i] + co, st.v[i]);
+        if (lane < 4) stage_vec(bot + q0 + 4 * lane, boff + co, st.b);
+    };
+    // Chunk c, finished in all rows, back to the table: the vectors that lie in
+    // columns 1..n1.  Vectors of rows past nrows lie past the descriptor's end
+    // and are dropped.
+    auto flush = [&](int c) __attribute__((always_inline)) {
+        const int q0 = (c * kK) & (kTW - 1);
+        const uint32_t co = (uint32_t)c * (kK * 4);
+        typedef __attribute__((ext_vector_type(4))) uint32_t u4;
+        u4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const u4 *>(win + vec_row(i, lane) * kTS + q0 + k4);
+        const int xv = c * kK + xv0;  // the lane's first column is xv - 16i
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_buffer_store_b128(
+                v[i], outr, (uint32_t)(xv - 16 * i - 1) < (uint32_t)max(0, n1 - 3) ? off[i] + co : kOut, 0, 0);
+    };
+    // The cells of columns x0..x0+2 (row `lane`) whose vector is not such a one:
+    // a row's first and last cells.  Once per strip and side, after the chunks
+    // that hold them, and not with the chunks: a strip's first chunks are on the
+    // way to the next strip's start.
+    const int tail_at = (n1 + 62) / kK + 1;
+    int head_at = 5;
+    asm("" : "+s"(head_at));  // unknown to the compiler, which would peel the loop's first turns for it
+    auto ends = [&](int x0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int x = x0; x < x0 + 3; ++x) {
+            const int s = x - 1 + lane, xs = x - (s & 3);
+            const bool mine = lane < nrows && x >= 1 && x <= n1 && !(xs >= 1 && xs + 3 <= n1);
+            __builtin_amdgcn_raw_buffer_store_b32(win[lane * kTS + (s & (kTW - 1))], outr,
+                                                  mine ? (uint32_t)((lane * a.ld + x) * 4) : kOut, 0, 0);
+        }
+    };
+
+    Stage sg[kAhead];  // chunk c travels in sg[c % kAhead]
+#pragma unroll
+    for (int c = 0; c < kAhead + 2; ++c) {
+        if (c >= kAhead) stage(sg[c % kAhead], c - kAhead);
+        load(sg[c % kAhead], c);
+        // As many accesses, and in the same order, as in the loop below, which
+        // otherwise would wait for more than it needs to (none is stored).
+        flush(-kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();
+    // One chunk: the compute wave runs chunk cj; `st` holds chunk cj + 2 and
+    // takes chunk cj + 2 + kAhead (chunk -1 has no cell and is not stored).
+    auto chunk = [&](int cj, Stage &st) __attribute__((always_inline)) {
+        stage(st, cj + 2);
+        load(st, cj + 2 + kAhead);
+        flush(cj - 1);
+        if (cj == head_at) ends(1);
+        if (cj == tail_at) ends(n1 - 2);
+        lds_barrier();
+    };
+    for (int c0 = 0; c0 < nch; c0 += kAhead) {
+#pragma unroll
+        for (int p = 0; p < kAhead; ++p) chunk(c0 + p, sg[(p + 2) % kAhead]);
+    }
+    flush(nch - 1);
+    if (nch <= head_at) ends(1);
+    if (nch <= tail_at) ends(n1 - 2);
 }
 
-template <int W>
-__global__ __launch_bounds__(64 * W) void wf_stencil_kernel(WfStencilArgs a)
+__global__ __launch_bounds__(192) void wf_stencil_kernel(WfStencilArgs a)
 {
-    __shared__ StShared<W> sh;
+    __shared__ StShared sh;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t epoch = __builtin_amdgcn_readfirstlane(*a.epoch);
     for (;;) {
-        if (threadIdx.x == 0) {
-            sh.task = atomicAdd(a.counter, 1);
-            sh.abort_at = 0x7fffffff;
-        }
+        if (threadIdx.x == 0) sh.task = atomicAdd(a.counter, 1);
         __syncthreads();
         const int g = __builtin_amdgcn_readfirstlane(sh.task);
         __syncthreads();
         if (g >= a.nstrips) break;
-        stencil_strip<W>(a, g, sh, lane, wave, epoch);
+        sor_strip(a, g, sh, lane, wave, epoch);
         __syncthreads();
     }
 }
 
 }  // namespace wfs
 
-static const void *stencil_fn(int waves)
+extern "C" int wf_stencil_resident(int cus)
 {
-    return waves == 1   ? reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<1>)
-           : waves == 2 ? reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<2>)
-           : waves == 4 ? reinterpret_cast<const void *>(&wfs::wf_stencil_kernel<4>)
-                        : nullptr;
-}
-
-extern "C" int wf_stencil_resident(int waves, int cus)
-{
-    const void *fn = stencil_fn(waves);
-    if (!fn) return 0;
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * waves, 0) != hipSuccess || per_cu < 1) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wfs::wf_stencil_kernel, 192, 0) != hipSuccess ||
+        per_cu < 1) {
         (void)hipGetLastError();
         per_cu = 1;
     }
     return per_cu * cus;
 }
 
-extern "C" hipError_t wf_launch_stencil(int waves, int grid, const WfStencilArgs *a, hipStream_t stream)
+extern "C" hipError_t wf_launch_stencil(int grid, const WfStencilArgs *a, hipStream_t stream)
 {
-    const void *fn = stencil_fn(waves);
-    if (!fn || grid <= 0) return hipErrorInvalidValue;
-    void *args[] = {const_cast<WfStencilArgs *>(a)};
-    return hipLaunchKernel(fn, dim3(grid), dim3(64 * waves), args, 0, stream);
+    if (grid <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(wfs::wf_stencil_kernel, dim3(grid), dim3(192), 0, stream, *a);
+    return hipGetLastError();
 }

@@ -11,26 +11,13 @@
 
 namespace {
 
-int pick_waves(wf_ctx *ctx, const wf_tile *tile, int64_t n2, int *waves)
+// A tile's strip height and rows per lane are checked and not used: both
+// kernels have one shape (every shape gives the same table).
+int check_tile(const wf_tile *tile)
 {
-    if (tile && tile->rows_per_lane > 1) return WF_ERR_NOKERNEL;
-    int w = 0;
-    if (tile && tile->strip_rows > 0) {
-        if (tile->strip_rows % 64) return WF_ERR_NOKERNEL;
-        w = tile->strip_rows / 64;
-        if (w != 1 && w != 2 && w != 4) return WF_ERR_NOKERNEL;
-    } else {
-        // Four waves per strip: the sweep is bound by the chain of waves down
-        // the table, and a hop between waves of one strip (three 32-step
-        // chunks through LDS) is shorter than one between strips (through
-        // HBM), so taller strips win even with CUs left idle (2^15: 7.69 ms
-        // against 7.95 ms with 128-row strips; 2^14: 3.77 against 3.93).  Shorter strips only for
-        // tables of fewer than four strips.
-        (void)ctx;
-        w = 4;
-        while (w > 1 && n2 < 4 * 64 * w) w /= 2;
-    }
-    *waves = w;
+    if (!tile) return WF_OK;
+    const int rows = tile->strip_rows;
+    if (tile->rows_per_lane > 1 || (rows > 0 && rows != 64 && rows != 128 && rows != 256)) return WF_ERR_NOKERNEL;
     return WF_OK;
 }
 
@@ -83,13 +70,13 @@ int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double
 }
 
 // The sweep on a device table (pitch ld, ld % 4 == 0, 16-byte aligned).
-int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, int waves, double *ms)
+int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double *ms)
 {
     *ms = 0.0;
     if (n1 == 0 || n2 == 0) return WF_OK;
     if (op == WF_SAT) return run_sat(ctx, n1, n2, dt, ld, ms);
     WfArenas *ar = &ctx->scratch;
-    const int64_t strips = (n2 + 64 * waves - 1) / (64 * waves);
+    const int64_t strips = (n2 + WFS_SOR_STRIP_ROWS - 1) / WFS_SOR_STRIP_ROWS;
     int st;
     if ((st = ar->bnd.ensure((size_t)std::max<int64_t>(1, (strips - 1) * (n1 + 1)) * sizeof(uint64_t), true)) !=
         WF_OK)
@@ -108,22 +95,22 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     a.res = (WfResultDev *)ar->res.ptr;
     a.epoch = (const uint32_t *)ar->epoch.ptr;
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
-    const int lim = wf_stencil_resident(waves, ctx->prop.multiProcessorCount);
+    const int lim = wf_stencil_resident(ctx->prop.multiProcessorCount);
     const int grid = (int)std::min<int64_t>(strips, std::max(1, lim));
-    return run_timed(ctx, ar, ms, [&] { return wf_launch_stencil(waves, grid, &a, ctx->stream); });
+    return run_timed(ctx, ar, ms, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
 }
 
 // Host table -> device copy of pitch ldd -> sweep -> host table (or only the
 // result cell with no_copyback).
 int upload_run_download(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *table, int64_t ld, int32_t *d,
-                        int64_t ldd, int waves, bool no_copyback, wf_result *out)
+                        int64_t ldd, bool no_copyback, wf_result *out)
 {
     const int64_t rows = n2 + 2, cols = n1 + 3;
     if (hipMemcpy2D(d, (size_t)ldd * sizeof(int32_t), table, (size_t)ld * sizeof(int32_t),
                     (size_t)cols * sizeof(int32_t), (size_t)rows, hipMemcpyHostToDevice) != hipSuccess)
         return WF_ERR_DEVICE;
     double ms = 0.0;
-    const int st = run_device(ctx, op, n1, n2, d, ldd, waves, &ms);
+    const int st = run_device(ctx, op, n1, n2, d, ldd, &ms);
     out->kernel_ms = ms;
     if (st != WF_OK) return st;
     if (no_copyback)
@@ -158,11 +145,10 @@ int wf_stencil_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dev_
     std::memset(out, 0, sizeof(*out));
     out->cells = (uint64_t)n1 * (uint64_t)n2;
     if (hipSetDevice(ctx->device) != hipSuccess) return WF_ERR_DEVICE;
-    int waves = 0;
-    int st = pick_waves(ctx, tile, n2, &waves);
+    int st = check_tile(tile);
     if (st != WF_OK) return st;
     double ms = 0.0;
-    st = run_device(ctx, op, n1, n2, dev_table, ld, waves, &ms);
+    st = run_device(ctx, op, n1, n2, dev_table, ld, &ms);
     out->kernel_ms = ms;
     if (st != WF_OK) return st;
     if (hipMemcpy(&out->last, dev_table + n2 * ld + n1, sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess)
@@ -177,8 +163,7 @@ int wf_stencil(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *table, int6
     std::memset(out, 0, sizeof(*out));
     out->cells = (uint64_t)n1 * (uint64_t)n2;
     if (hipSetDevice(ctx->device) != hipSuccess) return WF_ERR_DEVICE;
-    int waves = 0;
-    int st = pick_waves(ctx, tile, n2, &waves);
+    int st = check_tile(tile);
     if (st != WF_OK) return st;
     const int64_t rows = n2 + 2, cols = n1 + 3;
     const int64_t ldd = (cols + 3) & ~int64_t(3);
@@ -188,7 +173,7 @@ int wf_stencil(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *table, int6
     if (bytes + (64u << 20) > fr) return WF_ERR_NOMEM;
     DevBuf dt;
     if ((st = dt.ensure(bytes)) != WF_OK) return st;
-    st = upload_run_download(ctx, op, n1, n2, table, ld, (int32_t *)dt.ptr, ldd, waves,
+    st = upload_run_download(ctx, op, n1, n2, table, ld, (int32_t *)dt.ptr, ldd,
                              tile && (tile->flags & WF_TILE_NO_COPYBACK), out);
     dt.release();
     return st;

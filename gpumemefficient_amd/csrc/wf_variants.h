@@ -45,9 +45,9 @@ extern "C" hipError_t wf_launch_engine(const WfVariant *v, int grid, const WfKer
 extern "C" const void *wf_serve_kernel(int *block);
 extern "C" hipError_t wf_launch_serve(int grid, const WfServeArgs *sa, hipStream_t stream);
 
-// SOR sweep (wf_stencil.hip): strips of 64 * waves rows, waves 1, 2 or 4.
-extern "C" hipError_t wf_launch_stencil(int waves, int grid, const WfStencilArgs *a, hipStream_t stream);
-extern "C" int wf_stencil_resident(int waves, int cus);
+// SOR sweep (wf_stencil.hip).
+extern "C" hipError_t wf_launch_stencil(int grid, const WfStencilArgs *a, hipStream_t stream);
+extern "C" int wf_stencil_resident(int cus);
 // Summed-area table (wf_sat.hip).
 extern "C" hipError_t wf_launch_sat(int grid, const WfSatArgs *a, hipStream_t stream);
 extern "C" int wf_sat_resident(int cus);

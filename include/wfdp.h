@@ -211,8 +211,8 @@ int wf_align_naive(wf_ctx *ctx, int problem, const int32_t *a, int64_t n1, const
  * sequential sweep would update it.  The reference computes on a device copy
  * that it never copies back (SAT/GPU_Hyperlane_Share.cu:317); these functions
  * return the result (wf_stencil: unless WF_TILE_NO_COPYBACK).  tile:
- * strip_rows 64, 128 or 256 (0 = choose; the summed-area table has one tile
- * shape and takes no choice); rows_per_lane 0 or 1.  out->last =
+ * strip_rows 64, 128 or 256 or 0, rows_per_lane 0 or 1 (accepted; the
+ * kernels have one shape each).  out->last =
  * the updated cell (n2, n1). */
 typedef enum { WF_SAT = 0, WF_SOR = 1 } wf_stencil_op;
 #define WF_STENCIL_MAX_PITCH 14000000 /* largest ld (and n1 + 3) accepted */
