@@ -463,6 +463,27 @@ constexpr int64_t kSplitMinCols = 1024;
 // SW pairs narrower than this are not split (measured gains of the split:
 // 13% at 1024 x 1024, 17% at 2048 x 2048, 30% at 3000 x 600).
 constexpr int64_t kSwSplitMinCols = 1024;
+// Narrowest pair that is split in two or three parts (without f0, WfSplitDev)
+// where three or four have more strips than the chip has CUs.
+constexpr int64_t kSwTwoPartMinCols = 16384;
+
+// Columns where the strips of a column-split SW pair are cut (WfSplitDev):
+// strip g sweeps columns 1..c[g] forward and, reversed, the rest.  A strip
+// starts a lag after the strip above it (the strip below, reversed), so with
+// c falling by the lag from strip to strip both sweeps' strips all end at step
+// (n1 + (G - 1) lag) / 2, against n1 / 2 + (G - 1) lag with a straight cut.  The
+// lag of a 512-row strip is 13.2 us, 580 steps of 22.7 ns (16384 columns, 512 to
+// 32768 rows, unsplit); 640 steps gave the shortest runs at every size (lags of
+// 0 / 432 / 580 / 640 / 704: 8192^2 0.323 / 0.286 / 0.252 / 0.239 / 0.239 ms,
+// 32768^2 1.26 / 1.09 / 0.945 / 0.890 / 0.914 ms; with the maximum likewise).
+static std::vector<int32_t> sw_cuts(int64_t n1, int64_t n2, int64_t strip, int waves)
+{
+    const int64_t G = (n2 + strip - 1) / strip, lag = 160 * waves;
+    std::vector<int32_t> c((size_t)G);
+    for (int64_t g = 0; g < G; ++g)
+        c[g] = (int32_t)std::min(n1, std::max<int64_t>(0, (n1 + (G - 1) * lag) / 2 - g * lag));
+    return c;
+}
 
 int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile,
                   WfPlanHost *ph, int64_t max_groups)
@@ -490,9 +511,10 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     // finish in about half of it.
     std::vector<int64_t> mid(njobs, 0);
     std::vector<uint8_t> swsplit(njobs, 0);
+    bool two_part = false;  // SW splits without the part `f0` (WfSplitDev)
     std::vector<std::vector<uint8_t>> trial;  // SW split candidates' codes (a then b) and modes
     std::vector<int32_t> trial_mode;
-    int64_t nsplit = 0, nextra = 0;
+    int64_t nextra = 0;
     if (bitpar && split_enabled()) {
         int64_t strips = 0;
         for (int64_t i = 0; i < njobs; ++i)
@@ -502,14 +524,13 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
             for (int64_t i = 0; i < njobs; ++i)
                 if (jobs[i].n1 >= kSplitMinCols && jobs[i].n2 > 0) {
                     mid[i] = jobs[i].n1 / 2;
-                    ++nsplit;
+                    ++nextra;
                 }
-        nextra = nsplit;
     } else if (v->engine == WF_ENGINE_ASYNC && perm4 && split_enabled()) {
         // SW pairs on the byte tables split in three (bottom-right cell
-        // only) or four (with the running maximum) pairs of half the columns
-        // (WfSplitDev) when all of the launch's strips fit on the chip at
-        // once: the halves' strip chains run side by side.
+        // only) or four (with the running maximum) pairs (WfSplitDev) when all
+        // of the launch's strips fit on the chip at once: the parts' strip
+        // chains run side by side.
         int64_t strips = 0, extra = 0;
         std::vector<uint8_t> cand(njobs, 0);
         trial.resize(njobs);
@@ -532,25 +553,31 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
             cand[i] = nomax ? 2 : 3;  // extra pairs
             extra += cand[i] * si;
         }
-        // A split pays while every strip has a CU of its own.  Beyond that
-        // only three pairs of a launch of one pair still do, whose strips
-        // start staggered along one long chain (SW 65536², 384 strips on
-        // 256 CUs: 3.18 -> 3.03 ms); four pairs do not (with the maximum,
-        // 512 strips: 3.62 -> 4.27 ms), nor a batch, whose strips all run at
-        // once (16 pairs of 4096², 384 strips: 0.27 ms against 0.21).
+        // Three or four parts while every strip has a CU of its own.  Beyond
+        // that, a launch of one wide pair takes two or three parts, whose
+        // strips share CUs only towards the end (no maximum: 131072 x 65536
+        // 2.60 ms against 2.98 in three parts and 4.47 with a straight cut;
+        // 131072^2 4.74 against 6.55 unsplit; with it: 65536^2 2.02 against
+        // 3.62 unsplit), and a narrow one without the maximum three parts
+        // (4096 x 44032, 258 strips: 0.66 ms, unsplit 1.24).  A batch, whose
+        // strips all run at once, is not split beyond a strip per CU (16 pairs
+        // of 4096^2, 384 strips: 0.27 ms against 0.21 unsplit).
         const bool four = std::find(cand.begin(), cand.end(), 3) != cand.end();
         const int64_t cus = ctx ? ctx->prop.multiProcessorCount : 256;
-        const int64_t room = std::min({ctx ? (int64_t)wf_max_resident_groups(ctx, v) : 256,
-                                       (four || njobs > 1) ? cus : INT64_MAX,
-                                       max_groups > 0 ? max_groups : INT64_MAX});
-        if (extra > 0 && strips + extra <= room)
+        const int64_t resident = std::min(ctx ? (int64_t)wf_max_resident_groups(ctx, v) : 256,
+                                          max_groups > 0 ? max_groups : INT64_MAX);
+        const bool wide = njobs == 1 && cand[0] && jobs[0].n1 >= kSwTwoPartMinCols;
+        if (extra > 0 && strips + extra <= std::min(resident, (four || njobs > 1 || wide) ? cus : INT64_MAX)) {
             for (int64_t i = 0; i < njobs; ++i)
                 if (cand[i]) {
-                    mid[i] = jobs[i].n1 / 2;
                     swsplit[i] = cand[i];
-                    ++nsplit;
                     nextra += cand[i];
                 }
+        } else if (wide && cand[0] * strips <= resident) {
+            swsplit[0] = cand[0];
+            two_part = true;
+            nextra = cand[0] - 1;
+        }
     }
     const int64_t np = njobs + nextra;
     ph->njobs = njobs;
@@ -560,13 +587,14 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     ph->host_only.assign(np, 0);
     ph->cells.assign(np, 0);
     ph->splits.clear();
+    ph->cuts.clear();
     ph->colw_entries = 0;
     for (int64_t i = 0; i < njobs; ++i) ph->cells[i] = (uint64_t)(jobs[i].n1 * jobs[i].n2);
 
     // Codes: a then b per pair, 16-byte aligned; a split pair's reverse half
     // gets its own reversed copies after all jobs.
     int64_t code_bytes = 0, bnd_ints = 0;
-    auto place = [&](WfPairDev &p, int prob, int64_t n1, int64_t n2, int64_t a_bytes) {
+    auto place_codes = [&](WfPairDev &p, int prob, int64_t n1, int64_t n2, int64_t a_bytes) {
         p.prob = prob;
         p.n1 = (int32_t)n1;
         p.n2 = (int32_t)n2;
@@ -575,6 +603,9 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
         p.b_off = code_bytes;
         code_bytes += (n2 + 15) & ~15LL;
         p.ngroups = (int32_t)((n2 + strip - 1) / strip);
+    };
+    auto place = [&](WfPairDev &p, int prob, int64_t n1, int64_t n2, int64_t a_bytes) {
+        place_codes(p, prob, n1, n2, a_bytes);
         p.bnd_off = bnd_ints;
         bnd_ints += (int64_t)(p.ngroups - 1) * n1;
     };
@@ -594,42 +625,86 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
             p.ngroups = 0;
             continue;
         }
-        place(p, j.problem, mid[i] ? mid[i] : j.n1, j.n2, j.n1);
+        if (swsplit[i])
+            place_codes(p, j.problem, j.n1, j.n2, j.n1);
+        else
+            place(p, j.problem, mid[i] ? mid[i] : j.n1, j.n2, j.n1);
     }
     {
         int64_t r = njobs;
         for (int64_t i = 0; i < njobs; ++i) {
-            if (!mid[i]) continue;
+            if (!mid[i] && !swsplit[i]) continue;
             const wf_job &j = jobs[i];
             if (swsplit[i]) {
-                // Right half from a zero boundary (pair r), reversed right
-                // half (pair r + 1) and, with the running maximum, the
-                // clamped reversed right half (pair r + 2); the left and
-                // the reversed halves keep their last column.
-                const int64_t nr = j.n1 - mid[i];
-                for (int k = 0; k < swsplit[i]; ++k) place(ph->pairs[r + k], j.problem, nr, j.n2, nr);
+                // Right part from a zero boundary (pair r), reversed right
+                // part (pair r + 1) and, with the running maximum, the
+                // clamped reversed right part (pair r + 2); the left and the
+                // reversed parts keep their last columns.
+                const std::vector<int32_t> c = sw_cuts(j.n1, j.n2, strip, v->waves);
+                const int64_t G = (int64_t)c.size(), pad = G * strip - j.n2;
+                const int32_t base = c.back(), n1 = (int32_t)j.n1;
+                const int64_t ir = r + (two_part ? 0 : 1);  // the reversed part's pair
+                WfPairDev &f = ph->pairs[i], &rv = ph->pairs[ir];
+                f.n1 = c[0];
+                place_codes(rv, WFK_SW, n1 - base, G * strip, n1 - base);
                 WfSplitDev sp{};
                 sp.job = (int32_t)i;
-                sp.rev = (int32_t)(r + 1);
+                sp.rev = (int32_t)ir;
                 sp.prob = WFK_SW;
                 sp.n2 = (int32_t)j.n2;
-                sp.f0 = (int32_t)r;
-                sp.r0 = (int32_t)nr;
-                const int64_t entries = (j.n2 + 1) / 2;  // two words per entry, one per row
-                ph->pairs[i].col_off = ph->colw_entries;
-                sp.fwd_off = ph->colw_entries;
-                ph->colw_entries += entries;
-                ph->pairs[r + 1].col_off = ph->colw_entries;
-                sp.rev_off = ph->colw_entries;
-                ph->colw_entries += entries;
+                sp.f0 = two_part ? -1 : (int32_t)r;
+                sp.r0 = n1;
+                sp.strip = (int32_t)strip;
+                sp.pad = (int32_t)pad;
+                auto cut_pair = [&](WfPairDev &p, auto &&of) {
+                    p.cut = (int32_t)ph->cuts.size();
+                    for (int64_t g = 0; g < G; ++g) {
+                        WfCutDev cd = of(g);
+                        cd.bnd = bnd_ints;
+                        if (g + 1 < G) bnd_ints += cd.n;
+                        ph->cuts.push_back(cd);
+                    }
+                };
+                auto keep_columns = [&](WfPairDev &p, int64_t rows) {
+                    const int64_t at = ph->colw_entries;
+                    p.col_off = at;
+                    ph->colw_entries += (rows + 1) / 2;  // two words per entry, one per row
+                    return at;
+                };
+                cut_pair(f, [&](int64_t g) { return WfCutDev{0, 0, c[g], 0, 0, 0, 0}; });
+                if (!two_part) {
+                    WfPairDev &p0 = ph->pairs[r];
+                    p0.prob = WFK_SW;
+                    p0.n1 = n1 - base;
+                    p0.n2 = (int32_t)j.n2;
+                    p0.a_off = f.a_off + base;
+                    p0.b_off = f.b_off;
+                    p0.ngroups = f.ngroups;
+                    cut_pair(p0, [&](int64_t g) {
+                        return WfCutDev{0, c[g] - base, n1 - c[g], g ? c[g - 1] - base : 0, 0, 0, 0};
+                    });
+                }
+                // Strip k of the reversed parts is strip G - 1 - k; the first
+                // one is filled up with rows without a symbol.
+                auto reversed = [&](int64_t k) {
+                    return WfCutDev{0, 0, n1 - c[G - 1 - k], 0,
+                                    k == 0 ? (int32_t)(pad / (64 * v->rows_per_lane)) : 0, (int32_t)pad, 0};
+                };
+                cut_pair(rv, reversed);
+                sp.cut = f.cut;
+                sp.rcut = rv.cut;
+                sp.fwd_off = keep_columns(f, j.n2);
+                sp.rev_off = keep_columns(rv, G * strip);
                 if (swsplit[i] == 3) {
-                    sp.crev = (int32_t)(r + 2);
-                    ph->pairs[r + 2].col_off = ph->colw_entries;
-                    sp.crev_off = ph->colw_entries;
-                    ph->colw_entries += entries;
+                    WfPairDev &cv = ph->pairs[ir + 1];
+                    cv = rv;
+                    sp.crev = (int32_t)(ir + 1);
+                    cut_pair(cv, reversed);
+                    sp.ccut = cv.cut;
+                    sp.crev_off = keep_columns(cv, G * strip);
                 }
                 ph->splits.push_back(sp);
-                r += swsplit[i];
+                r += swsplit[i] - (two_part ? 1 : 0);
                 continue;
             }
             place(ph->pairs[r], j.problem, j.n1 - mid[i], j.n2, j.n1 - mid[i]);
@@ -672,30 +747,21 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     }
     for (WfSplitDev &sp : ph->splits) {
         if (sp.prob == WFK_SW) {
-            // Right half: a[mid..n1) and b as they are, the pair's modes;
-            // reverse half: both reversed, the unclamped recurrence.
+            // Reversed parts: the right part of a and b reversed, b behind
+            // its rows without a symbol; the unclamped recurrence, and the
+            // clamped one for the running maximum.
             const wf_job &j = jobs[sp.job];
             const WfPairDev &f = ph->pairs[sp.job];
-            WfPairDev &rp = ph->pairs[sp.f0];
             WfPairDev &rv = ph->pairs[sp.rev];
-            const int64_t m = mid[sp.job], nr = sp.r0;
-            const uint8_t *fa = ph->codes.data() + f.a_off;
-            const uint8_t *fb = ph->codes.data() + f.b_off;
-            std::memcpy(ph->codes.data() + rp.a_off, fa + m, (size_t)nr);
-            std::memcpy(ph->codes.data() + rp.b_off, fb, (size_t)j.n2);
-            uint8_t *ra = ph->codes.data() + rv.a_off;
-            uint8_t *rb = ph->codes.data() + rv.b_off;
-            reverse_codes(fa + m, nr, ra);
-            reverse_codes(fb, j.n2, rb);
-            rp.mode = f.mode;
-            rv.mode = (f.mode & (WFK_MODE_PERM4 | WFK_MODE_FREE_HEAD)) | WFK_MODE_NOMAX | WFK_MODE_SWE;
             if (!(f.mode & WFK_MODE_PERM4) || !(f.mode & WFK_MODE_NOMAX) != (sp.crev >= 0)) return WF_ERR_INVALID;
-            if (sp.crev >= 0) {
-                WfPairDev &cv = ph->pairs[sp.crev];
-                std::memcpy(ph->codes.data() + cv.a_off, ra, (size_t)nr);
-                std::memcpy(ph->codes.data() + cv.b_off, rb, (size_t)j.n2);
-                cv.mode = (f.mode & (WFK_MODE_PERM4 | WFK_MODE_FREE_HEAD)) | WFK_MODE_NOMAX;
-            }
+            uint8_t *codes = ph->codes.data();
+            reverse_codes(codes + f.a_off + (j.n1 - rv.n1), rv.n1, codes + rv.a_off);
+            std::memset(codes + rv.b_off, WFK_NO_SYMBOL, (size_t)sp.pad);
+            reverse_codes(codes + f.b_off, j.n2, codes + rv.b_off + sp.pad);
+            const int32_t mode = (f.mode & (WFK_MODE_PERM4 | WFK_MODE_FREE_HEAD)) | (two_part ? 0 : WFK_MODE_NOMAX);
+            if (sp.f0 >= 0) ph->pairs[sp.f0].mode = f.mode;
+            rv.mode = mode | WFK_MODE_SWE;
+            if (sp.crev >= 0) ph->pairs[sp.crev].mode = mode;
             continue;
         }
         // Reverse half: a[mid..n1) and b reversed, textbook ED boundary (its
@@ -747,11 +813,31 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     ph->tasks.clear();
     ph->task_begin.assign(np, 0);
     ph->task_end.assign(np, 0);
+    // The parts of a two-part split are one entry of the list, strip by strip:
+    // the early strips of all parts, which run from the start, are then claimed
+    // by the first workgroup of each CU and the late ones by the second (SW
+    // 131072^2, 512 strips: 4.74 ms, part by part 5.88).  Not so the other
+    // splits, whose f0 strips all start at once (65536^2, 384 strips: 1.74 ms
+    // part by part, 2.94 strip by strip).
+    std::vector<std::vector<int32_t>> parts(np);
+    std::vector<int64_t> owner(np);
+    std::iota(owner.begin(), owner.end(), 0);
+    for (int64_t i = 0; i < np; ++i) parts[i].push_back((int32_t)i);
+    if (two_part)
+        for (const WfSplitDev &sp : ph->splits)
+            for (int32_t p : {sp.rev, sp.crev})
+                if (p >= 0) {
+                    parts[sp.job].push_back(p);
+                    owner[p] = sp.job;
+                }
     for (int64_t k = 0; k < np; ++k) {
-        const int64_t i = order[k];
+        const int64_t i = owner[order[k]];
+        if (parts[i].empty()) continue;  // with the part that came first
         ph->task_begin[i] = (int64_t)ph->tasks.size();
-        for (int32_t g = 0; g < ph->pairs[i].ngroups; ++g) ph->tasks.push_back(WfTaskDev{(int32_t)i, g});
+        for (int32_t g = 0; g < ph->pairs[i].ngroups; ++g)
+            for (int32_t p : parts[i]) ph->tasks.push_back(WfTaskDev{p, g});
         ph->task_end[i] = (int64_t)ph->tasks.size();
+        parts[i].clear();
     }
     ph->bnd_ints = bnd_ints;
     ph->order = order;
@@ -773,7 +859,7 @@ void wf_plan_bytes(const WfPlanHost *ph, WfPlanBytes *b)
     b->counters = (size_t)(ph->npairs + 1) * sizeof(int32_t);
     b->epoch = sizeof(uint32_t);
     b->colw = (size_t)std::max<int64_t>(1, ph->colw_entries) * 2 * sizeof(uint32_t);
-    b->splits = std::max<size_t>(1, ph->splits.size()) * sizeof(WfSplitDev);
+    b->splits = std::max<size_t>(sizeof(WfSplitDev), wf_cuts_offset(ph) + ph->cuts.size() * sizeof(WfCutDev));
 }
 
 int wf_copy_plan(WfPlanHost *ph, WfArenas *ar, hipStream_t stream)
@@ -785,6 +871,10 @@ int wf_copy_plan(WfPlanHost *ph, WfArenas *ar, hipStream_t stream)
     if (!ph->splits.empty() &&
         hipMemcpyAsync(ar->splits.ptr, ph->splits.data(), ph->splits.size() * sizeof(WfSplitDev),
                        hipMemcpyHostToDevice, stream) != hipSuccess)
+        return WF_ERR_DEVICE;
+    if (!ph->cuts.empty() &&
+        hipMemcpyAsync((uint8_t *)ar->splits.ptr + wf_cuts_offset(ph), ph->cuts.data(),
+                       ph->cuts.size() * sizeof(WfCutDev), hipMemcpyHostToDevice, stream) != hipSuccess)
         return WF_ERR_DEVICE;
     if (!ph->pairs.empty() &&
         hipMemcpyAsync(ar->pairs.ptr, ph->pairs.data(), ph->pairs.size() * sizeof(WfPairDev),
@@ -857,7 +947,7 @@ struct PinnedLayout {
     explicit PinnedLayout(const WfPlanHost *ph)
     {
         splits = round256(ph->codes.size());
-        pairs = splits + round256(ph->splits.size() * sizeof(WfSplitDev));
+        pairs = splits + round256(wf_cuts_offset(ph) + ph->cuts.size() * sizeof(WfCutDev));
         tasks = pairs + round256(ph->pairs.size() * sizeof(WfPairDev));
         res = tasks + round256(ph->tasks.size() * sizeof(WfTaskDev));
         end = res + round256((size_t)std::max<int64_t>(1, ph->npairs) * sizeof(WfResultDev));
@@ -883,6 +973,8 @@ int upload_pinned(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar)
     };
     if (!put(L.codes, ar->codes.ptr, ph->codes.data(), ph->codes.size()) ||
         !put(L.splits, ar->splits.ptr, ph->splits.data(), ph->splits.size() * sizeof(WfSplitDev)) ||
+        !put(L.splits + wf_cuts_offset(ph), (uint8_t *)ar->splits.ptr + wf_cuts_offset(ph), ph->cuts.data(),
+             ph->cuts.size() * sizeof(WfCutDev)) ||
         !put(L.pairs, ar->pairs.ptr, ph->pairs.data(), ph->pairs.size() * sizeof(WfPairDev)) ||
         !put(L.tasks, ar->tasks.ptr, ph->tasks.data(), ph->tasks.size() * sizeof(WfTaskDev)))
         return WF_ERR_DEVICE;
@@ -950,12 +1042,24 @@ int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int max
     ka.epoch = (const uint32_t *)ar->epoch.ptr;
     ka.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
     ka.colw = (uint32_t *)ar->colw.ptr;
+    ka.cuts = (const WfCutDev *)((const uint8_t *)ar->splits.ptr + wf_cuts_offset(ph));
     ph->grid = 0;
     if (ph->tasks.empty()) return WF_OK;
     const WfVariant *v = ph->variant;
     const int lim = maxg > 0 ? maxg : wf_max_resident_groups(ctx, v);
     const int st = enqueue_engine(ph, v, lim, mode, ka, ar, stream);
     if (st != WF_OK) return st;
+    if (!ph->cuts.empty()) {
+        // About 8192 nodes of the cut a workgroup.
+        int64_t nodes = 0;
+        for (const WfSplitDev &sp : ph->splits) nodes = std::max<int64_t>(nodes, (int64_t)sp.r0 + sp.n2);
+        const int blocks = (int)std::min<int64_t>(32, 1 + nodes / 8192);
+        return wf_launch_sw_combine((const WfSplitDev *)ar->splits.ptr, (int)ph->splits.size(), blocks,
+                                    (const uint32_t *)ar->colw.ptr, ka.cuts, (const uint64_t *)ar->bnd.ptr,
+                                    (WfResultDev *)ar->res.ptr, stream) == hipSuccess
+                   ? WF_OK
+                   : WF_ERR_DEVICE;
+    }
     if (!ph->splits.empty() &&
         wf_launch_bitpar_combine((const WfSplitDev *)ar->splits.ptr, (int)ph->splits.size(),
                                  (const uint32_t *)ar->colw.ptr, (WfResultDev *)ar->res.ptr, stream) != hipSuccess)

@@ -719,34 +719,67 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
 // halves line up row by row.
 // ---------------------------------------------------------------------------
 
-// Column-split SW pair (prob WFK_SW): job holds columns 1..mid, f0 the
-// columns mid+1..n1 from a zero boundary (its bottom-right cell R0: the best
-// local alignment starting right of the cut), rev the reversed right half,
-// whose last column E(i) gives the best path weight from (n2 - i, mid) to
-// (n2, n1) as E(i) - 2 (i + r0).  The bottom-right cell is
-// max(R0, max_y H(y, mid) + that weight), H(0, mid) = 0, E(0) = 0.
-__device__ void sw_split_combine(const WfSplitDev &sp, const uint32_t *colw, WfResultDev *res)
+// Column-split SW pair.  The table is cut along a staircase: strip g of 512
+// rows (a row of cells from y_g + 1 to y_{g+1}) at column c_g, c falling with g,
+// so that the strips of the left part and of the reversed right part, each of
+// which starts a strip lag after the one before, all end together.  job holds
+// H left of the cut; f0 the cells right of it from a zero boundary (its
+// bottom-right cell: the best local alignment into the corner that starts
+// right of the cut); rev, for a node (y, x) on or right of the cut, the best
+// path weight F from it to the corner, as E = F + 2 ((n2 - y) + (n1 - x)).
+//
+// An alignment into the corner that starts left of the cut leaves the left
+// part at a node of the staircase: (y, c_g) inside strip g, or (y_{g+1}, x)
+// with c_{g+1} <= x <= c_g on the row between strips g and g+1.  So the corner
+// is the largest of f0's cell and H + F over those nodes, H from job's last
+// columns and bottom rows, E from rev's (rev's strips end where job's begin: its
+// first one is filled up with `pad` rows without a symbol).  H on row 0 and
+// column 0, E on row n2 and column n1 are 0.  The running maximum likewise: the
+// parts' own maxima, or H plus the best path from a node to any cell right of
+// the cut, C from the clamped reversed part.  Without f0, the alignments that
+// start right of the cut are the largest F of rev, and those that lie right of
+// it the largest C of crev.
+//
+// n1 + n2 nodes at most, over `gridDim.y` workgroups; the results by atomics
+// (the reset kernel clears res, and SW cells are >= 0).
+__global__ __launch_bounds__(1024) void wf_sw_combine(const WfSplitDev *splits, const uint32_t *colw,
+                                                      const WfCutDev *cuts, const uint64_t *bnd, WfResultDev *res)
 {
-    // Bottom-right cell: an alignment into (n2, n1) starts right of column
-    // mid (pair f0's cell) or leaves column mid last at some row y after a
-    // best local alignment into (y, mid), H(y, mid), and then takes the best
-    // path from (y, mid) to the corner, E(n2 - y) - 2 (n2 - y + r0) from the
-    // unclamped reverse pair (E(0) = H(0, mid) = 0).  The running maximum
-    // likewise: the halves' own maxima, or H(y, mid) plus the best path from
-    // (y, mid) to any cell right of it, C(n2 - y) from the clamped reverse
-    // pair (C(0) = 0).
-    const int n2 = sp.n2, nr = sp.r0;
+    const WfSplitDev sp = splits[blockIdx.x];
+    const int n1 = sp.r0, n2 = sp.n2, S = sp.strip;
+    const int G = (n2 + S - 1) / S;
     const bool mx = sp.crev >= 0;
     const int *h = reinterpret_cast<const int *>(colw) + 2 * sp.fwd_off;
     const int *e = reinterpret_cast<const int *>(colw) + 2 * sp.rev_off;
     const int *c = reinterpret_cast<const int *>(colw) + 2 * sp.crev_off;
+    const WfCutDev *fc = cuts + sp.cut, *rc = cuts + sp.rcut, *cc = cuts + sp.ccut;
     int best = INT_MIN, bestm = 0;
-    for (int y = threadIdx.x; y <= n2; y += blockDim.x) {
+    // (y, c_g) inside the strips, and the corner strip's end.
+    for (int y = blockIdx.y * blockDim.x + threadIdx.x; y <= n2; y += gridDim.y * blockDim.x) {
+        if (y > 0 && y < n2 && y % S == 0) continue;
+        const int g = y > 0 ? (y - 1) / S : 0;
+        const int cg = fc[g].n, dg = n1 - cg;
         const int i = n2 - y;
-        const int hv = y > 0 ? h[y - 1] : 0;
-        const int ev = i > 0 ? e[i - 1] : 0;
-        best = max(best, hv + ev - 2 * (i + nr));
-        if (mx) bestm = max(bestm, hv + (i > 0 ? c[i - 1] : 0));
+        const int hv = (y > 0 && cg > 0) ? h[y - 1] : 0;
+        const bool right = i > 0 && dg > 0;
+        const int ev = right ? e[i + sp.pad - 1] : 0;
+        best = max(best, hv + ev - 2 * (i + dg));
+        if (mx) bestm = max(bestm, hv + (right ? c[i + sp.pad - 1] : 0));
+    }
+    // (y_{g+1}, x) between the strips.
+    for (int g = blockIdx.y; g + 1 < G; g += gridDim.y) {
+        const int x0 = fc[g + 1].n, x1 = fc[g].n;
+        const int i = n2 - (g + 1) * S;
+        const uint64_t *hb = bnd + fc[g].bnd;                           // column x at word x - 1
+        const uint64_t *eb = bnd + rc[G - 2 - g].bnd;                   // column x at word n1 - x - 1
+        const uint64_t *cb = mx ? bnd + cc[G - 2 - g].bnd : nullptr;
+        for (int x = x0 + threadIdx.x; x <= x1; x += blockDim.x) {
+            const int j = n1 - x;
+            const int hv = x > 0 ? (int)(uint32_t)hb[x - 1] : 0;
+            const int ev = j > 0 ? (int)(uint32_t)eb[j - 1] : 0;
+            best = max(best, hv + ev - 2 * (i + j));
+            if (mx) bestm = max(bestm, hv + (j > 0 ? (int)(uint32_t)cb[j - 1] : 0));
+        }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -767,12 +800,13 @@ __device__ void sw_split_combine(const WfSplitDev &sp, const uint32_t *colw, WfR
             m = max(m, wm[k]);
         }
         WfResultDev &r = res[sp.job];
-        r.last = max(b, res[sp.f0].last);
-        r.status |= res[sp.rev].status | res[sp.f0].status;
+        atomicMax(&r.last, max(b, sp.f0 >= 0 ? res[sp.f0].last : res[sp.rev].maxs));
+        int status = res[sp.rev].status | (sp.f0 >= 0 ? res[sp.f0].status : 0);
         if (mx) {
-            r.maxs = max(max(m, r.maxs), res[sp.f0].maxs);
-            r.status |= res[sp.crev].status;
+            atomicMax(&r.maxs, max(m, res[sp.f0 >= 0 ? sp.f0 : sp.crev].maxs));
+            status |= res[sp.crev].status;
         }
+        if (status) atomicOr(&r.status, status);
     }
 }
 
@@ -780,10 +814,6 @@ __global__ __launch_bounds__(1024) void wf_bitpar_combine(const WfSplitDev *spli
                                                           WfResultDev *res)
 {
     const WfSplitDev sp = splits[blockIdx.x];
-    if (sp.prob == WFK_SW) {
-        sw_split_combine(sp, colw, res);
-        return;
-    }
     const bool ed = sp.prob == WFK_ED;
     const int n2 = sp.n2;
     const int nw = (n2 + 31) >> 5;
@@ -896,6 +926,15 @@ extern "C" hipError_t wf_launch_bitpar_combine(const WfSplitDev *splits, int nsp
 {
     if (nsplits <= 0) return hipSuccess;
     hipLaunchKernelGGL(wfb::wf_bitpar_combine, dim3(nsplits), dim3(1024), 0, stream, splits, colw, res);
+    return hipGetLastError();
+}
+
+extern "C" hipError_t wf_launch_sw_combine(const WfSplitDev *splits, int nsplits, int blocks, const uint32_t *colw,
+                                           const WfCutDev *cuts, const uint64_t *bnd, WfResultDev *res,
+                                           hipStream_t stream)
+{
+    if (nsplits <= 0 || blocks <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(wfb::wf_sw_combine, dim3(nsplits, blocks), dim3(1024), 0, stream, splits, colw, cuts, bnd, res);
     return hipGetLastError();
 }
 

@@ -129,20 +129,28 @@ struct Cell<WFK_SWP, CMP> {
 // The reverse half of a column-split SW pair (WFK_MODE_SWE): the same byte
 // tables and selectors with s + 4 (7 on a match, 1 else) and no clamp,
 // E = max3(up, left, diag + s + 4).  A never-matching column reads -1, so
-// lanes left of column 0 keep the zero boundary.
+// lanes left of column 0 stay far below 0 until column -1, where the lane
+// above delivers the zero boundary (as LCS's do; the maximum must not see
+// zeros left of it).
 template <bool CMP>
 struct Cell<WFK_SWE, CMP> {
-    static constexpr int idle = 0;
+    static constexpr int idle = -kIdleBig;
     static __device__ __forceinline__ uint32_t tables(uint32_t c0, uint32_t c1, int half)
     {
         uint32_t t = 0;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const uint32_t sym = 2u * (uint32_t)half + (uint32_t)k;
-            t |= (c0 == sym ? 0x07u : 0x01u) << (16 * k);
-            t |= (c1 == sym ? 0x07u : 0x01u) << (16 * k + 8);
+            t |= entry(c0, sym) << (16 * k);
+            t |= entry(c1, sym) << (16 * k + 8);
         }
         return t;
+    }
+    // A row that holds no symbol (code 5) adds nothing: it hands the zero
+    // boundary above it down.
+    static __device__ __forceinline__ uint32_t entry(uint32_t c, uint32_t sym)
+    {
+        return c == sym ? 0x07u : c == WFK_NO_SYMBOL ? 0x00u : 0x01u;
     }
     static __device__ __forceinline__ uint32_t selector(uint32_t c) { return Cell<WFK_SWP, CMP>::selector(c); }
     static constexpr uint32_t kNever = Cell<WFK_SWP, CMP>::kNever;
@@ -152,7 +160,7 @@ template <int R>
 struct LaneState {
     int h[R];        // H(row r, last column) -- the next step's "left"
     int dg;          // H(row above row 0, last column) -- the next step's "diag"
-    int best;        // SW running maximum
+    int best;        // SW running maximum (WFK_SWE: see step)
     uint32_t t[R];   // per-row table / code
 };
 
@@ -164,6 +172,14 @@ __device__ __forceinline__ void step(LaneState<R> &st, int inj, uint32_t ca, boo
     int diag = st.dg;
     uint32_t pp = 0;
     if (P == WFK_SWP || P == WFK_SWE) pp = __builtin_amdgcn_perm(st.t[1], st.t[0], ca);
+    // WFK_SWE: the largest F = E - 2 (i + j) of the lane.  The offset falls by 2
+    // a step and from row 0 to row 1, so E of row 0 and row 1's E of the step
+    // before have the same one, and st.best, kept relative to row 0's current
+    // offset, rises by 2 a step: one add and one max3.
+    if constexpr (P == WFK_SWE && TRACK) {
+        static_assert(R == 2, "rows 0 and 1");
+        if (!MASKED || valid) st.best = max(st.best + 2, st.h[R - 1]);
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int left = st.h[r];
@@ -176,11 +192,11 @@ __device__ __forceinline__ void step(LaneState<R> &st, int inj, uint32_t ca, boo
         } else {
             h = Cell<P, CMP>::f(up, left, diag, ca, st.t[r]);
         }
-        if (MASKED) {
-            h = valid ? h : left;
-            if (TRACK) st.best = max(st.best, valid ? h : 0);
+        if (MASKED) h = valid ? h : left;
+        if constexpr (P == WFK_SWE && TRACK) {
+            if (r == 0 && (!MASKED || valid)) st.best = max(st.best, h);
         } else if (TRACK) {
-            st.best = max(st.best, h);
+            st.best = max(st.best, (!MASKED || valid) ? h : 0);
         }
         diag = left;
         st.h[r] = h;

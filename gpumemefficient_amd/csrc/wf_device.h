@@ -29,10 +29,12 @@ enum {
     // The reverse half of a column-split SW pair (with WFK_MODE_PERM4): the
     // unclamped best path weight into each cell of the reversed sequences,
     // kept as E = F + 2 (x + y), so E = max3(up, left, diag + s + 4) with
-    // zero boundaries.
+    // zero boundaries.  Its maximum (without WFK_MODE_NOMAX) is the largest F.
     WFK_MODE_SWE = 64,
 };
 enum { WFK_MODE_NEVER_SHIFT = 8 };
+// Byte tables: code of a row above the first symbol's (WfSplitDev::pad).
+enum { WFK_NO_SYMBOL = 5 };
 
 // One sequence pair as the kernels see it.  x runs over a (n1 columns),
 // y over b (n2 rows).  Codes are one byte per symbol in the code arena.
@@ -54,7 +56,19 @@ struct WfPairDev {
     // resident server, whose one launch outlives many pairs in recycled
     // memory, gives every request a tag of its own.
     uint32_t tag = 0;
-    int32_t pad = 0;
+    // Index in WfKernelArgs::cuts of strip 0's columns, where the strips of a
+    // pair do not all sweep the columns 0..n1 (SW column split); -1: they do.
+    int32_t cut = -1;
+};
+
+// The columns one strip of a pair sweeps (WfPairDev::cut + strip).
+struct WfCutDev {
+    int64_t bnd;       // element offset of the strip's bottom row (n words, none for the pair's last strip)
+    int32_t x0, n;     // first column (0-based, in a's codes) and their number; 0: nothing to do
+    int32_t xp;        // first column the strip above sweeps: left of it the top boundary is row 0's
+    int32_t skip;      // waves at the top of the strip that hold no row of the pair
+    int32_t pad;       // rows at the pair's top that hold no symbol (WfSplitDev::pad)
+    int32_t spare;
 };
 
 // A pair computed as two column halves (bit-parallel engine, LCS and ED):
@@ -64,25 +78,29 @@ struct WfPairDev {
 // the score is min (ED) / max (LCS) over y of F(y) + R(y) (Hirschberg's
 // split, J. ACM 1975; CACM 18(6) 1975 for LCS).
 //
-// An SW pair (prob WFK_SW, cell engine with byte tables) splits into three:
-// `job` (columns 1..mid), `f0` (columns mid+1..n1 from a zero boundary) and
-// `rev` (the reversed right half, WFK_MODE_SWE); r0 is the right half's
-// column count.  A pair that keeps the running maximum adds a fourth, `crev`
-// (the reversed right half with the clamped recurrence, no maximum), whose
-// last column starts at colw entry crev_off (see sw_split_combine in
-// wf_bitpar.hip).
+// An SW pair (prob WFK_SW, cell engine with byte tables) is cut along a
+// staircase, strip g at column c(g), into the left part `job`, the right part
+// from a zero boundary `f0`, the right part reversed `rev` (WFK_MODE_SWE) and,
+// for a pair that keeps the running maximum, the right part reversed with the
+// clamped recurrence `crev` (see wf_sw_combine in wf_bitpar.hip).  A pair whose
+// three or four parts have too many strips for the chip does without f0 (-1):
+// rev and crev then keep their own maxima.  The left
+// and the reversed parts keep their last columns at colw entries fwd_off,
+// rev_off and crev_off, and their strips' bottom rows.
 struct WfSplitDev {
     int32_t job;       // result slot (the forward half's pair)
     int32_t rev;       // the reverse half's pair
     int32_t prob;      // WFK_ED / WFK_LCS / WFK_SW
     int32_t n2;        // rows
     int32_t f0;        // ED: F(0), row 0 of the table at column mid; LCS: 0; SW: the right half's pair
-    int32_t r0;        // ED: the reverse half's row 0 at its last column (n1 - mid); LCS: 0; SW: n1 - mid
+    int32_t r0;        // ED: the reverse half's row 0 at its last column (n1 - mid); LCS: 0; SW: n1
     int64_t fwd_off;   // colw entry offsets of the two halves
     int64_t rev_off;
     int32_t crev = -1; // SW with the running maximum: the clamped reverse pair; -1: none
-    int32_t pad = 0;
+    int32_t strip = 0; // SW: rows of a strip
     int64_t crev_off = 0;
+    int32_t cut = 0, rcut = 0, ccut = 0;  // SW: WfCutDev indices of job, rev and crev
+    int32_t pad = 0;   // SW: rows without a symbol above the reversed parts' rows (their strips end where job's begin)
 };
 
 // One unit of persistent work: strip `group` of pair `pair`.  Tasks of a
@@ -115,6 +133,7 @@ struct WfKernelArgs {
                              // every launch, so graph replays get fresh tags)
     int32_t *table;          // table-dump kernel only: H(y+1, x+1) of pair 0 at [y * n1 + x]
     uint32_t *colw;          // bit-parallel engine: last-column entries, two words each (WfPairDev::col_off)
+    const WfCutDev *cuts;    // WfPairDev::cut
 };
 
 // ----------------------------------------------------------------------------

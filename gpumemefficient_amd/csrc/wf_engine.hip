@@ -310,11 +310,22 @@ __device__ __forceinline__ bool run_steps(LaneState<R> &st, int q0, int ngr, int
     return ok;
 }
 
+// What a strip sweeps: its columns, its rows' neighbours in HBM.
+struct StripGeom {
+    const uint8_t *a;        // codes of its columns
+    const uint64_t *bprev;   // the bottom row of the strip above, from this strip's first column
+    uint64_t *bnext;         // its own bottom row
+    int n1;                  // columns
+    int xp;                  // columns left of it have row 0 above them, not the strip above
+    int wf;                  // first wave that holds rows
+    int pad;                 // rows of the pair above the first symbol's
+};
+
 // Forced inline into the kernel: left as a call it takes the kernel
 // arguments by address and copies them (and the pair) to scratch memory,
 // which the steady loop then reloads.
 template <int P, bool CMP, int R, int W, int G, int AW, int RS, bool NOMAX = false>
-__device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPairDev &pd, int pair, int g,
+__device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPairDev &pd, const StripGeom &sg, int pair, int g,
                             AsyncShared<W, G, AW, RS> &sh, int lane, int wave, uint32_t epoch, int task)
 {
 #ifdef WFK_TRACE
@@ -338,8 +349,8 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
         }
     };
 #endif
-    constexpr bool TRACK = (P == WFK_SW || P == WFK_SWP) && !NOMAX;
-    const int n1 = pd.n1, n2 = pd.n2;
+    constexpr bool TRACK = (P == WFK_SW || P == WFK_SWP || P == WFK_SWE) && !NOMAX;
+    const int n1 = sg.n1, n2 = pd.n2, wf = sg.wf;
     const int nsteps = n1 + 63;
     const bool has_prev = g > 0;
     const bool has_next = g + 1 < pd.ngroups;
@@ -349,7 +360,7 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
     const int64_t rows_left = (int64_t)n2 - (int64_t)g * (W * 64 * R);
     const int wa = (int)min<int64_t>(W, (rows_left + 64 * R - 1) / (64 * R));
 
-    if (wave < W && wave >= wa) {
+    if (wave < W && (wave >= wa || wave < wf)) {
         // Only padding rows: never block the wave above (its consumer).
         cnt_store(sh.cnt[wave + 1] + lane, 1 << 30);
         return;
@@ -377,7 +388,7 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
             }
         }
         st.dg = 0;
-        st.best = 0;
+        st.best = P == WFK_SWE ? -kIdleBig : 0;
         // Lanes left of column 0 run unmasked steps (see Cell::idle): lane 0
         // starts at column 0, lane l >= 1 at column -l from the idle state.
         const bool free_head = (pd.mode & WFK_MODE_FREE_HEAD) != 0;
@@ -387,13 +398,16 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
             st.dg = Cell<P, CMP>::idle;
         }
 
-        const int *cin = sh.cnt[w] + lane;        // producer of my input
+        // The strip's first wave reads what the input wave stages, the others
+        // the wave above.
+        const int win = w == wf ? 0 : w;
+        const int *cin = sh.cnt[win] + lane;      // producer of my input
         const int *cout = sh.cnt[w + 2] + lane;   // consumer of my output ring
         int *cmine = sh.cnt[w + 1] + lane;
         const int ngr = (nsteps + G - 1) / G;
         // Group q reads input columns < (q+1)G: staged (w = 0) or written by
         // lane 63 of wave w-1, which finishes column c at its step c + 63.
-        auto need_in = [&](int q) __attribute__((always_inline)) { return w == 0 ? min(n1, (q + 1) * G) : min(nsteps, (q + 1) * G + 63); };
+        auto need_in = [&](int q) __attribute__((always_inline)) { return w == wf ? min(n1, (q + 1) * G) : min(nsteps, (q + 1) * G + 63); };
         // Group q overwrites ring slots of columns up to (q+1)G - 64 - RS,
         // which the consumer must have read.
         auto need_out = [&](int q) __attribute__((always_inline)) { return (q + 1) * G - 63 - RS; };
@@ -449,7 +463,7 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
         // Counters first, then the first block's operands (check on use).
         int vin = cnt_load(cin), vout = cnt_load(cout);
         lds_acquire();
-        load_block<AW, RS>(blk, sh.ring[w], sh.aw, 0, lane);
+        load_block<AW, RS>(blk, sh.ring[win], sh.aw, 0, lane);
         // Published progress, kept in a VGPR of its own (it is loaded, so the
         // compiler treats it as per-lane): materialising it from an SGPR right
         // before the store would reuse a register of a capture store still in
@@ -505,15 +519,15 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
         int pend = 0;  // lane 63's last capture not yet in the ring (see run_steps)
         for (; !aborted && q < ngr && !(steady_from(q) && (q * G) % KU == 0); ++q)
             aborted = !run_steps<P, CMP, R, G, G, AW, RS, true, TRACK>(
-                st, q, ngr, lane, n1, xlo, sh.ring[w], sh.ring[w + 1], sh.dummy[w], sh.aw, blk, pend, cin, cout, vin, vout,
+                st, q, ngr, lane, n1, xlo, sh.ring[win], sh.ring[w + 1], sh.dummy[w], sh.aw, blk, pend, cin, cout, vin, vout,
                 need_in, need_out, wait_slow, publish);
         for (; !aborted && steady_from(q); q += UG)
             aborted = !run_steps<P, CMP, R, G, KU, AW, RS, false, TRACK>(
-                st, q, ngr, lane, n1, xlo, sh.ring[w], sh.ring[w + 1], sh.dummy[w], sh.aw, blk, pend, cin, cout, vin, vout,
+                st, q, ngr, lane, n1, xlo, sh.ring[win], sh.ring[w + 1], sh.dummy[w], sh.aw, blk, pend, cin, cout, vin, vout,
                 need_in, need_out, wait_slow, publish);
         for (; !aborted && q < ngr; ++q)
             aborted = !run_steps<P, CMP, R, G, G, AW, RS, true, TRACK>(
-                st, q, ngr, lane, n1, xlo, sh.ring[w], sh.ring[w + 1], sh.dummy[w], sh.aw, blk, pend, cin, cout, vin, vout,
+                st, q, ngr, lane, n1, xlo, sh.ring[win], sh.ring[w + 1], sh.dummy[w], sh.aw, blk, pend, cin, cout, vin, vout,
                 need_in, need_out, wait_slow, publish);
         if (aborted) {
             // Mark the pair failed: in a pair's last strip no output wave
@@ -532,10 +546,18 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
                 for (int r = 0; r < R; ++r)
                     if (r == rr) v = st.h[r];
                 if (P == WFK_ED) v += n1 + n2;
-                ka.res[pair].last = v;
+                // (The parts of a column-split SW pair keep their last column
+                // instead.)
+                if (!((P == WFK_SWP || P == WFK_SWE) && pd.col_off >= 0)) ka.res[pair].last = v;
             }
             if (TRACK) {
                 int m = st.best;
+                if constexpr (P == WFK_SWE) {
+                    // Relative to row 0's offset at the last column; rows
+                    // without a symbol do not count.
+                    const int64_t i0 = row0 + 1 - sg.pad;
+                    m = i0 < 0 ? 0 : max(m, st.h[R - 1] - 2) - 2 * (n1 + (int)i0);
+                }
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
                 if (lane == 0 && m > 0) atomicMax(&ka.res[pair].maxs, m);
@@ -557,9 +579,9 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
     // The two I/O waves share SIMDs with compute waves 0 and 1 and run below
     // them: they only take issue slots those waves leave idle.
     __builtin_amdgcn_s_setprio(0);
-    const uint8_t *acodes = ka.codes + pd.a_off;
-    const uint64_t *bprev = ka.bnd + pd.bnd_off + (int64_t)(g - 1) * n1;
-    uint64_t *bnext = ka.bnd + pd.bnd_off + (int64_t)g * n1;
+    const uint8_t *acodes = sg.a;
+    const uint64_t *bprev = sg.bprev;
+    uint64_t *bnext = sg.bnext;
     const int *clast = sh.cnt[wa] + lane;   // last compute wave: slowest reader of aw, producer of ring[W]
     bool aborted = false;
 
@@ -625,7 +647,10 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
     // stages its ready prefix (the lanes up to the first stale tag).
     // Row 0 of the table in the kernels' value representation.
     const int topv = (P == WFK_ED && !(pd.mode & WFK_MODE_TEXTBOOK)) ? -1 : 0;
-    const int *c0 = sh.cnt[1] + lane;       // compute wave 0: reads ring[0] and aw
+    const int *c0 = sh.cnt[1 + wf] + lane;  // first compute wave: reads ring[0] and aw
+    // Columns whose top boundary is the strip above's bottom row (SW: the rows
+    // left of them are row 0's zeros).
+    const int xp = (P == WFK_SWP) ? sg.xp : 0;
     // Column x lives in code slot (x + 64) mod AW; the slots of columns
     // -64..-1, read by lanes left of column 0, hold a code that matches no
     // row (see WFK_MODE_FREE_HEAD).  Written before the first staging
@@ -666,7 +691,7 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
         const bool in = x < n1;
         p.c = in ? (uint32_t)acodes[x] : 0u;
         if (P == WFK_SWP || P == WFK_SWE) p.c = Cell<WFK_SWP, false>::selector(p.c & 3u);
-        p.t = (has_prev && in)
+        p.t = (has_prev && in && x >= xp)
                   ? (lane < p.width ? __hip_atomic_load(bprev + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0)
                   : tag;
     };
@@ -782,37 +807,64 @@ __global__ __launch_bounds__(64 * (W + 2)) void wf_engine_async(WfKernelArgs ka)
         const WfTaskDev td = ka.tasks[t];
         const WfPairDev pd = ka.pairs[td.pair];
         set_wave_priority(pd.prio);
+        StripGeom sg;
+        if (pd.cut < 0) {
+            sg.a = ka.codes + pd.a_off;
+            sg.bprev = ka.bnd + pd.bnd_off + (int64_t)(td.group - 1) * pd.n1;
+            sg.bnext = ka.bnd + pd.bnd_off + (int64_t)td.group * pd.n1;
+            sg.n1 = pd.n1;
+            sg.xp = 0;
+            sg.wf = 0;
+            sg.pad = 0;
+        } else {
+            const WfCutDev cd = ka.cuts[pd.cut + td.group];
+            const WfCutDev ab = ka.cuts[pd.cut + max(0, td.group - 1)];
+            sg.a = ka.codes + pd.a_off + cd.x0;
+            sg.bprev = ka.bnd + ab.bnd + (cd.x0 - ab.x0);
+            sg.bnext = ka.bnd + cd.bnd;
+            sg.n1 = cd.n;
+            sg.xp = cd.xp - cd.x0;
+            sg.wf = cd.skip;
+            sg.pad = cd.pad;
+            if (cd.n == 0) {
+                __syncthreads();
+                continue;
+            }
+        }
         const bool cmp = (pd.mode & WFK_MODE_CMP) != 0;
         switch (pd.prob * 2 + (cmp ? 1 : 0)) {
-        case WFK_LCS * 2 + 0: async_strip<WFK_LCS, false, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t); break;
-        case WFK_LCS * 2 + 1: async_strip<WFK_LCS, true, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t); break;
-        case WFK_ED * 2 + 0: async_strip<WFK_ED, false, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t); break;
-        case WFK_ED * 2 + 1: async_strip<WFK_ED, true, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t); break;
+        case WFK_LCS * 2 + 0: async_strip<WFK_LCS, false, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t); break;
+        case WFK_LCS * 2 + 1: async_strip<WFK_LCS, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t); break;
+        case WFK_ED * 2 + 0: async_strip<WFK_ED, false, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t); break;
+        case WFK_ED * 2 + 1: async_strip<WFK_ED, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t); break;
         case WFK_SW * 2 + 0: {
             // Instances without the running maximum for WFK_MODE_NOMAX.
             const bool nomax = (pd.mode & WFK_MODE_NOMAX) != 0;
             if constexpr (R == 2) {
                 if (pd.mode & WFK_MODE_SWE) {
-                    async_strip<WFK_SWE, false, R, W, G, AW, RS, true>(ka, pd, td.pair, td.group, sh, lane, wave,
-                                                                      epoch, t);
+                    if (nomax)
+                        async_strip<WFK_SWE, false, R, W, G, AW, RS, true>(ka, pd, sg, td.pair, td.group, sh, lane, wave,
+                                                                          epoch, t);
+                    else
+                        async_strip<WFK_SWE, false, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
                     break;
                 }
                 if (pd.mode & WFK_MODE_PERM4) {
                     if (nomax)
-                        async_strip<WFK_SWP, false, R, W, G, AW, RS, true>(ka, pd, td.pair, td.group, sh, lane, wave,
+                        async_strip<WFK_SWP, false, R, W, G, AW, RS, true>(ka, pd, sg, td.pair, td.group, sh, lane, wave,
                                                                           epoch, t);
                     else
-                        async_strip<WFK_SWP, false, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t);
+                        async_strip<WFK_SWP, false, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
                     break;
                 }
             }
             if (nomax)
-                async_strip<WFK_SW, false, R, W, G, AW, RS, true>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t);
+                async_strip<WFK_SW, false, R, W, G, AW, RS, true>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
             else
-                async_strip<WFK_SW, false, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t);
+                async_strip<WFK_SW, false, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
             break;
         }
-        default: async_strip<WFK_SW, true, R, W, G, AW, RS>(ka, pd, td.pair, td.group, sh, lane, wave, epoch, t); break;
+        default: async_strip<WFK_SW, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t); break;
         }
         __syncthreads();
     }

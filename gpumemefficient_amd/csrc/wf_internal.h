@@ -84,6 +84,7 @@ struct WfPlanHost {
     int64_t njobs = 0;   // result slots 0..njobs-1
     int64_t npairs = 0;  // njobs plus the reverse halves of split pairs
     std::vector<WfSplitDev> splits;
+    std::vector<WfCutDev> cuts;  // columns of the strips of SW splits' pairs; device: behind the splits
     int64_t colw_entries = 0;
     const WfVariant *variant = nullptr;
     std::vector<WfPairDev> pairs;
@@ -124,6 +125,8 @@ int wf_default_rows_per_lane(int waves, int64_t max_rows, int64_t total_cells, i
 // strips fit in them.
 int wf_build_plan(struct wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile,
                   WfPlanHost *ph, int64_t max_groups = 0);
+// Bytes from the splits to the cuts behind them.
+inline size_t wf_cuts_offset(const WfPlanHost *ph) { return (ph->splits.size() * sizeof(WfSplitDev) + 15) & ~size_t(15); }
 // Device bytes of every buffer a plan needs.
 struct WfPlanBytes {
     size_t codes, pairs, tasks, bnd, res, counters, epoch, colw, splits;

@@ -38,6 +38,11 @@ extern "C" hipError_t wf_launch_naive(int method, int prob, int textbook, int *t
 // Combine the two halves of each split pair (WfSplitDev) into res[job].
 extern "C" hipError_t wf_launch_bitpar_combine(const WfSplitDev *splits, int nsplits, const uint32_t *colw,
                                                WfResultDev *res, hipStream_t stream);
+// The same for column-split SW pairs (`blocks` workgroups a pair), after the
+// reset kernel and the engine launches that filled colw and bnd.
+extern "C" hipError_t wf_launch_sw_combine(const WfSplitDev *splits, int nsplits, int blocks, const uint32_t *colw,
+                                           const WfCutDev *cuts, const uint64_t *bnd, WfResultDev *res,
+                                           hipStream_t stream);
 extern "C" hipError_t wf_launch_engine(const WfVariant *v, int grid, const WfKernelArgs *ka,
                                        hipStream_t stream);
 // Resident server engine (lock-step <2, 4, 64>): the kernel (for occupancy
