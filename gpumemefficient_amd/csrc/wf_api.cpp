@@ -607,7 +607,8 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     auto place = [&](WfPairDev &p, int prob, int64_t n1, int64_t n2, int64_t a_bytes) {
         place_codes(p, prob, n1, n2, a_bytes);
         p.bnd_off = bnd_ints;
-        bnd_ints += (int64_t)(p.ngroups - 1) * n1;
+        // One word per column, or (bs_row_words in wf_bitpar.hip) 4 per 64 steps.
+        bnd_ints += (int64_t)(p.ngroups - 1) * (v->engine == WF_ENGINE_BITPAR_STAGED ? 4 * ((n1 + 126) / 64) : n1);
     };
     for (int64_t i = 0; i < njobs; ++i) {
         const wf_job &j = jobs[i];

@@ -98,10 +98,12 @@ __device__ __forceinline__ void bp_step(BpState &st, int2 inj, uint32_t eq)
     if (P == WFK_ED) {
         const int nph = __builtin_amdgcn_update_dpp(inj.x, st.ph, kDppWaveShr1, 0xf, 0xf, false);
         const int nmh = __builtin_amdgcn_update_dpp(inj.y, st.mh, kDppWaveShr1, 0xf, 0xf, false);
+        // A delta of -1 from above makes row 0 a match (Eq | 1).  Added to the
+        // sum instead, it does the same to xh's bit 0 and to the carry out of it
+        // whatever Pv's and Eq's bits are, and needs no Eq | 1 of its own.
         const uint32_t hm = (uint32_t)nmh >> 31;  // hin == -1
         const uint32_t xv = eq | st.mv;
-        const uint32_t eq2 = eq | hm;
-        const uint32_t xh = (((eq2 & st.pv) + st.pv) ^ st.pv) | eq2;
+        const uint32_t xh = (((eq & st.pv) + st.pv + hm) ^ st.pv) | eq;
         const uint32_t ph = st.mv | ~(xh | st.pv);
         const uint32_t mh = st.pv & xh;
         // (h << 1) | the word above's last-row delta.
@@ -118,9 +120,9 @@ __device__ __forceinline__ void bp_step(BpState &st, int2 inj, uint32_t eq)
         const uint32_t u = st.pv & eq;
         const uint32_t sum = st.pv + u + ((uint32_t)cw >> 31);
         // Carry out of bit 31: majority of the operands' top bits and the
-        // carry into it, i.e. (V & U) | ((V | U) & ~sum).
-        st.ph = (int)((st.pv & u) | ((st.pv | u) & ~sum));
-        st.pv = sum | (st.pv & ~u);
+        // carry into it, (V & U) | ((V | U) & ~sum), with U = V & Eq.
+        st.ph = (int)(st.pv & (eq | ~sum));
+        st.pv = sum | (st.pv & ~eq);
     }
 }
 
@@ -415,23 +417,28 @@ __global__ __launch_bounds__(64 * W) void wf_engine_bitpar(WfKernelArgs ka)
 // address, the table read).  Here a staging wave does those lookups for the
 // compute waves one chunk ahead and leaves each lane's masks in LDS in step
 // order, four steps per 16-byte word, so a compute wave fetches the masks of
-// four steps with one ds_read_b128 and no address arithmetic (ED: 16.8
-// instructions per step instead of 19.6).  The staging wave also loads the
-// column codes and the strip's top boundary and stores the bottom row, so
-// the compute waves issue no global memory operation at all.  The mask
-// buffers take 16 KB of LDS per compute wave and chunk parity (W = 1: 51 KB
-// per workgroup): the planner takes this variant for launches whose strips
-// fit on the chip at once (single large pairs), and the engine above, which
-// packs more compute waves per CU, for throughput-bound batches.  Measured
-// on ED 65536^2: W = 1 2.75 ms (plain engine 3.23 ms at its best W = 2);
-// W = 2 3.14 ms, W = 3 3.93 ms (one staging wave cannot feed more).
+// four steps with one ds_read_b128 and no address arithmetic.  The staging wave
+// also loads the column codes, lays out what the row above hands to lane 0, and
+// publishes the bottom row, so the compute waves issue no global memory
+// operation at all.  The mask buffers take 16 KB of LDS per compute wave and
+// chunk parity: the planner takes this variant for launches whose strips fit on
+// the chip at once (single large pairs), and the engine above, which packs more
+// compute waves per CU, for throughput-bound batches.
+//
+// A step is bound by the issue of a lone wave (about 5 cycles an instruction):
+// 13 VALU operations for ED and 6 for LCS, one or two to collect what lane 63
+// hands down, and the LDS reads.  Per step, W = 1: ED 38.4 -> 33.1 ns, LCS 25.5 ->
+// 19.3 (before: every step's words stored to LDS, ED with one more operation);
+// ED 65536^2 1.51 -> 1.33 ms, LCS 32768^2 0.547 -> 0.399.  W = 2 overloads the one
+// staging wave.
 // ---------------------------------------------------------------------------
 
 template <int W>
 struct BsCfg {
     static constexpr int K = 64;
-    static constexpr int D = (K + 62) / K + 1;
-    static constexpr int RS = pow2_at_least((D + 2) * K + 64);
+    // Chunks between consecutive waves: wave w's upper words of a chunk are
+    // taken out of wave w-1's (two chunks of it) one iteration ahead.
+    static constexpr int D = 3;
     static constexpr int AW = pow2_at_least((2 + (W - 1) * D) * K + 64 + K);
 };
 
@@ -439,40 +446,62 @@ template <int W>
 struct BsShared {
     static constexpr int K = BsCfg<W>::K;
     static constexpr int AW = BsCfg<W>::AW;
-    static constexpr int RS = BsCfg<W>::RS;
     // eqb[i & 1][w][q / 4][lane]: lane's match masks for steps q..q+3 of
     // compute wave w's chunk in iteration i (written during iteration i - 1).
     int4 eqb[2][W][K / 4][64];
-    // As in BpShared.
-    __attribute__((aligned(16))) int2 ring[W + 1][RS];
-    int peq[W][32 * 64];
-    int2 dummy[W][64 + K];
+    // injb[i & 1][w][q]: what the row above wave w hands to lane 0 at step q of
+    // that chunk.  ED: (Ph, Mh) words whose top bits are the horizontal delta
+    // (+1, -1); LCS: one word (the first K ints) whose top bit is the carry.
+    __attribute__((aligned(16))) int2 injb[2][W][K];
+    // cap[w][k & 7]: what lane 63 of wave w handed down in its steps 32k ..
+    // 32k+31 (columns 32k-63 ..), one bit per step, the first in bit 31; ED: .x
+    // +1, .y -1; LCS: .x the carry.
+    int2 cap[W][8];
+    int2 dummy[64];  // lanes 0..62 store here, so that the capture is one unmasked write
+    int peq[W][32 * 64];  // as in BpShared
     uint32_t aw[AW + K];
     int task;
     int abort_at;
 };
 
-// One chunk of K steps of a compute wave; masks from `eqw` (= eqb[i & 1][w]).
-template <int P, int K, int RS, bool MASKED>
-__device__ __forceinline__ void bs_chunk(BpState &st, int s0, int lane, int n1, const int2 *ring_prev, int2 *ring_cur,
-                                         int2 *dummy, const int4 *eqw)
+// Steps of one 64-bit-word row of a strip's bottom boundary in HBM: chunk c's
+// 64 steps of lane 63 are words 2c and 2c+1 (LCS), each (epoch << 32 | 32 bits
+// as in BsShared::cap), or pairs of words (ED: +1 bits, -1 bits).
+__device__ __forceinline__ int64_t bs_row_words(int n1) { return 4 * (int64_t)((n1 + 126) / 64); }
+
+// One chunk of K steps of a compute wave; masks from `eqw` (= eqb[i & 1][w]),
+// upper words from `inj` (= injb[i & 1][w]), lane 63's bits to cap[0] and cap[1]
+// (`cap`: a dummy in the other lanes).  The bits are collected in a register
+// (one v_alignbit a step and word) and stored once per 32 steps: storing
+// every step's words instead took 55 cycles a step for LCS and 79 for ED where
+// this takes 39 and 70 (one wave, operands from LDS, no staging wave beside).
+template <int P, int K, bool MASKED>
+__device__ __forceinline__ void bs_chunk(BpState &st, int s0, int lane, int n1, const int2 *inj, int2 *cap,
+                                         const int4 *eqw)
 {
-    int2 *cap = (lane == 63) ? ring_cur + ((s0 + 1) & (RS - 1)) : dummy + lane;
-    int2 *cap_last = (lane == 63) ? ring_cur + ((s0 + K) & (RS - 1)) : dummy + lane + (K - 1);
+    constexpr bool ED = P == WFK_ED;
     auto load_inj = [&](int q, int2 (&v)[4]) {
-        const int2 *ib = ring_prev + ((s0 + 64 + (q & ~63)) & (RS - 1)) + (q & 63);
-        const int4 i01 = *reinterpret_cast<const int4 *>(ib);
-        const int4 i23 = *reinterpret_cast<const int4 *>(ib + 2);
-        v[0] = make_int2(i01.x, i01.y);
-        v[1] = make_int2(i01.z, i01.w);
-        v[2] = make_int2(i23.x, i23.y);
-        v[3] = make_int2(i23.z, i23.w);
+        if (ED) {
+            const int4 i01 = *reinterpret_cast<const int4 *>(inj + q);
+            const int4 i23 = *reinterpret_cast<const int4 *>(inj + q + 2);
+            v[0] = make_int2(i01.x, i01.y);
+            v[1] = make_int2(i01.z, i01.w);
+            v[2] = make_int2(i23.x, i23.y);
+            v[3] = make_int2(i23.z, i23.w);
+        } else {
+            const int4 i = *reinterpret_cast<const int4 *>(reinterpret_cast<const int *>(inj) + q);
+            v[0].x = i.x;
+            v[1].x = i.y;
+            v[2].x = i.z;
+            v[3].x = i.w;
+        }
     };
     const int4 *ep = eqw + lane;
     // Masks and lane 0's upper words are read one group of 4 steps ahead.
     int4 eqv = ep[0];
-    int2 injv[4];
+    int2 injv[4] = {};
     load_inj(0, injv);
+    uint32_t accp = 0, accm = 0;
 #pragma unroll
     for (int q = 0; q < K; q += 4) {
         int4 eqn = make_int4(0, 0, 0, 0);
@@ -482,7 +511,6 @@ __device__ __forceinline__ void bs_chunk(BpState &st, int s0, int lane, int n1, 
             load_inj(q + 4, injn);
         }
         const uint32_t e[4] = {(uint32_t)eqv.x, (uint32_t)eqv.y, (uint32_t)eqv.z, (uint32_t)eqv.w};
-        int2 capv[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             if (MASKED) {
@@ -493,16 +521,10 @@ __device__ __forceinline__ void bs_chunk(BpState &st, int s0, int lane, int n1, 
             } else {
                 bp_step<P>(st, injv[u], e[u]);
             }
-            capv[u] = make_int2(st.ph, st.mh);
+            accp = __builtin_amdgcn_alignbit(accp, (uint32_t)st.ph, 31);
+            if (ED) accm = __builtin_amdgcn_alignbit(accm, (uint32_t)st.mh, 31);
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = q + u;
-            if (j == K - 1)
-                *cap_last = capv[u];
-            else
-                cap[j] = capv[u];
-        }
+        if (q % 32 == 28) cap[q / 32] = make_int2((int)accp, (int)accm);
         if (q + 4 < K) {
             eqv = eqn;
 #pragma unroll
@@ -518,8 +540,9 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
 {
     constexpr int K = BsCfg<W>::K;
     constexpr int AW = BsCfg<W>::AW;
-    constexpr int RS = BsCfg<W>::RS;
     constexpr int kD = BsCfg<W>::D;
+    constexpr bool ED = P == WFK_ED;
+    constexpr int NP = ED ? 2 : 1;  // bit planes of the handed-down words
     const bool stager = wave == W;
     const int n1 = pd.n1, n2 = pd.n2;
     const int64_t row0 = (int64_t)g * (W * kRowsPerWave) + wave * kRowsPerWave + lane * 32;
@@ -546,13 +569,13 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
     const int total = nch + (wa - 1) * kD;
     const bool has_prev = g > 0;
     const bool has_next = g + 1 < pd.ngroups;
-    const uint64_t *bprev = ka.bnd + pd.bnd_off + (int64_t)(g - 1) * n1;
-    uint64_t *bnext = ka.bnd + pd.bnd_off + (int64_t)g * n1;
+    const uint64_t *bprev = ka.bnd + pd.bnd_off + (g - 1) * bs_row_words(n1);
+    uint64_t *bnext = ka.bnd + pd.bnd_off + g * bs_row_words(n1);
     const uint64_t tag = (uint64_t)epoch << 32;
 
     // Staging wave: column codes of chunk c (column c*K + lane per lane) into
-    // the code window, the strip's top boundary of chunk c into ring[0]
-    // (values as in bp_group), and the masks of an iteration's chunks.
+    // the code window, the strip's top boundary of chunk c into injb, and the
+    // masks of an iteration's chunks.
     auto load_code = [&](int c) -> uint32_t {
         const int x = c * K + lane;
         return x < n1 ? (uint32_t)acodes[x] : 0u;
@@ -565,42 +588,52 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
             if (slot < K) sh.aw[AW + slot] = code;
         }
     };
+    // Column c*K + q of chunk c is step c*K + q + 63 of lane 63 of the wave
+    // above, so the chunk's columns are in its words 2c + 1 .. 2c + 3.
+    const int word_of = ((lane + 63) >> 5) - 1, bit_of = 31 - ((lane + 63) & 31);
+    auto put_inj = [&](int it, int w, uint32_t plus, uint32_t minus) {
+        if (ED)
+            sh.injb[it & 1][w][lane] = make_int2((int)(plus << 31), (int)(minus << 31));
+        else
+            reinterpret_cast<int *>(sh.injb[it & 1][w])[lane] = (int)(plus << 31);
+    };
+    // The strip above's words (lane i: word 2c + 1 + i / NP, plane i % NP).
+    auto has_word = [&](int c) { return has_prev && lane < 3 * NP && 2 * c + 1 + lane / NP < 2 * nch; };
     auto load_top = [&](int c) -> uint64_t {
-        const int x = c * K + lane;
-        return (!has_prev || x >= n1) ? tag : __hip_atomic_load(bprev + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return has_word(c) ? __hip_atomic_load(bprev + (2 * c + 1) * NP + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                           : tag;
     };
     auto fill_top = [&](int c, uint64_t top) -> bool {
-        const int x = c * K + lane;
         if (__builtin_amdgcn_ballot_w64((top >> 32) != (uint64_t)epoch) != 0) {
             const int64_t t0 = now_ticks();
             for (;;) {
                 __builtin_amdgcn_s_sleep(1);
-                if ((top >> 32) != (uint64_t)epoch)
-                    top = __hip_atomic_load(bprev + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((top >> 32) != (uint64_t)epoch) top = load_top(c);
                 if (__builtin_amdgcn_ballot_w64((top >> 32) != (uint64_t)epoch) == 0) break;
                 if (now_ticks() - t0 > ka.timeout_ticks) return false;
             }
         }
-        if (x < n1) {
-            uint32_t v;
-            if (has_prev)
-                v = (uint32_t)top;
-            else
-                v = (P == WFK_ED && (x >= 1 || textbook)) ? 1u : 0u;
-            sh.ring[0][(x + 64) & (RS - 1)] = (P == WFK_ED)
-                                                  ? make_int2((int)((v & 1u) << 31), (int)(((v >> 1) & 1u) << 31))
-                                                  : make_int2((int)((v & 1u) << 31), 0);
+        uint32_t plus, minus = 0;
+        if (has_prev) {
+            plus = ((uint32_t)__shfl((int)(uint32_t)top, word_of * NP) >> bit_of) & 1u;
+            if (ED) minus = ((uint32_t)__shfl((int)(uint32_t)top, word_of * NP + 1) >> bit_of) & 1u;
+        } else {
+            plus = (ED && (c * K + lane >= 1 || textbook)) ? 1u : 0u;
         }
+        put_inj(c, 0, plus, minus);  // wave 0 runs chunk c in iteration c
         return true;
     };
-    // Masks of iteration `it`: compute wave w runs chunk it - w*D; its lane
-    // l at step q reads column (it - w*D)*K + q - l (codes of columns
-    // outside the pair are stale, masked to a table row; those steps keep
-    // their state).
+    // Iteration `it`: compute wave w runs chunk it - w*D; its lane l at step q
+    // reads column (it - w*D)*K + q - l (codes of columns outside the pair are
+    // stale, masked to a table row; those steps keep their state).
     auto produce = [&](int it) {
         for (int w = 0; w < wa; ++w) {
             const int c = it - w * kD;
             if (c < 0 || c >= nch) continue;
+            if (w > 0) {
+                const int2 v = sh.cap[w - 1][(2 * c + 1 + word_of) & 7];
+                put_inj(it, w, ((uint32_t)v.x >> bit_of) & 1u, ((uint32_t)v.y >> bit_of) & 1u);
+            }
             const uint32_t *cp = sh.aw + ((c * K - lane) & (AW - 1));
             const int *pq = sh.peq[w] + lane;
             int4 *d = &sh.eqb[it & 1][w][0][lane];
@@ -617,6 +650,14 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
             for (int gq = 0; gq < K / 4; ++gq) d[gq * 64] = make_int4(e[4 * gq], e[4 * gq + 1], e[4 * gq + 2], e[4 * gq + 3]);
         }
     };
+    // The last compute wave's chunk c, to HBM for the strip below.
+    auto publish = [&](int c) {
+        if (lane < 2 * NP) {
+            const int2 v = sh.cap[W - 1][(2 * c + lane / NP) & 7];
+            __hip_atomic_store(bnext + 2 * c * NP + lane, tag | (uint32_t)((lane % NP) ? v.y : v.x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+    };
 
     __syncthreads();  // match-mask tables built
     uint32_t code_next = 0u;  // stager: codes of chunk j + 2, loaded in iteration j
@@ -628,22 +669,6 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
     }
     __syncthreads();
 
-    int copied = 0;  // stager: columns already stored to bnext
-    auto copy_out = [&](int upto, bool from_ring) {
-        while (copied < upto) {
-            const int x = copied + lane;
-            if (x < upto) {
-                uint32_t v = 0;
-                if (from_ring) {
-                    const int2 w = sh.ring[W][(x + 64) & (RS - 1)];
-                    v = (P == WFK_ED) ? (((uint32_t)w.x >> 31) | (((uint32_t)w.y >> 31) << 1)) : ((uint32_t)w.x >> 31);
-                }
-                __hip_atomic_store(bnext + x, tag | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            copied = min(upto, copied + 64);
-        }
-    };
-
     BpState st;
     st.pv = 0xffffffffu;  // ED: column 0 rises by 1 per row; LCS: V = all ones
     st.mv = 0u;
@@ -653,12 +678,10 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
     bool aborted = sh.abort_at <= -1;
     for (int j = 0; j < total && !aborted; ++j) {
         if (stager) {
-            // The bottom row's columns the last compute wave finished in
-            // iteration j - 1, to HBM for the strip below (here rather than
-            // in that wave, whose next chunk would otherwise wait for the
-            // stores to complete).
+            // (Here rather than in the compute wave, whose next chunk would
+            // otherwise wait for the stores to complete.)
             const int cl = j - 1 - (wa - 1) * kD;
-            if (has_next && cl >= 0 && cl < nch) copy_out(min(n1, cl * K + K - 63), true);
+            if (has_next && cl >= 0 && cl < nch) publish(cl);
             if (j + 1 < nch) put_code(j + 1, code_next);
             if (j + 2 < nch) code_next = load_code(j + 2);
             const uint64_t top = (j + 1 < nch) ? load_top(j + 1) : tag;
@@ -670,10 +693,14 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
                 const int s0 = cj * K;
                 const bool steady = (s0 >= 63) && (s0 + K - 1 <= n1 - 1);
                 const int4 *eqw = &sh.eqb[j & 1][wave][0][0];
+                const int2 *inj = sh.injb[j & 1][wave];
+                // (In the dummy, lanes 62 and 63 of different waves overlap:
+                // nobody reads it.)
+                int2 *cap = lane == 63 ? &sh.cap[wave][(2 * cj) & 7] : &sh.dummy[lane];
                 if (steady)
-                    bs_chunk<P, K, RS, false>(st, s0, lane, n1, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave], eqw);
+                    bs_chunk<P, K, false>(st, s0, lane, n1, inj, cap, eqw);
                 else
-                    bs_chunk<P, K, RS, true>(st, s0, lane, n1, sh.ring[wave], sh.ring[wave + 1], sh.dummy[wave], eqw);
+                    bs_chunk<P, K, true>(st, s0, lane, n1, inj, cap, eqw);
             }
         }
         __syncthreads();
@@ -682,10 +709,13 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
 
     if (aborted) {
         if (threadIdx.x == 0) atomicOr(&ka.res[pair].status, 1);
-        if (stager && has_next) copy_out(n1, false);
+        // Placeholders release the strip below.
+        if (stager && has_next)
+            for (int k = lane; k < 2 * nch * NP; k += 64)
+                __hip_atomic_store(bnext + k, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
-    if (stager && has_next) copy_out(n1, true);
+    if (stager && has_next) publish(nch - 1);
 
     if (active) {
         int v;
