@@ -941,44 +941,70 @@ int ensure_pinned(wf_ctx *ctx, size_t bytes)
     return WF_OK;
 }
 
-// Byte offsets of a plan's buffers in the pinned block: codes, splits,
-// pairs, tasks, then the results.
-struct PinnedLayout {
-    size_t codes = 0, splits, pairs, tasks, res, end;
-    explicit PinnedLayout(const WfPlanHost *ph)
+// Byte offsets of a call's buffers in the pinned block and, alike, in the
+// device block it is copied to: codes, splits and cuts, pairs, tasks, the
+// cleared results and claim counters, the launch epoch.
+struct BlockLayout {
+    size_t codes = 0, splits, pairs, tasks, res, counters, epoch, end;
+    explicit BlockLayout(const WfPlanHost *ph)
     {
+        WfPlanBytes nb;
+        wf_plan_bytes(ph, &nb);
         splits = round256(ph->codes.size());
-        pairs = splits + round256(wf_cuts_offset(ph) + ph->cuts.size() * sizeof(WfCutDev));
-        tasks = pairs + round256(ph->pairs.size() * sizeof(WfPairDev));
-        res = tasks + round256(ph->tasks.size() * sizeof(WfTaskDev));
-        end = res + round256((size_t)std::max<int64_t>(1, ph->npairs) * sizeof(WfResultDev));
+        pairs = splits + round256(ph->splits.empty() ? 0 : nb.splits);
+        tasks = pairs + round256(nb.pairs);
+        res = tasks + round256(nb.tasks);
+        counters = res + round256(nb.res);
+        epoch = counters + round256(nb.counters);
+        end = epoch + 256;
     }
 };
 
-// wf_upload_plan through the context's pinned block: the copies are
-// asynchronous DMA from pinned memory, and the stream orders them before
-// the launch, so the host does not wait for them.  The block must not be
-// rewritten before the stream has drained (wf_align_batch synchronises
-// before it returns).
-int upload_pinned(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar)
+// A call's plan to the device in one copy: the plan is laid out in the
+// context's pinned block, results and counters cleared and the epoch set, and
+// one asynchronous DMA takes the block to its twin in HBM, which `ar` then
+// points into (nothing may release or grow those buffers).  Against a copy per
+// buffer and a reset kernel a 256-symbol pair's call loses four launches.  The
+// stream orders the copy before the launch; the block must not be rewritten
+// before the stream has drained (wf_align_batch synchronises before it
+// returns).
+int upload_block(wf_ctx *ctx, WfPlanHost *ph, const BlockLayout &L, WfArenas *ar)
 {
+    WfArenas *sc = &ctx->scratch;
+    WfPlanBytes nb;
+    wf_plan_bytes(ph, &nb);
     int st;
-    if ((st = ensure_arenas(ph, ar)) != WF_OK) return st;
-    const PinnedLayout L(ph);
+    if ((st = sc->codes.ensure(L.end)) != WF_OK) return st;
+    if ((st = sc->bnd.ensure(nb.bnd, true)) != WF_OK) return st;
+    if ((st = sc->colw.ensure(nb.colw)) != WF_OK) return st;
     if ((st = ensure_pinned(ctx, L.end)) != WF_OK) return st;
     ctx->pinned_busy = true;
-    auto put = [&](size_t off, void *dst, const void *src, size_t n) -> bool {
-        if (!n) return true;
-        std::memcpy(ctx->pinned + off, src, n);
-        return hipMemcpyAsync(dst, ctx->pinned + off, n, hipMemcpyHostToDevice, ctx->stream) == hipSuccess;
+    uint8_t *p = ctx->pinned;
+    auto put = [&](size_t off, const void *src, size_t n) {
+        if (n) std::memcpy(p + off, src, n);
     };
-    if (!put(L.codes, ar->codes.ptr, ph->codes.data(), ph->codes.size()) ||
-        !put(L.splits, ar->splits.ptr, ph->splits.data(), ph->splits.size() * sizeof(WfSplitDev)) ||
-        !put(L.splits + wf_cuts_offset(ph), (uint8_t *)ar->splits.ptr + wf_cuts_offset(ph), ph->cuts.data(),
-             ph->cuts.size() * sizeof(WfCutDev)) ||
-        !put(L.pairs, ar->pairs.ptr, ph->pairs.data(), ph->pairs.size() * sizeof(WfPairDev)) ||
-        !put(L.tasks, ar->tasks.ptr, ph->tasks.data(), ph->tasks.size() * sizeof(WfTaskDev)))
-        return WF_ERR_DEVICE;
+    put(L.codes, ph->codes.data(), ph->codes.size());
+    put(L.splits, ph->splits.data(), ph->splits.size() * sizeof(WfSplitDev));
+    put(L.splits + wf_cuts_offset(ph), ph->cuts.data(), ph->cuts.size() * sizeof(WfCutDev));
+    put(L.pairs, ph->pairs.data(), ph->pairs.size() * sizeof(WfPairDev));
+    put(L.tasks, ph->tasks.data(), ph->tasks.size() * sizeof(WfTaskDev));
+    std::memset(p + L.res, 0, L.epoch - L.res);
+    // Tags of calls have the top bit set, those of the sweeps and table dumps
+    // that share the boundary rows, counted on the device, do not.
+    ctx->calls = (ctx->calls + 1) & 0x7fffffffu;
+    const uint32_t epoch = 0x80000000u | ctx->calls;
+    put(L.epoch, &epoch, sizeof(epoch));
+    if (hipMemcpyAsync(sc->codes.ptr, p, L.end, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
+    auto at = [&](size_t off) { return (void *)((uint8_t *)sc->codes.ptr + off); };
+    ar->codes.ptr = at(L.codes);
+    ar->splits.ptr = at(L.splits);
+    ar->pairs.ptr = at(L.pairs);
+    ar->tasks.ptr = at(L.tasks);
+    ar->res.ptr = at(L.res);
+    ar->counters.ptr = at(L.counters);
+    ar->epoch.ptr = at(L.epoch);
+    ar->bnd = sc->bnd;
+    ar->colw = sc->colw;
     return WF_OK;
 }
 
@@ -1027,12 +1053,13 @@ static int enqueue_engine(WfPlanHost *ph, const WfVariant *v, int lim, int mode,
 
 // Enqueue the reset kernel and the engine launch(es) of a plan on the
 // context stream (also used inside hipGraph capture: no memset nodes, and
-// the epoch that tags boundary values is advanced on the device).
-int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int maxg, hipStream_t stream)
+// the epoch that tags boundary values is advanced on the device).  `reset`
+// false: results, counters and the epoch came with the plan's upload.
+int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int maxg, hipStream_t stream, bool reset)
 {
     const int64_t ncounters = ph->npairs + 1;
-    if (wf_launch_reset((WfResultDev *)ar->res.ptr, ph->npairs, (int32_t *)ar->counters.ptr, ncounters,
-                        (uint32_t *)ar->epoch.ptr, stream) != hipSuccess)
+    if (reset && wf_launch_reset((WfResultDev *)ar->res.ptr, ph->npairs, (int32_t *)ar->counters.ptr, ncounters,
+                                 (uint32_t *)ar->epoch.ptr, stream) != hipSuccess)
         return WF_ERR_DEVICE;
     WfKernelArgs ka{};
     ka.pairs = (const WfPairDev *)ar->pairs.ptr;
@@ -1231,18 +1258,23 @@ int wf_align_batch(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile
     WfPlanHost ph;
     int st = wf_build_plan(ctx, jobs, njobs, tile, &ph);
     if (st != WF_OK) return st;
-    if ((st = upload_pinned(ctx, &ph, &ctx->scratch)) != WF_OK) return st;
-    double ms = 0.0;
-    if ((st = wf_run_plan(ctx, &ph, &ctx->scratch, WF_RUN_PERSISTENT, &ms, nullptr)) != WF_OK) return st;
-    // Results into the pinned block (its upload part is no longer read).
-    const PinnedLayout L(&ph);
+    const BlockLayout L(&ph);
+    WfArenas ar;
+    if ((st = upload_block(ctx, &ph, L, &ar)) != WF_OK) return st;
+    if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
+    if ((st = wf_enqueue_plan(ctx, &ph, &ar, WF_RUN_PERSISTENT, wf_max_resident_groups(ctx, ph.variant), ctx->stream,
+                              false)) != WF_OK)
+        return st;
+    if (hipEventRecord(ctx->ev1, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
+    // Results into the pinned block (its upload part is no longer read by
+    // then), behind the launch: one wait for everything.
     WfResultDev *r = reinterpret_cast<WfResultDev *>(ctx->pinned + L.res);
-    if (ph.npairs > 0 &&
-        (hipMemcpyAsync(r, ctx->scratch.res.ptr, ph.npairs * sizeof(WfResultDev), hipMemcpyDeviceToHost,
-                        ctx->stream) != hipSuccess ||
-         hipStreamSynchronize(ctx->stream) != hipSuccess))
+    if (hipMemcpyAsync(r, ar.res.ptr, ph.npairs * sizeof(WfResultDev), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess)
         return WF_ERR_DEVICE;
     ctx->pinned_busy = false;
+    float ms = 0.f;
+    if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
     return fill_results(&ph, r, ms, out, njobs);
 }
 

@@ -77,6 +77,7 @@ struct wf_ctx {
     // grown on demand, freed with the context).
     uint8_t *pinned = nullptr;
     size_t pinned_cap = 0;
+    uint32_t calls = 0;        // wf_align / wf_align_batch calls so far (their launch epochs)
     bool pinned_busy = false;  // copies from or to the block may be in flight on `stream`
 };
 
@@ -138,7 +139,8 @@ int wf_copy_plan(WfPlanHost *ph, WfArenas *ar, hipStream_t stream);
 int wf_upload_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar);
 int wf_upload_plan_async(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, hipStream_t stream, bool sync);
 int wf_max_resident_groups(wf_ctx *ctx, const WfVariant *v);
-int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int maxg, hipStream_t stream);
+int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int maxg, hipStream_t stream,
+                    bool reset = true);
 // Reset + engine launch(es) (or a captured graph), timed with HIP events on
 // the context stream; returns after the stream has drained.
 int wf_run_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, double *kernel_ms, hipGraphExec_t exec);
