@@ -34,6 +34,7 @@ struct wf_plan {
     WfPlanHost host;
     double kernel_ms = 0.0;
     bool ran = false;
+    std::vector<WfResultDev> res;                  // of the last run
     hipGraph_t graph[2] = {nullptr, nullptr};      // per run mode, when captured
     hipGraphExec_t exec[2] = {nullptr, nullptr};
 };
@@ -916,13 +917,11 @@ int wf_upload_plan_async(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, hipStream_t 
     return WF_OK;
 }
 
-namespace {
-
-size_t round256(size_t n) { return (n + 255) & ~size_t(255); }
+static size_t round256(size_t n) { return (n + 255) & ~size_t(255); }
 
 // The context's pinned block, at least `bytes` long and idle (a call that
 // failed after queueing its copies may have left them in flight).
-int ensure_pinned(wf_ctx *ctx, size_t bytes)
+int wf_ensure_pinned(wf_ctx *ctx, size_t bytes)
 {
     if (ctx->pinned_busy) {
         if (hipStreamSynchronize(ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
@@ -940,6 +939,8 @@ int ensure_pinned(wf_ctx *ctx, size_t bytes)
     ctx->pinned_cap = cap;
     return WF_OK;
 }
+
+namespace {
 
 // Byte offsets of a call's buffers in the pinned block and, alike, in the
 // device block it is copied to: codes, splits and cuts, pairs, tasks, the
@@ -977,7 +978,7 @@ int upload_block(wf_ctx *ctx, WfPlanHost *ph, const BlockLayout &L, WfArenas *ar
     if ((st = sc->codes.ensure(L.end)) != WF_OK) return st;
     if ((st = sc->bnd.ensure(nb.bnd, true)) != WF_OK) return st;
     if ((st = sc->colw.ensure(nb.colw)) != WF_OK) return st;
-    if ((st = ensure_pinned(ctx, L.end)) != WF_OK) return st;
+    if ((st = wf_ensure_pinned(ctx, L.end)) != WF_OK) return st;
     ctx->pinned_busy = true;
     uint8_t *p = ctx->pinned;
     auto put = [&](size_t off, const void *src, size_t n) {
@@ -1095,20 +1096,35 @@ int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int max
     return WF_OK;
 }
 
-// Run a plan (directly, or by replaying its captured graph) and time the
-// device work with HIP events on the context stream.
-int wf_run_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, double *kernel_ms, hipGraphExec_t exec)
+// Run a plan (directly, or by replaying its captured graph), time the device
+// work with HIP events on the context stream and bring its pairs' results,
+// which follow the launch through the context's pinned block, into `res`, if
+// not null: one wait for everything.
+int wf_run_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, double *kernel_ms, hipGraphExec_t exec,
+                std::vector<WfResultDev> *res)
 {
     const int maxg = wf_max_resident_groups(ctx, ph->variant);
+    const size_t bytes = res ? (size_t)ph->npairs * sizeof(WfResultDev) : 0;
+    int st;
+    if (bytes && (st = wf_ensure_pinned(ctx, bytes)) != WF_OK) return st;
     if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
     if (exec) {
         if (hipGraphLaunch(exec, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
-    } else {
-        const int st = wf_enqueue_plan(ctx, ph, ar, mode, maxg, ctx->stream);
-        if (st != WF_OK) return st;
+    } else if ((st = wf_enqueue_plan(ctx, ph, ar, mode, maxg, ctx->stream)) != WF_OK) {
+        return st;
     }
     if (hipEventRecord(ctx->ev1, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
-    if (hipEventSynchronize(ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
+    if (bytes) {
+        ctx->pinned_busy = true;
+        if (hipMemcpyAsync(ctx->pinned, ar->res.ptr, bytes, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
+            return WF_ERR_DEVICE;
+    }
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
+    if (bytes) {
+        ctx->pinned_busy = false;
+        const WfResultDev *r = reinterpret_cast<const WfResultDev *>(ctx->pinned);
+        res->assign(r, r + ph->npairs);
+    }
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
     *kernel_ms = ms;
@@ -1116,7 +1132,7 @@ int wf_run_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, double *ker
 }
 
 // The caller's results from the device results r of the plan's pairs.
-static int fill_results(const WfPlanHost *ph, const WfResultDev *r, double kernel_ms, wf_result *out, int64_t n)
+int wf_fill_results(const WfPlanHost *ph, const WfResultDev *r, double kernel_ms, wf_result *out, int64_t n)
 {
     int worst = WF_OK;
     for (int64_t i = 0; i < std::min(n, ph->njobs); ++i) {
@@ -1146,7 +1162,7 @@ int wf_download_results(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, double kernel
             hipSuccess)
         return WF_ERR_DEVICE;
     (void)ctx;
-    return fill_results(ph, r.data(), kernel_ms, out, n);
+    return wf_fill_results(ph, r.data(), kernel_ms, out, n);
 }
 
 // ----------------------------------------------------------------------------
@@ -1275,7 +1291,7 @@ int wf_align_batch(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile
     ctx->pinned_busy = false;
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
-    return fill_results(&ph, r, ms, out, njobs);
+    return wf_fill_results(&ph, r, ms, out, njobs);
 }
 
 int wf_align(wf_ctx *ctx, int problem, const int32_t *a, int64_t n1, const int32_t *b, int64_t n2,
@@ -1396,6 +1412,7 @@ int wf_plan_create(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile
     p->ctx = ctx;
     int st = wf_build_plan(ctx, jobs, njobs, tile, &p->host);
     if (st == WF_OK) st = wf_upload_plan(ctx, &p->host, &p->own);
+    if (st == WF_OK) st = wf_ensure_pinned(ctx, (size_t)p->host.npairs * sizeof(WfResultDev));
     if (st != WF_OK) {
         p->own.release();
         delete p;
@@ -1409,7 +1426,8 @@ int wf_plan_run(wf_plan *plan, int mode)
 {
     if (!plan || (mode != WF_RUN_PERSISTENT && mode != WF_RUN_PER_PAIR)) return WF_ERR_INVALID;
     if (hipSetDevice(plan->ctx->device) != hipSuccess) return WF_ERR_DEVICE;
-    const int st = wf_run_plan(plan->ctx, &plan->host, &plan->own, mode, &plan->kernel_ms, plan->exec[mode]);
+    const int st = wf_run_plan(plan->ctx, &plan->host, &plan->own, mode, &plan->kernel_ms, plan->exec[mode],
+                               &plan->res);
     plan->ran = (st == WF_OK);
     return st;
 }
@@ -1444,8 +1462,7 @@ int wf_plan_results(wf_plan *plan, wf_result *out, int64_t n)
 {
     if (!plan || !out || n < 0) return WF_ERR_INVALID;
     if (!plan->ran) return WF_ERR_INVALID;
-    if (hipSetDevice(plan->ctx->device) != hipSuccess) return WF_ERR_DEVICE;
-    return wf_download_results(plan->ctx, &plan->host, &plan->own, plan->kernel_ms, out, n);
+    return wf_fill_results(&plan->host, plan->res.data(), plan->kernel_ms, out, n);
 }
 
 double wf_plan_kernel_ms(const wf_plan *plan) { return plan ? plan->kernel_ms : -1.0; }

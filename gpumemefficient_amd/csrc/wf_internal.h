@@ -73,8 +73,8 @@ struct wf_ctx {
     double timeout_s = 10.0;
     WfArenas scratch;    // used by wf_align / wf_align_batch
     // Pinned host block of wf_align / wf_align_batch: stages a plan's codes
-    // and descriptors for upload and receives the results (hipHostMalloc,
-    // grown on demand, freed with the context).
+    // and descriptors for upload and receives the results, also the sweeps'
+    // (hipHostMalloc, grown on demand, freed with the context).
     uint8_t *pinned = nullptr;
     size_t pinned_cap = 0;
     uint32_t calls = 0;        // wf_align / wf_align_batch calls so far (their launch epochs)
@@ -138,12 +138,18 @@ void wf_plan_bytes(const WfPlanHost *ph, WfPlanBytes *b);
 int wf_copy_plan(WfPlanHost *ph, WfArenas *ar, hipStream_t stream);
 int wf_upload_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar);
 int wf_upload_plan_async(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, hipStream_t stream, bool sync);
+// The context's pinned block, at least `bytes` long and idle.
+int wf_ensure_pinned(wf_ctx *ctx, size_t bytes);
 int wf_max_resident_groups(wf_ctx *ctx, const WfVariant *v);
 int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int maxg, hipStream_t stream,
                     bool reset = true);
 // Reset + engine launch(es) (or a captured graph), timed with HIP events on
-// the context stream; returns after the stream has drained.
-int wf_run_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, double *kernel_ms, hipGraphExec_t exec);
+// the context stream; the pairs' results to `res`, if not null; returns after the
+// stream has drained.
+int wf_run_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, double *kernel_ms, hipGraphExec_t exec,
+                std::vector<WfResultDev> *res);
+// The caller's results from the device results r of the plan's pairs.
+int wf_fill_results(const WfPlanHost *ph, const WfResultDev *r, double kernel_ms, wf_result *out, int64_t n);
 // wf_noalloc.hip: device address of this device's static scratch array
 // (looked up and cleared on the first call per device).
 int wf_noalloc_setup(int device, hipStream_t stream, uint8_t **out);

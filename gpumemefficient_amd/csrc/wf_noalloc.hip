@@ -125,6 +125,8 @@ extern "C" int wf_align_noalloc(wf_ctx *ctx, int problem, const int32_t *a, int6
     // The arenas point into `scratch`: nothing here may release or grow them.
     if ((st = wf_copy_plan(&ph, &ar, ctx->stream)) != WF_OK) return st;
     double ms = 0.0;
-    if ((st = wf_run_plan(ctx, &ph, &ar, WF_RUN_PERSISTENT, &ms, nullptr)) != WF_OK) return st;
+    // (No results through the context's pinned block: this call allocates
+    // nothing.)
+    if ((st = wf_run_plan(ctx, &ph, &ar, WF_RUN_PERSISTENT, &ms, nullptr, nullptr)) != WF_OK) return st;
     return wf_download_results(ctx, &ph, &ar, ms, out, 1);
 }

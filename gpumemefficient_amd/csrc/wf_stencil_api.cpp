@@ -21,27 +21,37 @@ int check_tile(const wf_tile *tile)
     return WF_OK;
 }
 
-// Reset, one launch and the wait of a sweep, timed with HIP events.
+// Reset and one launch of a sweep, timed with HIP events; the status and the
+// table's last interior cell come back behind it through the context's pinned
+// block, with one wait for everything.
 template <class Launch>
-int run_timed(wf_ctx *ctx, WfArenas *ar, double *ms, Launch &&launch)
+int run_timed(wf_ctx *ctx, WfArenas *ar, const int32_t *cell, double *ms, int32_t *last, Launch &&launch)
 {
+    int st;
+    if ((st = wf_ensure_pinned(ctx, 256)) != WF_OK) return st;
+    WfResultDev *r = reinterpret_cast<WfResultDev *>(ctx->pinned);
+    int32_t *l = reinterpret_cast<int32_t *>(ctx->pinned + 128);
     if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
     if (wf_launch_reset((WfResultDev *)ar->res.ptr, 1, (int32_t *)ar->counters.ptr, 2, (uint32_t *)ar->epoch.ptr,
                         ctx->stream) != hipSuccess)
         return WF_ERR_DEVICE;
     if (launch() != hipSuccess) return WF_ERR_DEVICE;
     if (hipEventRecord(ctx->ev1, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
-    if (hipEventSynchronize(ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
+    ctx->pinned_busy = true;
+    if (hipMemcpyAsync(r, ar->res.ptr, sizeof(*r), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+        hipMemcpyAsync(l, cell, sizeof(*l), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess)
+        return WF_ERR_DEVICE;
+    ctx->pinned_busy = false;
     float f = 0.f;
     if (hipEventElapsedTime(&f, ctx->ev0, ctx->ev1) != hipSuccess) return WF_ERR_DEVICE;
     *ms = f;
-    WfResultDev r{};
-    if (hipMemcpy(&r, ar->res.ptr, sizeof(r), hipMemcpyDeviceToHost) != hipSuccess) return WF_ERR_DEVICE;
-    return r.status ? WF_ERR_TIMEOUT : WF_OK;
+    *last = *l;
+    return r->status ? WF_ERR_TIMEOUT : WF_OK;
 }
 
 // The summed-area table: tiles instead of strips (wf_sat.hip).
-int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double *ms)
+int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double *ms, int32_t *last)
 {
     WfArenas *ar = &ctx->scratch;
     const int cus = ctx->prop.multiProcessorCount;
@@ -66,15 +76,18 @@ int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double
     a.epoch = (const uint32_t *)ar->epoch.ptr;
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
     const int grid = (int)std::min<int64_t>(ntr * ntc, std::max(1, wf_sat_resident(cus)));
-    return run_timed(ctx, ar, ms, [&] { return wf_launch_sat(grid, &a, ctx->stream); });
+    return run_timed(ctx, ar, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_sat(grid, &a, ctx->stream); });
 }
 
-// The sweep on a device table (pitch ld, ld % 4 == 0, 16-byte aligned).
-int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double *ms)
+// The sweep on a device table (pitch ld, ld % 4 == 0, 16-byte aligned); last:
+// its cell (n2, n1).
+int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double *ms, int32_t *last)
 {
     *ms = 0.0;
-    if (n1 == 0 || n2 == 0) return WF_OK;
-    if (op == WF_SAT) return run_sat(ctx, n1, n2, dt, ld, ms);
+    if (n1 == 0 || n2 == 0)  // no interior: the cell (n2, n1) is a boundary value
+        return hipMemcpy(last, dt + n2 * ld + n1, sizeof(*last), hipMemcpyDeviceToHost) == hipSuccess ? WF_OK
+                                                                                                      : WF_ERR_DEVICE;
+    if (op == WF_SAT) return run_sat(ctx, n1, n2, dt, ld, ms, last);
     WfArenas *ar = &ctx->scratch;
     const int64_t strips = (n2 + WFS_SOR_STRIP_ROWS - 1) / WFS_SOR_STRIP_ROWS;
     int st;
@@ -97,7 +110,7 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
     const int lim = wf_stencil_resident(ctx->prop.multiProcessorCount);
     const int grid = (int)std::min<int64_t>(strips, std::max(1, lim));
-    return run_timed(ctx, ar, ms, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
+    return run_timed(ctx, ar, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
 }
 
 // Host table -> device copy of pitch ldd -> sweep -> host table (or only the
@@ -110,17 +123,12 @@ int upload_run_download(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *ta
                     (size_t)cols * sizeof(int32_t), (size_t)rows, hipMemcpyHostToDevice) != hipSuccess)
         return WF_ERR_DEVICE;
     double ms = 0.0;
-    const int st = run_device(ctx, op, n1, n2, d, ldd, &ms);
+    const int st = run_device(ctx, op, n1, n2, d, ldd, &ms, &out->last);
     out->kernel_ms = ms;
-    if (st != WF_OK) return st;
-    if (no_copyback)
-        return hipMemcpy(&out->last, d + n2 * ldd + n1, sizeof(int32_t), hipMemcpyDeviceToHost) == hipSuccess
-                   ? WF_OK
-                   : WF_ERR_DEVICE;
+    if (st != WF_OK || no_copyback) return st;
     if (hipMemcpy2D(table, (size_t)ld * sizeof(int32_t), d, (size_t)ldd * sizeof(int32_t),
                     (size_t)cols * sizeof(int32_t), (size_t)rows, hipMemcpyDeviceToHost) != hipSuccess)
         return WF_ERR_DEVICE;
-    out->last = table[n2 * ld + n1];
     return WF_OK;
 }
 
@@ -148,12 +156,9 @@ int wf_stencil_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dev_
     int st = check_tile(tile);
     if (st != WF_OK) return st;
     double ms = 0.0;
-    st = run_device(ctx, op, n1, n2, dev_table, ld, &ms);
+    st = run_device(ctx, op, n1, n2, dev_table, ld, &ms, &out->last);
     out->kernel_ms = ms;
-    if (st != WF_OK) return st;
-    if (hipMemcpy(&out->last, dev_table + n2 * ld + n1, sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess)
-        return WF_ERR_DEVICE;
-    return WF_OK;
+    return st;
 }
 
 int wf_stencil(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *table, int64_t ld, const wf_tile *tile,
