@@ -43,9 +43,34 @@ def _stencil_id(op) -> int:
     return int(op)
 
 
+_I32 = np.dtype(np.int32)
+
+
+def _view_dtype(struct) -> np.dtype:
+    """The numpy dtype of a ctypes structure of integers, doubles and pointers
+    (as addresses)."""
+    names = [f for f, _ in struct._fields_]
+    formats = [np.uintp if issubclass(t, C._Pointer) else np.dtype(t) for _, t in struct._fields_]
+    return np.dtype({"names": names, "formats": formats, "offsets": [getattr(struct, f).offset for f in names],
+                     "itemsize": C.sizeof(struct)})
+
+
+_JOB = _view_dtype(_lib.wf_job)
+_RESULT = _view_dtype(_lib.wf_result)
+
+
 def _as_i32(x) -> np.ndarray:
+    if type(x) is np.ndarray and x.ndim == 1 and x.dtype == _I32 and x.flags.c_contiguous:
+        return x  # already what C reads
     arr = np.ascontiguousarray(np.asarray(x, dtype=np.int32).reshape(-1))
     return arr
+
+
+def _address(arr: np.ndarray) -> int:
+    try:
+        return C.addressof(C.c_char.from_buffer(arr))  # 0.2 us, against 1.0 for arr.ctypes.data
+    except (TypeError, ValueError):  # read-only, empty
+        return arr.ctypes.data
 
 
 def _ptr(arr: np.ndarray):
@@ -63,6 +88,12 @@ class Result:
     @classmethod
     def _from(cls, r: _lib.wf_result) -> "Result":
         return cls(int(r.last), int(r.max_score), int(r.status), float(r.kernel_ms), int(r.cells))
+
+    @classmethod
+    def _list(cls, out) -> "list[Result]":
+        """The results of a wf_result array, converted a field at a time."""
+        v = np.frombuffer(out, dtype=_RESULT)
+        return list(map(cls, *(v[f].tolist() for f in ("last", "max_score", "status", "kernel_ms", "cells"))))
 
 
 @dataclass
@@ -109,18 +140,28 @@ class Job:
 
 
 class _JobArray:
-    """Keeps the int32 arrays alive while C holds pointers into them."""
+    """Keeps the int32 arrays alive while C holds pointers into them.
+
+    The wf_job array is filled a field at a time: one ctypes structure a job,
+    with its two typed pointers, cost 7.9 us a job against 1.5."""
 
     def __init__(self, jobs: Iterable[Job]):
-        self.arrays = []
         jl = list(jobs)
-        self.c = (_lib.wf_job * max(1, len(jl)))()
-        for i, j in enumerate(jl):
-            a, b = _as_i32(j.a), _as_i32(j.b)
-            self.arrays += [a, b]
-            flags = (_lib.WF_TILE_ED_TEXTBOOK if j.ed_textbook else 0) | (_lib.WF_TILE_NO_MAX if j.no_max else 0)
-            self.c[i] = _lib.wf_job(_problem_id(j.problem), flags, _ptr(a), a.size, _ptr(b), b.size)
         self.n = len(jl)
+        self.c = (_lib.wf_job * max(1, self.n))()
+        a = [_as_i32(j.a) for j in jl]
+        b = [_as_i32(j.b) for j in jl]
+        self.arrays = a + b
+        if not jl:
+            return
+        v = np.frombuffer(self.c, dtype=_JOB)
+        v["problem"] = [_problem_id(j.problem) for j in jl]
+        v["flags"] = [(_lib.WF_TILE_ED_TEXTBOOK if j.ed_textbook else 0) | (_lib.WF_TILE_NO_MAX if j.no_max else 0)
+                      for j in jl]
+        v["a"] = [_address(x) for x in a]
+        v["n1"] = [x.size for x in a]
+        v["b"] = [_address(x) for x in b]
+        v["n2"] = [x.size for x in b]
 
 
 class Plan:
@@ -155,7 +196,7 @@ class Plan:
         st = self.ctx._lib.wf_plan_results(self._h, out, self.n)
         if raise_on_error:
             check(st, "wf_plan_results")
-        return [Result._from(out[i]) for i in range(self.n)]
+        return Result._list(out)[:self.n]
 
     def describe(self) -> dict:
         e, r, w, k, g = C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32()
@@ -259,7 +300,7 @@ class Context:
         out = (_lib.wf_result * max(1, ja.n))()
         t = tile._c() if tile else None
         check(self._lib.wf_align_batch(self._h, ja.c, ja.n, C.byref(t) if t else None, out), "wf_align_batch")
-        return [Result._from(out[i]) for i in range(ja.n)]
+        return Result._list(out)[:ja.n]
 
     def plan(self, jobs: Iterable[Job], tile: Tile | None = None) -> Plan:
         return Plan(self, jobs, tile)
