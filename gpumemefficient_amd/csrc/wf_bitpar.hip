@@ -92,6 +92,15 @@ struct BpState {
     int ph, mh;        // ED: this column's horizontal deltas (pre-shift); LCS: ph = carry out in bit 31
 };
 
+// A state word that the next step reads in one register.  Without it the compiler
+// keeps its terms apart to fold them into the next step's three-input operations:
+// a shorter chain, but an operation more a step, and issue is what bounds a wave
+// (staged, one pair: LCS 32768^2 0.398 -> 0.375 ms, ED 65536^2 1.33 -> 1.30).
+__device__ __forceinline__ void one_form(uint32_t &w)
+{
+    asm("" : "+v"(w));
+}
+
 template <int P>
 __device__ __forceinline__ void bp_step(BpState &st, int2 inj, uint32_t eq)
 {
@@ -111,6 +120,8 @@ __device__ __forceinline__ void bp_step(BpState &st, int2 inj, uint32_t eq)
         const uint32_t mhs = __builtin_amdgcn_alignbit(mh, (uint32_t)nmh, 31);
         st.pv = mhs | ~(xv | phs);
         st.mv = phs & xv;
+        one_form(st.pv);
+        one_form(st.mv);
         st.ph = (int)ph;
         st.mh = (int)mh;
     } else {
@@ -123,6 +134,7 @@ __device__ __forceinline__ void bp_step(BpState &st, int2 inj, uint32_t eq)
         // carry into it, (V & U) | ((V | U) & ~sum), with U = V & Eq.
         st.ph = (int)(st.pv & (eq | ~sum));
         st.pv = sum | (st.pv & ~eq);
+        one_form(st.pv);
     }
 }
 
@@ -425,12 +437,13 @@ __global__ __launch_bounds__(64 * W) void wf_engine_bitpar(WfKernelArgs ka)
 // the chip at once (single large pairs), and the engine above, which packs more
 // compute waves per CU, for throughput-bound batches.
 //
-// A step is bound by the issue of a lone wave (about 5 cycles an instruction):
-// 13 VALU operations for ED and 6 for LCS, one or two to collect what lane 63
-// hands down, and the LDS reads.  Per step, W = 1: ED 38.4 -> 33.1 ns, LCS 25.5 ->
-// 19.3 (before: every step's words stored to LDS, ED with one more operation);
-// ED 65536^2 1.51 -> 1.33 ms, LCS 32768^2 0.547 -> 0.399.  W = 2 overloads the one
-// staging wave.
+// A step is bound by the issue of a lone wave (4 cycles an instruction at best,
+// more where 8-byte instructions follow each other off their alignment): 13
+// VALU operations for ED and 6 for LCS, one or two to collect what lane 63
+// hands down, and the LDS reads.  Per step, W = 1: ED 38.4 -> 31.2 ns, LCS 25.5 ->
+// 16.7 (before: every step's words stored to LDS, ED with two more operations,
+// LCS with one, and the reads at their use); ED 65536^2 1.51 -> 1.25 ms, LCS
+// 32768^2 0.547 -> 0.353.  W = 2 overloads the one staging wave.
 // ---------------------------------------------------------------------------
 
 template <int W>
@@ -459,6 +472,8 @@ struct BsShared {
     int2 cap[W][8];
     int2 dummy[64];  // lanes 0..62 store here, so that the capture is one unmasked write
     int peq[W][32 * 64];  // as in BpShared
+    // Column codes as in BpShared, times 64 (a row of peq): two operations less a
+    // step for the staging wave, which bounds LCS (32768^2 0.363 -> 0.353 ms).
     uint32_t aw[AW + K];
     int task;
     int abort_at;
@@ -474,7 +489,7 @@ __device__ __forceinline__ int64_t bs_row_words(int n1) { return 4 * (int64_t)((
 // (`cap`: a dummy in the other lanes).  The bits are collected in a register
 // (one v_alignbit a step and word) and stored once per 32 steps: storing
 // every step's words instead took 55 cycles a step for LCS and 79 for ED where
-// this takes 39 and 70 (one wave, operands from LDS, no staging wave beside).
+// this took 39 and 70 (one wave, operands from LDS, no staging wave beside).
 template <int P, int K, bool MASKED>
 __device__ __forceinline__ void bs_chunk(BpState &st, int s0, int lane, int n1, const int2 *inj, int2 *cap,
                                          const int4 *eqw)
@@ -497,38 +512,46 @@ __device__ __forceinline__ void bs_chunk(BpState &st, int s0, int lane, int n1, 
         }
     };
     const int4 *ep = eqw + lane;
-    // Masks and lane 0's upper words are read one group of 4 steps ahead.
-    int4 eqv = ep[0];
-    int2 injv[4] = {};
-    load_inj(0, injv);
+    // Masks and lane 0's upper words are read A groups of 4 steps ahead, and
+    // held there: the compiler moves the reads down to their use, where each
+    // waits behind the staging wave's (0.375 -> 0.363 and 1.30 -> 1.26 ms; A = 1
+    // or 3 within 1%).
+    constexpr int A = 2;
+    int4 eqv[A + 1];
+    int2 injv[A + 1][4] = {};
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+        eqv[i] = ep[4 * i * 16];
+        load_inj(4 * i, injv[i]);
+    }
     uint32_t accp = 0, accm = 0;
 #pragma unroll
     for (int q = 0; q < K; q += 4) {
-        int4 eqn = make_int4(0, 0, 0, 0);
-        int2 injn[4] = {};
-        if (q + 4 < K) {
-            eqn = ep[(q + 4) * 16];
-            load_inj(q + 4, injn);
+        if (q + 4 * A < K) {
+            eqv[A] = ep[(q + 4 * A) * 16];
+            load_inj(q + 4 * A, injv[A]);
         }
-        const uint32_t e[4] = {(uint32_t)eqv.x, (uint32_t)eqv.y, (uint32_t)eqv.z, (uint32_t)eqv.w};
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t e[4] = {(uint32_t)eqv[0].x, (uint32_t)eqv[0].y, (uint32_t)eqv[0].z, (uint32_t)eqv[0].w};
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             if (MASKED) {
                 const bool valid = (unsigned)(s0 + q + u - lane) < (unsigned)n1;
                 BpState nx = st;
-                bp_step<P>(nx, injv[u], e[u]);
+                bp_step<P>(nx, injv[0][u], e[u]);
                 if (valid) st = nx;
             } else {
-                bp_step<P>(st, injv[u], e[u]);
+                bp_step<P>(st, injv[0][u], e[u]);
             }
             accp = __builtin_amdgcn_alignbit(accp, (uint32_t)st.ph, 31);
             if (ED) accm = __builtin_amdgcn_alignbit(accm, (uint32_t)st.mh, 31);
         }
         if (q % 32 == 28) cap[q / 32] = make_int2((int)accp, (int)accm);
-        if (q + 4 < K) {
-            eqv = eqn;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) injv[u] = injn[u];
+        for (int i = 0; i < A; ++i) {
+            eqv[i] = eqv[i + 1];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) injv[i][u] = injv[i + 1][u];
         }
     }
 }
@@ -584,8 +607,8 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
         const int x = c * K + lane;
         if (x < n1) {
             const int slot = x & (AW - 1);
-            sh.aw[slot] = code;
-            if (slot < K) sh.aw[AW + slot] = code;
+            sh.aw[slot] = (code & 31u) * 64;
+            if (slot < K) sh.aw[AW + slot] = (code & 31u) * 64;
         }
     };
     // Column c*K + q of chunk c is step c*K + q + 63 of lane 63 of the wave
@@ -645,7 +668,7 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
             for (int q = 0; q < K; ++q) code[q] = cp[q];
             int e[K];
 #pragma unroll
-            for (int q = 0; q < K; ++q) e[q] = pq[(code[q] & 31u) * 64];
+            for (int q = 0; q < K; ++q) e[q] = pq[code[q]];
 #pragma unroll
             for (int gq = 0; gq < K / 4; ++gq) d[gq * 64] = make_int4(e[4 * gq], e[4 * gq + 1], e[4 * gq + 2], e[4 * gq + 3]);
         }
