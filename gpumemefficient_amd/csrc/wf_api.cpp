@@ -528,10 +528,9 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
                     ++nextra;
                 }
     } else if (v->engine == WF_ENGINE_ASYNC && perm4 && split_enabled()) {
-        // SW pairs on the byte tables split in three (bottom-right cell
-        // only) or four (with the running maximum) pairs (WfSplitDev) when all
-        // of the launch's strips fit on the chip at once: the parts' strip
-        // chains run side by side.
+        // SW pairs split in three (bottom-right cell only) or four (with the
+        // running maximum) pairs (WfSplitDev) when all of the launch's strips
+        // fit on the chip at once: the parts' strip chains run side by side.
         int64_t strips = 0, extra = 0;
         std::vector<uint8_t> cand(njobs, 0);
         trial.resize(njobs);
@@ -546,12 +545,18 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
             // The trial encoding is kept for the plan's codes below.
             std::vector<uint8_t> t((size_t)(j.n1 + j.n2));
             int32_t mode = 0;
-            if (wf_encode_job(j, tile ? tile->flags : 0, perm4, t.data(), t.data() + j.n1, &mode) != WF_OK ||
-                !(mode & WFK_MODE_PERM4))
-                continue;
+            if (wf_encode_job(j, tile ? tile->flags : 0, perm4, t.data(), t.data() + j.n1, &mode) != WF_OK) continue;
             trial[i] = std::move(t);
             trial_mode[i] = mode;
-            cand[i] = nomax ? 2 : 3;  // extra pairs
+            // Compared codes (7013 x 3001, 20 symbols: 391 us a call unsplit, 246
+            // split): only on the kernels of G = 32 (the planner's own
+            // choice).  Pairs of 5 to 8 symbols change over to them for the
+            // four parts with the maximum; without it they stay in one part on
+            // the 4-bit row tables, which have no running maximum to carry.
+            // Pairs of more than 8 symbols keep the maximum whether asked to
+            // or not.
+            if (!(mode & WFK_MODE_PERM4) && (v->chunk != 32 || (nomax && !(mode & WFK_MODE_CMP)))) continue;
+            cand[i] = nomax && !(mode & WFK_MODE_CMP) ? 2 : 3;  // extra pairs
             extra += cand[i] * si;
         }
         // Three or four parts while every strip has a CU of its own.  Beyond
@@ -743,6 +748,13 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
         // engines have instances without it).
         if (j.problem == WF_SW && !(mode & WFK_MODE_CMP) && ((j.flags | (tile ? tile->flags : 0)) & WF_TILE_NO_MAX))
             mode |= WFK_MODE_NOMAX;
+        // The parts of a split pair take the byte tables or compare codes:
+        // 5 to 8 symbols leave the 4-bit fields' bit offsets.
+        if (swsplit[i] && !(mode & (WFK_MODE_PERM4 | WFK_MODE_CMP))) {
+            shr2(ph->codes.data() + p.a_off, j.n1);
+            shr2(ph->codes.data() + p.b_off, j.n2);
+            mode = WFK_MODE_CMP | WFK_MODE_FREE_HEAD | (0x1FF << WFK_MODE_NEVER_SHIFT);
+        }
         p.mode = mode;
         // The bit-parallel kernel indexes a 32-row table with the codes.
         if (bitpar && (j.problem == WF_SW || (mode & WFK_MODE_CMP))) return WF_ERR_NOKERNEL;
@@ -755,12 +767,14 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
             const wf_job &j = jobs[sp.job];
             const WfPairDev &f = ph->pairs[sp.job];
             WfPairDev &rv = ph->pairs[sp.rev];
-            if (!(f.mode & WFK_MODE_PERM4) || !(f.mode & WFK_MODE_NOMAX) != (sp.crev >= 0)) return WF_ERR_INVALID;
+            if (!(f.mode & (WFK_MODE_PERM4 | WFK_MODE_CMP)) || !(f.mode & WFK_MODE_NOMAX) != (sp.crev >= 0))
+                return WF_ERR_INVALID;
             uint8_t *codes = ph->codes.data();
             reverse_codes(codes + f.a_off + (j.n1 - rv.n1), rv.n1, codes + rv.a_off);
+            // (Compared codes: the engine goes by WfCutDev::pad.)
             std::memset(codes + rv.b_off, WFK_NO_SYMBOL, (size_t)sp.pad);
             reverse_codes(codes + f.b_off, j.n2, codes + rv.b_off + sp.pad);
-            const int32_t mode = (f.mode & (WFK_MODE_PERM4 | WFK_MODE_FREE_HEAD)) | (two_part ? 0 : WFK_MODE_NOMAX);
+            const int32_t mode = (f.mode & ~WFK_MODE_NOMAX) | (two_part ? 0 : WFK_MODE_NOMAX);
             if (sp.f0 >= 0) ph->pairs[sp.f0].mode = f.mode;
             rv.mode = mode | WFK_MODE_SWE;
             if (sp.crev >= 0) ph->pairs[sp.crev].mode = mode;

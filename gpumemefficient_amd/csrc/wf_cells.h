@@ -126,6 +126,17 @@ struct Cell<WFK_SWP, CMP> {
     static constexpr uint32_t kNever = 0x0c0c0d0du;
 };
 
+// SW, more than 4 symbols, two rows per lane (WFK_MODE_CMP with WFK_SWP or
+// WFK_SWE): t[r] is the row's code (0x100 where it holds no symbol), the
+// column value the column's code, and a row's s + 2 (s + 4) is chosen by a
+// compare: two operations a row where the byte tables take half of one perm
+// and a byte select inside the add.  A row of WFK_SWE that holds no symbol
+// must add 0 where others add 1 on a mismatch, so that value is a register
+// (LaneState::miss).  A step is 12 operations with the maximum (byte tables
+// 10); what bounds a pair is the strip chain, so taking these pairs into the
+// column split is what pays: 7013 x 3001, 20 symbols, maximum kept: 391 -> 246
+// us a call (planning included), 1.5 to 1.9 times at 1000 to 10000 symbols.
+
 // The reverse half of a column-split SW pair (WFK_MODE_SWE): the same byte
 // tables and selectors with s + 4 (7 on a match, 1 else) and no clamp,
 // E = max3(up, left, diag + s + 4).  A never-matching column reads -1, so
@@ -162,6 +173,7 @@ struct LaneState {
     int dg;          // H(row above row 0, last column) -- the next step's "diag"
     int best;        // SW running maximum (WFK_SWE: see step)
     uint32_t t[R];   // per-row table / code
+    int miss[R];     // WFK_SWE, compared codes: s + 4 of a column symbol that is not the row's
 };
 
 template <int P, bool CMP, int R, bool MASKED, bool TRACK>
@@ -171,7 +183,7 @@ __device__ __forceinline__ void step(LaneState<R> &st, int inj, uint32_t ca, boo
     int up = up0;
     int diag = st.dg;
     uint32_t pp = 0;
-    if (P == WFK_SWP || P == WFK_SWE) pp = __builtin_amdgcn_perm(st.t[1], st.t[0], ca);
+    if ((P == WFK_SWP || P == WFK_SWE) && !CMP) pp = __builtin_amdgcn_perm(st.t[1], st.t[0], ca);
     // WFK_SWE: the largest F = E - 2 (i + j) of the lane.  The offset falls by 2
     // a step and from row 0 to row 1, so E of row 0 and row 1's E of the step
     // before have the same one, and st.best, kept relative to row 0's current
@@ -185,8 +197,14 @@ __device__ __forceinline__ void step(LaneState<R> &st, int inj, uint32_t ca, boo
         const int left = st.h[r];
         int h;
         if constexpr (P == WFK_SWP || P == WFK_SWE) {
-            static_assert(R == 2, "the byte tables hold two rows per lane");
-            const int s2 = (int)(int8_t)(uint8_t)(pp >> (8 * r));
+            static_assert(R == 2, "two rows per lane");
+            int s2;
+            if constexpr (!CMP)
+                s2 = (int)(int8_t)(uint8_t)(pp >> (8 * r));
+            else if constexpr (P == WFK_SWE)
+                s2 = ca == st.t[r] ? 7 : st.miss[r];
+            else
+                s2 = ca == st.t[r] ? 5 : -1;
             const int m = max(max(up, left), diag + s2);
             h = (P == WFK_SWE) ? m : (int)__builtin_elementwise_sub_sat((uint32_t)m, 2u);
         } else {

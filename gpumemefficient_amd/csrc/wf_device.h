@@ -6,8 +6,8 @@
 
 // Problem ids match include/wfdp.h (WF_LCS, WF_ED, WF_SW).
 enum { WFK_LCS = 0, WFK_ED = 1, WFK_SW = 2 };
-// Kernel-internal problem ids (never stored in a pair): SW in
-// WFK_MODE_PERM4, and the reverse half of a column-split SW pair
+// Kernel-internal problem ids (never stored in a pair): SW with two rows per
+// lane in WFK_MODE_PERM4 or WFK_MODE_CMP (column split), and the reverse half of a column-split SW pair
 // (WFK_MODE_SWE).
 enum { WFK_SWP = 3, WFK_SWE = 4 };
 
@@ -26,14 +26,16 @@ enum {
     WFK_MODE_PERM4 = 16,
     // SW without the running maximum (only the bottom-right cell).
     WFK_MODE_NOMAX = 32,
-    // The reverse half of a column-split SW pair (with WFK_MODE_PERM4): the
+    // The reverse half of a column-split SW pair (with WFK_MODE_PERM4 or
+    // WFK_MODE_CMP): the
     // unclamped best path weight into each cell of the reversed sequences,
     // kept as E = F + 2 (x + y), so E = max3(up, left, diag + s + 4) with
     // zero boundaries.  Its maximum (without WFK_MODE_NOMAX) is the largest F.
     WFK_MODE_SWE = 64,
 };
 enum { WFK_MODE_NEVER_SHIFT = 8 };
-// Byte tables: code of a row above the first symbol's (WfSplitDev::pad).
+// Byte tables: code of a row above the first symbol's (WfSplitDev::pad);
+// compared codes may be any byte, there the row number tells.
 enum { WFK_NO_SYMBOL = 5 };
 
 // One sequence pair as the kernels see it.  x runs over a (n1 columns),
@@ -78,7 +80,7 @@ struct WfCutDev {
 // the score is min (ED) / max (LCS) over y of F(y) + R(y) (Hirschberg's
 // split, J. ACM 1975; CACM 18(6) 1975 for LCS).
 //
-// An SW pair (prob WFK_SW, cell engine with byte tables) is cut along a
+// An SW pair (prob WFK_SW, asynchronous engine, byte tables or compared codes) is cut along a
 // staircase, strip g at column c(g), into the left part `job`, the right part
 // from a zero boundary `f0`, the right part reversed `rev` (WFK_MODE_SWE) and,
 // for a pair that keeps the running maximum, the right part reversed with the

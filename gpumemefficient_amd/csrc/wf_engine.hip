@@ -51,8 +51,8 @@ __device__ TraceRec g_trace[kTraceTasks * kTraceWaves];
 // granularity G): one loop back-edge per kU steps, the counter checks in
 // between are not-taken branches.  kB: steps per block of LDS operands.
 constexpr int kU = 32;
-// The SW byte-table strips of the four-wave, G = 32 kernels (the single-pair
-// SW path) run 256 steps per iteration instead: one lap of the 256-slot
+// The SW strips (byte tables and compared codes) of the four-wave, G = 32
+// kernels (the single-pair SW path) run 256 steps per iteration instead: one lap of the 256-slot
 // rings, so every ring address of an iteration is a constant offset and the
 // per-iteration scalar address arithmetic is amortised over 8 times the
 // steps (SW 131072^2 7.07 -> 6.75 ms).  Other strips keep kU, which keeps
@@ -372,10 +372,20 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
         const uint8_t *bcodes = ka.codes + pd.b_off;
         LaneState<R> st;
         if constexpr (P == WFK_SWP || P == WFK_SWE) {
-            const uint32_t c0 = row0 < n2 ? (uint32_t)bcodes[row0] : 4u;
-            const uint32_t c1 = row0 + 1 < n2 ? (uint32_t)bcodes[row0 + 1] : 4u;
-            st.t[0] = Cell<P, CMP>::tables(c0, c1, 0);
-            st.t[1] = Cell<P, CMP>::tables(c0, c1, 1);
+            if constexpr (CMP) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int64_t y = row0 + r;
+                    const bool v = y >= sg.pad && y < n2;
+                    st.t[r] = v ? (uint32_t)bcodes[y] : 0x100u;
+                    st.miss[r] = v ? 1 : 0;
+                }
+            } else {
+                const uint32_t c0 = row0 < n2 ? (uint32_t)bcodes[row0] : 4u;
+                const uint32_t c1 = row0 + 1 < n2 ? (uint32_t)bcodes[row0 + 1] : 4u;
+                st.t[0] = Cell<P, CMP>::tables(c0, c1, 0);
+                st.t[1] = Cell<P, CMP>::tables(c0, c1, 1);
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r) st.h[r] = 0;
         } else {
@@ -657,8 +667,8 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
     // counter store, so every compute wave reads them after they are set.
     {
         const uint32_t never =
-            (P == WFK_SWP || P == WFK_SWE) ? Cell<WFK_SWP, false>::kNever
-                                           : ((uint32_t)pd.mode >> WFK_MODE_NEVER_SHIFT) & 0x1FFu;
+            ((P == WFK_SWP || P == WFK_SWE) && !CMP) ? Cell<WFK_SWP, false>::kNever
+                                                     : ((uint32_t)pd.mode >> WFK_MODE_NEVER_SHIFT) & 0x1FFu;
         sh.aw[lane] = never;
         if (lane < kUMax + kB) sh.aw[AW + lane] = never;
     }
@@ -690,7 +700,7 @@ __device__ __forceinline__ void async_strip(const WfKernelArgs &ka, const WfPair
         const int x = in_next + lane;
         const bool in = x < n1;
         p.c = in ? (uint32_t)acodes[x] : 0u;
-        if (P == WFK_SWP || P == WFK_SWE) p.c = Cell<WFK_SWP, false>::selector(p.c & 3u);
+        if ((P == WFK_SWP || P == WFK_SWE) && !CMP) p.c = Cell<WFK_SWP, false>::selector(p.c & 3u);
         p.t = (has_prev && in && x >= xp)
                   ? (lane < p.width ? __hip_atomic_load(bprev + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0)
                   : tag;
@@ -864,7 +874,27 @@ __global__ __launch_bounds__(64 * (W + 2)) void wf_engine_async(WfKernelArgs ka)
                 async_strip<WFK_SW, false, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
             break;
         }
-        default: async_strip<WFK_SW, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t); break;
+        default:
+            // (The parts of a split pair and WFK_MODE_NOMAX: G = 32 only, the
+            // planner's own choice, for the build's time.)
+            if constexpr (R == 2 && G == 32) {
+                const bool nomax = (pd.mode & WFK_MODE_NOMAX) != 0;
+                if (pd.mode & WFK_MODE_SWE) {
+                    if (nomax)
+                        async_strip<WFK_SWE, true, R, W, G, AW, RS, true>(ka, pd, sg, td.pair, td.group, sh, lane, wave,
+                                                                         epoch, t);
+                    else
+                        async_strip<WFK_SWE, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
+                } else if (nomax) {
+                    async_strip<WFK_SWP, true, R, W, G, AW, RS, true>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch,
+                                                                      t);
+                } else {
+                    async_strip<WFK_SWP, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
+                }
+            } else {
+                async_strip<WFK_SW, true, R, W, G, AW, RS>(ka, pd, sg, td.pair, td.group, sh, lane, wave, epoch, t);
+            }
+            break;
         }
         __syncthreads();
     }
