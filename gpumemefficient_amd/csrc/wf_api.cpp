@@ -904,28 +904,28 @@ int wf_copy_plan(WfPlanHost *ph, WfArenas *ar, hipStream_t stream)
 }
 
 // Sizes every device buffer of the plan (growing them as needed).
-static int ensure_arenas(WfPlanHost *ph, WfArenas *ar)
+static int ensure_arenas(WfPlanHost *ph, WfArenas *ar, hipStream_t stream)
 {
     WfPlanBytes nb;
     wf_plan_bytes(ph, &nb);
     int st;
-    if ((st = ar->codes.ensure(nb.codes)) != WF_OK) return st;
-    if ((st = ar->pairs.ensure(nb.pairs)) != WF_OK) return st;
-    if ((st = ar->tasks.ensure(nb.tasks)) != WF_OK) return st;
-    if ((st = ar->bnd.ensure(nb.bnd, true)) != WF_OK) return st;
-    if ((st = ar->res.ensure(nb.res)) != WF_OK) return st;
-    if ((st = ar->counters.ensure(nb.counters)) != WF_OK) return st;
+    if ((st = ar->codes.ensure(nb.codes, false, stream, ar->retired)) != WF_OK) return st;
+    if ((st = ar->pairs.ensure(nb.pairs, false, stream, ar->retired)) != WF_OK) return st;
+    if ((st = ar->tasks.ensure(nb.tasks, false, stream, ar->retired)) != WF_OK) return st;
+    if ((st = ar->bnd.ensure(nb.bnd, true, stream, ar->retired)) != WF_OK) return st;
+    if ((st = ar->res.ensure(nb.res, false, stream, ar->retired)) != WF_OK) return st;
+    if ((st = ar->counters.ensure(nb.counters, false, stream, ar->retired)) != WF_OK) return st;
     // Launch epoch: zero on allocation, so it never matches a zeroed boundary word.
-    if ((st = ar->epoch.ensure(nb.epoch, true)) != WF_OK) return st;
-    if ((st = ar->colw.ensure(nb.colw)) != WF_OK) return st;
-    return ar->splits.ensure(nb.splits);
+    if ((st = ar->epoch.ensure(nb.epoch, true, stream, ar->retired)) != WF_OK) return st;
+    if ((st = ar->colw.ensure(nb.colw, false, stream, ar->retired)) != WF_OK) return st;
+    return ar->splits.ensure(nb.splits, false, stream, ar->retired);
 }
 
 int wf_upload_plan_async(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, hipStream_t stream, bool sync)
 {
     (void)ctx;
     int st;
-    if ((st = ensure_arenas(ph, ar)) != WF_OK) return st;
+    if ((st = ensure_arenas(ph, ar, stream)) != WF_OK) return st;
     if ((st = wf_copy_plan(ph, ar, stream)) != WF_OK) return st;
     if (sync && hipStreamSynchronize(stream) != hipSuccess) return WF_ERR_DEVICE;
     return WF_OK;

@@ -18,22 +18,36 @@ struct DevBuf {
     void *ptr = nullptr;
     size_t cap = 0;
     // zero_fill: clear new memory (boundary rows must not hold a stale tag).
-    int ensure(size_t bytes, bool zero_fill = false)
+    // stream: clears the memory in this stream's order, not the null stream's.
+    // retired: takes the memory outgrown, to be freed once the device is idle
+    // (hipFree waits for every launch that runs).
+    int ensure(size_t bytes, bool zero_fill = false, hipStream_t stream = nullptr,
+               std::vector<void *> *retired = nullptr)
     {
         if (bytes <= cap) return WF_OK;
         if (ptr) {
-            (void)hipFree(ptr);
+            if (retired)
+                retired->push_back(ptr);
+            else
+                (void)hipFree(ptr);
             ptr = nullptr;
             cap = 0;
         }
         size_t want = std::max<size_t>(bytes, 256);
         want = (want + 255) & ~size_t(255);
-        if (hipMalloc(&ptr, want) != hipSuccess) {
+        bool got = hipMalloc(&ptr, want) == hipSuccess;
+        if (!got && retired && !retired->empty()) {
+            for (void *p : *retired) (void)hipFree(p);
+            retired->clear();
+            got = hipMalloc(&ptr, want) == hipSuccess;
+        }
+        if (!got) {
             (void)hipGetLastError();
             ptr = nullptr;
             return WF_ERR_NOMEM;
         }
-        if (zero_fill && hipMemset(ptr, 0, want) != hipSuccess) {
+        if (zero_fill &&
+            (stream ? hipMemsetAsync(ptr, 0, want, stream) : hipMemset(ptr, 0, want)) != hipSuccess) {
             (void)hipFree(ptr);
             ptr = nullptr;
             return WF_ERR_DEVICE;
@@ -51,6 +65,7 @@ struct DevBuf {
 
 struct WfArenas {
     DevBuf codes, pairs, tasks, bnd, res, counters, epoch, splits, colw;
+    std::vector<void *> *retired = nullptr;  // DevBuf::ensure; null: outgrown memory is freed at once
     void release()
     {
         splits.release();

@@ -155,6 +155,7 @@ struct wf_server {
     wf_ctx *ctx = nullptr;
     wf_server_opts opts{};
     std::vector<Slot> slots;
+    std::vector<void *> retired;           // arenas the slots have outgrown, freed while no slot runs
     std::thread sched;
     std::mutex mu;
     std::condition_variable cv;
@@ -258,6 +259,7 @@ static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
     // fit in the launch's workgroups, or the launch would go to the lock-step
     // engine below).
     sl.ph = WfPlanHost();
+    sl.ar.retired = &s->retired;
     int st = wf_build_plan(s->ctx, jobs.data(), (int64_t)jobs.size(), nullptr, &sl.ph);
     if (st != WF_OK) return st;
     if (sl.ph.variant->engine == WF_ENGINE_ASYNC && !sl.ph.splits.empty() &&
@@ -282,9 +284,12 @@ static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
     if (n > sl.pinned_cap) {
         if (sl.pinned) (void)hipHostFree(sl.pinned);
         sl.pinned = nullptr;
-        if (hipHostMalloc((void **)&sl.pinned, n * sizeof(WfResultDev), hipHostMallocDefault) != hipSuccess)
+        // (Growing it waits for every launch, so it starts with room for most.)
+        sl.pinned_cap = 0;
+        const int64_t cap = std::max<int64_t>(n, 1024);
+        if (hipHostMalloc((void **)&sl.pinned, cap * sizeof(WfResultDev), hipHostMallocDefault) != hipSuccess)
             return WF_ERR_NOMEM;
-        sl.pinned_cap = n;
+        sl.pinned_cap = cap;
     }
     if (hipMemcpyAsync(sl.pinned, sl.ar.res.ptr, n * sizeof(WfResultDev), hipMemcpyDeviceToHost, sl.stream) !=
         hipSuccess)
@@ -312,6 +317,10 @@ static void scheduler(wf_server *s)
                 std::lock_guard<std::mutex> lk(s->mu);
                 s->error = WF_ERR_DEVICE;
             }
+        }
+        if (!s->retired.empty() && std::none_of(s->slots.begin(), s->slots.end(), [](const Slot &x) { return x.busy; })) {
+            for (void *p : s->retired) (void)hipFree(p);
+            s->retired.clear();
         }
         // 2. admission by HBM budget, in arrival order
         {
@@ -746,7 +755,8 @@ int wf_server_create(int device, const wf_server_opts *opts, wf_server **out)
     }
     s->slots.resize(s->opts.streams);
     for (Slot &sl : s->slots) {
-        if (hipStreamCreate(&sl.stream) != hipSuccess || hipEventCreateWithFlags(&sl.done, hipEventDisableTiming) !=
+        // (Not ordered with the null stream, on which other code may wait.)
+        if (hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&sl.done, hipEventDisableTiming) !=
                                                              hipSuccess) {
             wf_server_destroy(s);
             return WF_ERR_DEVICE;
@@ -831,6 +841,7 @@ void wf_server_destroy(wf_server *s)
         if (sl.done) (void)hipEventDestroy(sl.done);
         if (sl.stream) (void)hipStreamDestroy(sl.stream);
     }
+    for (void *p : s->retired) (void)hipFree(p);
     if (s->ctx) wf_ctx_destroy(s->ctx);
     delete s;
 }
