@@ -55,6 +55,7 @@ struct Request {
     std::vector<int32_t> a, b;
     int64_t bytes;      // device footprint charged to the HBM budget
     bool bitpar;        // can run on the bit-parallel engine (LCS/ED, <= 32 symbols)
+    bool is_long = false;  // see is_long()
     double t_submit;
     double t_start = 0; // launch time
 };
@@ -65,6 +66,7 @@ struct Slot {
     WfArenas ar;
     WfPlanHost ph;
     std::vector<Request> reqs;
+    bool alone = false;  // runs one long request (is_long)
     WfResultDev *pinned = nullptr;
     int64_t pinned_cap = 0;
     bool busy = false;
@@ -209,6 +211,24 @@ static bool alphabet_fits(const wf_job *job)
     return distinct <= 256;
 }
 
+// A request whose strip chain would set the time of any launch it shares: it
+// gets a launch of its own on the whole chip, where a pair is column split and
+// runs on the asynchronous (LCS, ED: staged bit-parallel) engine, while the
+// other slots run the rest.  The lines lie where the chain costs about 2.5 ms
+// in a shared launch (lock-step SW 35 ns for each of n1 + 1.5 n2 steps, plain
+// bit-parallel 45 ns a column).
+static bool is_long(const Request &r)
+{
+    const int64_t n1 = (int64_t)r.a.size(), n2 = (int64_t)r.b.size();
+    if (n2 == 0 || n2 > 512 * 256) return false;  // more strips than the asynchronous engine is chosen for
+    return r.bitpar ? n1 >= 49152 : r.problem == WF_SW && n1 + n2 + n2 / 2 >= 65536;
+}
+// Long requests, waiting or running, up to which each runs alone; with more of
+// them a shared launch fills the chip, which costs less than their launches
+// one after another (SW 65536^2: 2.0 ms alone, 1.0 each in a full launch, 5.7
+// for one in a shared launch; ED 65536^2: 1.3 ms alone, 3.2 in a shared one).
+constexpr int kFewLongSw = 3, kFewLongBitpar = 6;
+
 static void finish_slot(wf_server *s, Slot &sl)
 {
     std::vector<wf_completion> out;
@@ -240,6 +260,7 @@ static void finish_slot(wf_server *s, Slot &sl)
     s->done.insert(s->done.end(), out.begin(), out.end());
     sl.reqs.clear();
     sl.busy = false;
+    sl.alone = false;
     s->cv.notify_all();
 }
 
@@ -251,7 +272,9 @@ static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
         const Request &r = sl.reqs[i];
         jobs[i] = wf_job{r.problem, r.flags, r.a.data(), (int64_t)r.a.size(), r.b.data(), (int64_t)r.b.size()};
     }
-    const int nslots = (int)s->slots.size();
+    // A long request's launch may take the whole chip: no strip waits on one
+    // that no running workgroup holds, so launches that overlap only share it.
+    const int nslots = sl.alone ? 1 : (int)s->slots.size();
     auto share = [&](const WfVariant *v) {
         return std::max(1, wf_max_resident_groups(s->ctx, v) / std::max(1, nslots));
     };
@@ -358,10 +381,35 @@ static void scheduler(wf_server *s)
                 // admitted requests of its class (bit-parallel LCS/ED, or the
                 // rest), in arrival order; the other class waits for the
                 // next free slot.
-                if (!s->admitted.empty()) {
-                    const bool cls = s->admitted.front().bitpar;
-                    for (auto it = s->admitted.begin(); it != s->admitted.end() && (int)batch.size() < maxb;) {
-                        if (it->bitpar == cls) {
+                // A long request, while there are few, goes alone; one slot is
+                // left to the others.
+                int nlong[2] = {0, 0}, alone = 0;
+                for (const Slot &x : s->slots)
+                    if (x.busy && x.alone) {
+                        ++alone;
+                        ++nlong[x.reqs[0].bitpar];
+                    }
+                for (const Request &r : s->admitted) nlong[r.bitpar] += r.is_long;
+                auto apart = [&](const Request &r) {
+                    return r.is_long && !s->opts.per_request && s->slots.size() > 1 &&
+                           nlong[r.bitpar] <= (r.bitpar ? kFewLongBitpar : kFewLongSw);
+                };
+                auto first = s->admitted.begin();
+                while (first != s->admitted.end() && apart(*first) && alone + 1 >= (int)s->slots.size()) ++first;
+                sl.alone = false;
+                if (first != s->admitted.end() && apart(*first)) {
+                    // A split needs up to twice the boundary rows.
+                    sl.alone = s->used + first->bytes <= s->budget;
+                    if (sl.alone) {
+                        s->used += first->bytes;
+                        first->bytes *= 2;
+                    }
+                    batch.push_back(std::move(*first));
+                    s->admitted.erase(first);
+                } else if (first != s->admitted.end()) {
+                    const bool cls = first->bitpar;
+                    for (auto it = first; it != s->admitted.end() && (int)batch.size() < maxb;) {
+                        if (it->bitpar == cls && !apart(*it)) {
                             batch.push_back(std::move(*it));
                             it = s->admitted.erase(it);
                         } else {
@@ -392,6 +440,7 @@ static void scheduler(wf_server *s)
                 }
                 sl.reqs.clear();
                 sl.busy = false;
+                sl.alone = false;
             }
             did = true;
         }
@@ -781,6 +830,7 @@ int wf_server_submit(wf_server *s, const wf_job *job, uint64_t *ticket)
     r.b.assign(job->b, job->b + job->n2);
     r.bytes = request_bytes(job->n1, job->n2, 512);
     r.bitpar = wf_bitpar_eligible(job, 1);
+    r.is_long = is_long(r);
     std::lock_guard<std::mutex> lk(s->mu);
     if ((int64_t)s->pending.size() >= s->opts.queue_capacity) return WF_ERR_AGAIN;
     r.ticket = s->next_ticket++;
