@@ -486,6 +486,21 @@ static std::vector<int32_t> sw_cuts(int64_t n1, int64_t n2, int64_t strip, int w
     return c;
 }
 
+// The same for LCS and ED on the staged bit-parallel engine (2048-row strips),
+// with a smaller lag where the pair is too narrow for it, so that every strip
+// keeps columns on both sides.  Lags of 0 / 160 / 176 / 192 / 208 / 256 steps:
+// ED 65536^2 1.274 / 1.198 / 1.192 / 1.194 / 1.201 / 1.219 ms, LCS 32768^2 0.360 /
+// 0.342 / 0.340 / 0.338 / 0.337 / 0.341, ED 20000 x 60000 0.547 / 0.455 / 0.448 /
+// 0.449 / 0.456 / 0.474.
+static std::vector<int32_t> bitpar_cuts(int64_t n1, int64_t n2, int64_t strip)
+{
+    const int64_t G = (n2 + strip - 1) / strip;
+    const int64_t lag = G > 1 ? std::min<int64_t>(192, (n1 - 64) / (G - 1)) : 0;
+    std::vector<int32_t> c((size_t)G);
+    for (int64_t g = 0; g < G; ++g) c[g] = (int32_t)((n1 + (G - 1) * lag) / 2 - g * lag);
+    return c;
+}
+
 int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile,
                   WfPlanHost *ph, int64_t max_groups)
 {
@@ -600,6 +615,12 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     // Codes: a then b per pair, 16-byte aligned; a split pair's reverse half
     // gets its own reversed copies after all jobs.
     int64_t code_bytes = 0, bnd_ints = 0;
+    // Bit-parallel halves that meet along a staircase: pairs of several strips
+    // (one strip has no lag to share out, and its call of 1531 x 1187 took 73 us
+    // with the cut's descriptors against 70 without).
+    auto stairs = [&](int64_t i) {
+        return mid[i] && v->engine == WF_ENGINE_BITPAR_STAGED && v->waves == 1 && jobs[i].n2 > strip;
+    };
     auto place_codes = [&](WfPairDev &p, int prob, int64_t n1, int64_t n2, int64_t a_bytes) {
         p.prob = prob;
         p.n1 = (int32_t)n1;
@@ -632,7 +653,7 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
             p.ngroups = 0;
             continue;
         }
-        if (swsplit[i])
+        if (swsplit[i] || stairs(i))
             place_codes(p, j.problem, j.n1, j.n2, j.n1);
         else
             place(p, j.problem, mid[i] ? mid[i] : j.n1, j.n2, j.n1);
@@ -714,12 +735,40 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
                 r += swsplit[i] - (two_part ? 1 : 0);
                 continue;
             }
-            place(ph->pairs[r], j.problem, j.n1 - mid[i], j.n2, j.n1 - mid[i]);
             WfSplitDev sp{};
             sp.job = (int32_t)i;
             sp.rev = (int32_t)r;
             sp.prob = j.problem;
             sp.n2 = (int32_t)j.n2;
+            if (stairs(i)) {
+                // (f0 and r0, the ends of the staircase, below.)
+                const std::vector<int32_t> c = bitpar_cuts(j.n1, j.n2, strip);
+                const int64_t G = (int64_t)c.size(), pad = G * strip - j.n2;
+                const int32_t n1 = (int32_t)j.n1;
+                WfPairDev &f = ph->pairs[i], &rv = ph->pairs[r];
+                f.n1 = c[0];
+                mid[i] = c.back();
+                place_codes(rv, j.problem, n1 - c.back(), G * strip, n1 - c.back());
+                auto cut_pair = [&](WfPairDev &p, auto &&of) {
+                    p.cut = (int32_t)ph->cuts.size();
+                    for (int64_t g = 0; g < G; ++g) {
+                        WfCutDev cd = of(g);
+                        cd.bnd = bnd_ints;
+                        if (g + 1 < G) bnd_ints += 4 * ((cd.n + 126) / 64);  // bs_row_words in wf_bitpar.hip
+                        ph->cuts.push_back(cd);
+                    }
+                    return p.cut;
+                };
+                sp.cut = cut_pair(f, [&](int64_t g) { return WfCutDev{0, 0, c[g], 0, 0, 0, 0}; });
+                sp.rcut = cut_pair(rv, [&](int64_t k) {
+                    return WfCutDev{0, 0, n1 - c[G - 1 - k], 0, 0, (int32_t)pad, 0};
+                });
+                sp.strip = (int32_t)strip;
+                sp.pad = (int32_t)pad;
+                sp.cols = n1;
+            } else {
+                place(ph->pairs[r], j.problem, j.n1 - mid[i], j.n2, j.n1 - mid[i]);
+            }
             ph->pairs[i].col_off = ph->colw_entries;
             sp.fwd_off = ph->colw_entries;
             ph->colw_entries += (int64_t)ph->pairs[i].ngroups * v->waves * 64;
@@ -791,10 +840,12 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
         uint8_t *ra = ph->codes.data() + r.a_off;
         uint8_t *rb = ph->codes.data() + r.b_off;
         reverse_codes(fa + m, nr, ra);
-        reverse_codes(fb, j.n2, rb);
+        std::memset(rb, 0, (size_t)sp.pad);  // rows without a symbol: the engine goes by WfCutDev::pad
+        reverse_codes(fb, j.n2, rb + sp.pad);
         r.mode = (f.mode & ~WFK_MODE_TEXTBOOK) | (j.problem == WF_ED ? WFK_MODE_TEXTBOOK : 0);
         if (j.problem == WF_ED) {
-            sp.f0 = (int32_t)((f.mode & WFK_MODE_TEXTBOOK) ? m : m - 1);  // row 0 at column mid
+            // Row 0 at column mid (the staircase's first column).
+            sp.f0 = (f.mode & WFK_MODE_TEXTBOOK) ? f.n1 : f.n1 - 1;
             sp.r0 = (int32_t)nr;
         }
     }
@@ -1092,7 +1143,7 @@ int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int max
     const int lim = maxg > 0 ? maxg : wf_max_resident_groups(ctx, v);
     const int st = enqueue_engine(ph, v, lim, mode, ka, ar, stream);
     if (st != WF_OK) return st;
-    if (!ph->cuts.empty()) {
+    if (!ph->cuts.empty() && v->engine == WF_ENGINE_ASYNC) {
         // About 8192 nodes of the cut a workgroup.
         int64_t nodes = 0;
         for (const WfSplitDev &sp : ph->splits) nodes = std::max<int64_t>(nodes, (int64_t)sp.r0 + sp.n2);
@@ -1105,7 +1156,8 @@ int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int max
     }
     if (!ph->splits.empty() &&
         wf_launch_bitpar_combine((const WfSplitDev *)ar->splits.ptr, (int)ph->splits.size(),
-                                 (const uint32_t *)ar->colw.ptr, (WfResultDev *)ar->res.ptr, stream) != hipSuccess)
+                                 (const uint32_t *)ar->colw.ptr, ka.cuts, (const uint64_t *)ar->bnd.ptr,
+                                 (WfResultDev *)ar->res.ptr, stream) != hipSuccess)
         return WF_ERR_DEVICE;
     return WF_OK;
 }

@@ -443,7 +443,7 @@ __global__ __launch_bounds__(64 * W) void wf_engine_bitpar(WfKernelArgs ka)
 // hands down, and the LDS reads.  Per step, W = 1: ED 38.4 -> 31.2 ns, LCS 25.5 ->
 // 16.7 (before: every step's words stored to LDS, ED with two more operations,
 // LCS with one, and the reads at their use); ED 65536^2 1.51 -> 1.25 ms, LCS
-// 32768^2 0.547 -> 0.353.  W = 2 overloads the one staging wave.
+// 32768^2 0.547 -> 0.353 (and 1.19 and 0.338 along a staircase).  W = 2 overloads the one staging wave.
 // ---------------------------------------------------------------------------
 
 template <int W>
@@ -567,7 +567,11 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
     constexpr bool ED = P == WFK_ED;
     constexpr int NP = ED ? 2 : 1;  // bit planes of the handed-down words
     const bool stager = wave == W;
-    const int n1 = pd.n1, n2 = pd.n2;
+    // The strips of a split pair end at columns of their own, and the rows of a
+    // reversed part start with some that hold no symbol (WfSplitDev::pad).
+    const bool cut = pd.cut >= 0;
+    const int n1 = cut ? ka.cuts[pd.cut + g].n : pd.n1, n2 = pd.n2;
+    const int pad = cut ? ka.cuts[pd.cut + g].pad : 0;
     const int64_t row0 = (int64_t)g * (W * kRowsPerWave) + wave * kRowsPerWave + lane * 32;
     const uint8_t *acodes = ka.codes + pd.a_off;
     const uint8_t *bcodes = ka.codes + pd.b_off;
@@ -581,7 +585,7 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
     if (active) {
         int *peq = sh.peq[wave];
         for (int i = lane; i < 32 * 64; i += 64) peq[i] = 0;
-        for (int r = 0; r < nvalid; ++r) {
+        for (int r = (int)max<int64_t>(0, min<int64_t>(32, pad - row0)); r < nvalid; ++r) {
             const uint32_t code = bcodes[row0 + r] & 31u;
             atomicOr(&peq[code * 64 + lane], (int)(1u << r));
         }
@@ -592,8 +596,9 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
     const int total = nch + (wa - 1) * kD;
     const bool has_prev = g > 0;
     const bool has_next = g + 1 < pd.ngroups;
-    const uint64_t *bprev = ka.bnd + pd.bnd_off + (g - 1) * bs_row_words(n1);
-    uint64_t *bnext = ka.bnd + pd.bnd_off + g * bs_row_words(n1);
+    const uint64_t *bprev =
+        ka.bnd + (cut ? ka.cuts[pd.cut + max(0, g - 1)].bnd : pd.bnd_off + (g - 1) * bs_row_words(n1));
+    uint64_t *bnext = ka.bnd + (cut ? ka.cuts[pd.cut + g].bnd : pd.bnd_off + g * bs_row_words(n1));
     const uint64_t tag = (uint64_t)epoch << 32;
 
     // Staging wave: column codes of chunk c (column c*K + lane per lane) into
@@ -694,6 +699,9 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
 
     BpState st;
     st.pv = 0xffffffffu;  // ED: column 0 rises by 1 per row; LCS: V = all ones
+    // Rows without a symbol hand the boundary above them down: no match, and
+    // for ED no vertical difference either (the boundary rises by 1 a column).
+    if (ED && row0 < pad) st.pv = pad - row0 >= 32 ? 0u : 0xffffffffu << (int)(pad - row0);
     st.mv = 0u;
     st.ph = 0;
     st.mh = 0;
@@ -761,15 +769,19 @@ __device__ void bs_group(const WfKernelArgs &ka, const WfPairDev &pd, int pair, 
 // ---------------------------------------------------------------------------
 // Split pairs: the score from the two halves' last-column words.
 //
-// Row r (0-based, r < n2) of the forward half's column mid changes by
-// d_r = Pv_r - Mv_r (ED) or z_r = 1 - V_r (LCS, the LCS grows by one where V
-// has a zero); F(y) = f0 + sum_{r<y} d_r.  The reverse half's last column
-// at reverse row n2 - y is R(y) = r0 + T' - sum_{r<y} d'_{n2-1-r}, T' the sum
-// of all its deltas.  So F(y) + R(y) = f0 + r0 + T' + sum_{r<y} e_r with
-// e_r = d_r - d'_{n2-1-r}, and the score is that constant plus the smallest
-// (ED) or largest (LCS) prefix sum of e, the empty prefix included.  One
-// workgroup per split; the reverse words are read bit-reversed so that both
-// halves line up row by row.
+// The parts meet along a staircase (staged engine; otherwise a straight column):
+// strip g of the forward half ends at column c_g, c falling with g by the lag of
+// a strip, so that both halves' strip chains end together.  From (0, c_0) the
+// staircase goes down strip 0, left along its bottom row to c_1, down strip 1 and
+// so on to (n2, c_{G-1}).  The score is the smallest (ED) or largest (LCS) sum
+// F + R over its nodes: an alignment leaves the forward half's region at one.
+// A step down row r changes F by d_r = Pv_r - Mv_r (ED) or 1 - V_r (LCS) of the
+// forward half's last column, and R by -d' of the reverse half's row for r (row
+// n2 - 1 - r, behind `pad` rows without a symbol); a step left over column x
+// changes F by minus the horizontal difference that the strip handed down
+// there, and R by the reverse half's.  At the start F = f0 and R = r0 + the sum
+// of all of R's differences.  32 steps a thread and turn, one workgroup a pair
+// (10 us for 65536 rows).  Against a straight column: see bitpar_cuts.
 // ---------------------------------------------------------------------------
 
 // Column-split SW pair.  The table is cut along a staircase: strip g of 512
@@ -863,13 +875,23 @@ __global__ __launch_bounds__(1024) void wf_sw_combine(const WfSplitDev *splits, 
     }
 }
 
+// 32 steps of a strip's bottom row from column x (0-based) on, plane `h`: bit 31
+// is column x.
+__device__ __forceinline__ uint32_t bs_row_bits(const uint64_t *row, int n, int np, int x, int h)
+{
+    const int s = x + 63, w = s >> 5, words = 2 * ((n + 126) / 64);
+    const uint32_t a = (uint32_t)row[w * np + h], b = w + 1 < words ? (uint32_t)row[(w + 1) * np + h] : 0u;
+    return (uint32_t)(((((uint64_t)a << 32) | b) << (s & 31)) >> 32);
+}
+
 __global__ __launch_bounds__(1024) void wf_bitpar_combine(const WfSplitDev *splits, const uint32_t *colw,
-                                                          WfResultDev *res)
+                                                          const WfCutDev *cuts, const uint64_t *bnd, WfResultDev *res)
 {
     const WfSplitDev sp = splits[blockIdx.x];
     const bool ed = sp.prob == WFK_ED;
     const int n2 = sp.n2;
     const int nw = (n2 + 31) >> 5;
+    const int nwr = (n2 + sp.pad + 31) >> 5;
     const uint32_t *fw = colw + 2 * sp.fwd_off;
     const uint32_t *rw = colw + 2 * sp.rev_off;
     // Bits of reverse rows [base, base + 32) (base > -32), bit k = row
@@ -878,31 +900,58 @@ __global__ __launch_bounds__(1024) void wf_bitpar_combine(const WfSplitDev *spli
         const int lo = base >= 0 ? (base >> 5) : -1;
         const int sh = base - 32 * lo;
         const uint32_t wl = lo >= 0 ? rw[2 * lo + h] : 0u;
-        const uint32_t wh = (lo + 1 < nw) ? rw[2 * (lo + 1) + h] : 0u;
+        const uint32_t wh = (lo + 1 < nwr) ? rw[2 * (lo + 1) + h] : 0u;
         return (uint32_t)((((uint64_t)wh << 32) | wl) >> sh);
     };
+    // The staircase in words: per strip its rows, then the row below it.
+    const int G = sp.strip > 0 ? (n2 + sp.strip - 1) / sp.strip : 1;
+    const int ws = sp.strip > 0 ? sp.strip >> 5 : nw;
+    const WfCutDev *fc = cuts + sp.cut, *rc = cuts + sp.rcut;
+    const int hs = G > 1 ? (fc[0].n - fc[1].n + 31) >> 5 : 0;  // c falls by the same everywhere
+    const int items = G * (ws + hs);
     const int tid = threadIdx.x;
-    const int per = (nw + 1023) >> 10;
-    const int w0 = min(nw, tid * per), w1 = min(nw, w0 + per);
+    const int per = (items + 1023) >> 10;
+    const int w0 = min(items, tid * per), w1 = min(items, w0 + per);
     int run = 0, best = 0, rtot = 0;
-    for (int w = w0; w < w1; ++w) {
-        const int nk = min(32, n2 - 32 * w);
-        const uint32_t m = nk >= 32 ? 0xffffffffu : ((1u << nk) - 1u);
-        const int base = n2 - 32 * w - 32;  // reverse rows of original rows 32w+31 .. 32w
+    for (int it = w0; it < w1; ++it) {
+        const int g = it / (ws + hs), t = it - g * (ws + hs);
+        // fa, fb: F rises, falls; ra, rb: R falls, rises (bit k: step k).
         uint32_t fa, fb, ra, rb;
-        if (ed) {
-            fa = fw[2 * w] & m;
-            fb = fw[2 * w + 1] & m;
-            ra = __builtin_bitreverse32(rev_bits(base, 0)) & m;
-            rb = __builtin_bitreverse32(rev_bits(base, 1)) & m;
-            rtot += __builtin_popcount(ra) - __builtin_popcount(rb);
+        int nk;
+        if (t < ws) {
+            const int w = g * ws + t;
+            nk = min(32, n2 - 32 * w);
+            if (nk <= 0) continue;
+            const uint32_t m = nk >= 32 ? 0xffffffffu : ((1u << nk) - 1u);
+            const int base = sp.pad + n2 - 32 * w - 32;  // reverse rows of original rows 32w+31 .. 32w
+            if (ed) {
+                fa = fw[2 * w] & m;
+                fb = fw[2 * w + 1] & m;
+                ra = __builtin_bitreverse32(rev_bits(base, 0)) & m;
+                rb = __builtin_bitreverse32(rev_bits(base, 1)) & m;
+            } else {
+                fa = ~fw[2 * w] & m;  // zeros of V: the LCS grows at that row
+                fb = 0u;
+                ra = __builtin_bitreverse32(~rev_bits(base, 0)) & m;
+                rb = 0u;
+            }
         } else {
-            fa = ~fw[2 * w] & m;  // zeros of V: the LCS grows at that row
-            fb = 0u;
-            ra = __builtin_bitreverse32(~rev_bits(base, 0)) & m;
-            rb = 0u;
-            rtot += __builtin_popcount(ra);
+            // Columns x .. x - nk + 1 (1-based), leftwards.
+            if (g + 1 >= G) continue;
+            const int x = fc[g].n - 32 * (t - ws);
+            nk = min(32, x - fc[g + 1].n);
+            if (nk <= 0) continue;
+            const uint32_t m = nk >= 32 ? 0xffffffffu : ((1u << nk) - 1u);
+            const uint64_t *f = bnd + fc[g].bnd, *r = bnd + rc[G - 2 - g].bnd;
+            const int nf = fc[g].n, nr = rc[G - 2 - g].n, np = ed ? 2 : 1, xr = sp.cols - x;
+            // F's columns x - nk .. x - 1 (0-based), the last of which is step 0;
+            // the reverse half's from cols - x on, the first of which is.
+            fb = bs_row_bits(f, nf, np, x - nk, 0) >> (32 - nk) & m;
+            rb = __builtin_bitreverse32(bs_row_bits(r, nr, np, xr, 0)) & m;
+            fa = ed ? bs_row_bits(f, nf, np, x - nk, 1) >> (32 - nk) & m : 0u;
+            ra = ed ? __builtin_bitreverse32(bs_row_bits(r, nr, np, xr, 1)) & m : 0u;
         }
+        rtot += __builtin_popcount(ra) - __builtin_popcount(rb);
         for (int k = 0; k < nk; ++k) {
             run += (int)((fa >> k) & 1u) - (int)((fb >> k) & 1u) - (int)((ra >> k) & 1u) + (int)((rb >> k) & 1u);
             best = ed ? min(best, run) : max(best, run);
@@ -975,10 +1024,11 @@ __global__ __launch_bounds__(64 * (W + 1)) void wf_engine_bitpar_staged(WfKernel
 }  // namespace wfb
 
 extern "C" hipError_t wf_launch_bitpar_combine(const WfSplitDev *splits, int nsplits, const uint32_t *colw,
-                                               WfResultDev *res, hipStream_t stream)
+                                               const WfCutDev *cuts, const uint64_t *bnd, WfResultDev *res,
+                                               hipStream_t stream)
 {
     if (nsplits <= 0) return hipSuccess;
-    hipLaunchKernelGGL(wfb::wf_bitpar_combine, dim3(nsplits), dim3(1024), 0, stream, splits, colw, res);
+    hipLaunchKernelGGL(wfb::wf_bitpar_combine, dim3(nsplits), dim3(1024), 0, stream, splits, colw, cuts, bnd, res);
     return hipGetLastError();
 }
 

@@ -79,6 +79,7 @@ struct WfCutDev {
 // half's column mid and R(y) the reverse half's last column at row n2 - y,
 // the score is min (ED) / max (LCS) over y of F(y) + R(y) (Hirschberg's
 // split, J. ACM 1975; CACM 18(6) 1975 for LCS).
+// On the staged engine the halves meet along a staircase (wf_bitpar_combine).
 //
 // An SW pair (prob WFK_SW, asynchronous engine, byte tables or compared codes) is cut along a
 // staircase, strip g at column c(g), into the left part `job`, the right part
@@ -99,10 +100,11 @@ struct WfSplitDev {
     int64_t fwd_off;   // colw entry offsets of the two halves
     int64_t rev_off;
     int32_t crev = -1; // SW with the running maximum: the clamped reverse pair; -1: none
-    int32_t strip = 0; // SW: rows of a strip
+    int32_t strip = 0; // rows of a strip (0: LCS, ED cut at one column)
     int64_t crev_off = 0;
-    int32_t cut = 0, rcut = 0, ccut = 0;  // SW: WfCutDev indices of job, rev and crev
-    int32_t pad = 0;   // SW: rows without a symbol above the reversed parts' rows (their strips end where job's begin)
+    int32_t cut = 0, rcut = 0, ccut = 0;  // WfCutDev indices of job, rev and crev
+    int32_t cols = 0;  // LCS, ED along a staircase: columns of the pair
+    int32_t pad = 0;   // rows without a symbol above the reversed parts' rows (their strips end where job's begin)
 };
 
 // One unit of persistent work: strip `group` of pair `pair`.  Tasks of a

@@ -37,7 +37,8 @@ extern "C" hipError_t wf_launch_naive(int method, int prob, int textbook, int *t
                                       const int32_t *b, int n1, int n2, int *smax, hipStream_t stream);
 // Combine the two halves of each split pair (WfSplitDev) into res[job].
 extern "C" hipError_t wf_launch_bitpar_combine(const WfSplitDev *splits, int nsplits, const uint32_t *colw,
-                                               WfResultDev *res, hipStream_t stream);
+                                               const WfCutDev *cuts, const uint64_t *bnd, WfResultDev *res,
+                                               hipStream_t stream);
 // The same for column-split SW pairs (`blocks` workgroups a pair), after the
 // reset kernel and the engine launches that filled colw and bnd.
 extern "C" hipError_t wf_launch_sw_combine(const WfSplitDev *splits, int nsplits, int blocks, const uint32_t *colw,
