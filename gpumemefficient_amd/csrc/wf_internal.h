@@ -13,21 +13,39 @@
 #include "wf_device.h"
 #include "wf_variants.h"
 
+// Device memory that buffers have outgrown, up to `limit` bytes, to be freed once
+// the device is idle (hipFree waits for every launch that runs).
+struct RetiredMem {
+    std::vector<void *> mem;
+    size_t bytes = 0, limit = 0;
+    void add(void *p, size_t n)
+    {
+        if (bytes + n > limit) release();
+        mem.push_back(p);
+        bytes += n;
+        if (bytes > limit) release();
+    }
+    void release()
+    {
+        for (void *p : mem) (void)hipFree(p);
+        mem.clear();
+        bytes = 0;
+    }
+};
+
 // Grow-only device buffer.
 struct DevBuf {
     void *ptr = nullptr;
     size_t cap = 0;
     // zero_fill: clear new memory (boundary rows must not hold a stale tag).
     // stream: clears the memory in this stream's order, not the null stream's.
-    // retired: takes the memory outgrown, to be freed once the device is idle
-    // (hipFree waits for every launch that runs).
-    int ensure(size_t bytes, bool zero_fill = false, hipStream_t stream = nullptr,
-               std::vector<void *> *retired = nullptr)
+    // retired: takes the memory outgrown.
+    int ensure(size_t bytes, bool zero_fill = false, hipStream_t stream = nullptr, RetiredMem *retired = nullptr)
     {
         if (bytes <= cap) return WF_OK;
         if (ptr) {
             if (retired)
-                retired->push_back(ptr);
+                retired->add(ptr, cap);
             else
                 (void)hipFree(ptr);
             ptr = nullptr;
@@ -36,9 +54,8 @@ struct DevBuf {
         size_t want = std::max<size_t>(bytes, 256);
         want = (want + 255) & ~size_t(255);
         bool got = hipMalloc(&ptr, want) == hipSuccess;
-        if (!got && retired && !retired->empty()) {
-            for (void *p : *retired) (void)hipFree(p);
-            retired->clear();
+        if (!got && retired && !retired->mem.empty()) {
+            retired->release();
             got = hipMalloc(&ptr, want) == hipSuccess;
         }
         if (!got) {
@@ -65,7 +82,7 @@ struct DevBuf {
 
 struct WfArenas {
     DevBuf codes, pairs, tasks, bnd, res, counters, epoch, splits, colw;
-    std::vector<void *> *retired = nullptr;  // DevBuf::ensure; null: outgrown memory is freed at once
+    RetiredMem *retired = nullptr;  // DevBuf::ensure; null: outgrown memory is freed at once
     void release()
     {
         splits.release();

@@ -157,7 +157,7 @@ struct wf_server {
     wf_ctx *ctx = nullptr;
     wf_server_opts opts{};
     std::vector<Slot> slots;
-    std::vector<void *> retired;           // arenas the slots have outgrown, freed while no slot runs
+    RetiredMem retired;                    // arenas the slots have outgrown, freed while no slot runs
     std::thread sched;
     std::mutex mu;
     std::condition_variable cv;
@@ -341,10 +341,9 @@ static void scheduler(wf_server *s)
                 s->error = WF_ERR_DEVICE;
             }
         }
-        if (!s->retired.empty() && std::none_of(s->slots.begin(), s->slots.end(), [](const Slot &x) { return x.busy; })) {
-            for (void *p : s->retired) (void)hipFree(p);
-            s->retired.clear();
-        }
+        if (!s->retired.mem.empty() &&
+            std::none_of(s->slots.begin(), s->slots.end(), [](const Slot &x) { return x.busy; }))
+            s->retired.release();
         // 2. admission by HBM budget, in arrival order
         {
             std::lock_guard<std::mutex> lk(s->mu);
@@ -792,6 +791,7 @@ int wf_server_create(int device, const wf_server_opts *opts, wf_server **out)
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
     s->budget = s->opts.hbm_budget > 0 ? s->opts.hbm_budget : (int64_t)(fr / 2);
+    s->retired.limit = (size_t)std::min<int64_t>(s->budget / 8, 1 << 30);
     if (s->opts.resident) {
         s->t0 = Clock::now();
         if ((st = resident_create(s)) != WF_OK) {
@@ -891,7 +891,7 @@ void wf_server_destroy(wf_server *s)
         if (sl.done) (void)hipEventDestroy(sl.done);
         if (sl.stream) (void)hipStreamDestroy(sl.stream);
     }
-    for (void *p : s->retired) (void)hipFree(p);
+    s->retired.release();
     if (s->ctx) wf_ctx_destroy(s->ctx);
     delete s;
 }
