@@ -459,8 +459,11 @@ static bool split_enabled()
 }
 // Byte row tables for SW pairs of at most 4 symbols (WFK_MODE_PERM4): on
 // unless WFDP_PERM=0 (wf_perm4_enabled).
-// Pairs narrower than this are not split.
-constexpr int64_t kSplitMinCols = 1024;
+// Bit-parallel pairs narrower than this are not split: half the steps have to
+// pay for the combine launch (us a call, split / unsplit: ED 512^2 53 / 53, 640^2 55
+// / 58, 800^2 60 / 65, 1000^2 62 / 71; LCS, whose steps are shorter, 640^2 47 / 46,
+// 800^2 50 / 50, 1000^2 52 / 54).
+constexpr int64_t kSplitMinColsEd = 576, kSplitMinColsLcs = 832;
 // SW pairs narrower than this are not split (measured gains of the split:
 // 13% at 1024 x 1024, 17% at 2048 x 2048, 30% at 3000 x 600).
 constexpr int64_t kSwSplitMinCols = 1024;
@@ -538,7 +541,7 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
         const int64_t cus = ctx ? ctx->prop.multiProcessorCount : 256;
         if (2 * strips <= cus)
             for (int64_t i = 0; i < njobs; ++i)
-                if (jobs[i].n1 >= kSplitMinCols && jobs[i].n2 > 0) {
+                if (jobs[i].n1 >= (jobs[i].problem == WF_ED ? kSplitMinColsEd : kSplitMinColsLcs) && jobs[i].n2 > 0) {
                     mid[i] = jobs[i].n1 / 2;
                     ++nextra;
                 }

@@ -47,6 +47,20 @@ def test_bitpar_staircase(ctx, n1, n2, problem, textbook, related):
     p.close()
 
 
+@pytest.mark.parametrize("problem,edge", [("ED", 576), ("LCS", 832)])
+def test_bitpar_split_narrowest(ctx, problem, edge):
+    """One column either side of the narrowest split pair, one strip and many
+    (whose lag is then a few steps)."""
+    rng = np.random.default_rng(edge)
+    for n1, n2 in ((edge - 1, 900), (edge, 900), (edge, 30001), (edge + 1, 4097)):
+        a, b = _pair(rng, n1, n2, 20 if problem == "ED" else 4, "head")
+        p = ctx.plan([Job(problem, a, b)])
+        assert p.describe()["tasks"] == (1 if n1 < edge else 2) * -(-n2 // 2048)
+        p.run()
+        assert p.results()[0].last == O.score(problem, a, b)[0]
+        p.close()
+
+
 def test_bitpar_staircase_graph_replays(ctx):
     rng = np.random.default_rng(5)
     jobs = [Job("ED", *_pair(rng, 3001, 7000, 20, "head")), Job("LCS", *_pair(rng, 700, 900, 4, "")),
