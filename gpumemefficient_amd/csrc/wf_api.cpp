@@ -883,29 +883,37 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     ph->tasks.clear();
     ph->task_begin.assign(np, 0);
     ph->task_end.assign(np, 0);
-    // The parts of a two-part split are one entry of the list, strip by strip:
+    // The parts of a split pair are one entry of the list, so that a launch per
+    // pair (WF_RUN_PER_PAIR) runs them side by side too (SW 7013 x 3001, 20
+    // symbols: 200 us, 700 in a launch per part, unsplit 333).  Those of a two-part
+    // split go strip by strip:
     // the early strips of all parts, which run from the start, are then claimed
     // by the first workgroup of each CU and the late ones by the second (SW
-    // 131072^2, 512 strips: 4.74 ms, part by part 5.88).  Not so the other
-    // splits, whose f0 strips all start at once (65536^2, 384 strips: 1.74 ms
-    // part by part, 2.94 strip by strip).
+    // 131072^2, 512 strips: 4.74 ms, part by part 5.88).  The other splits' go
+    // part by part: their f0 strips all start at once (65536^2, 384 strips:
+    // 1.74 ms part by part, 2.94 strip by strip).
     std::vector<std::vector<int32_t>> parts(np);
     std::vector<int64_t> owner(np);
     std::iota(owner.begin(), owner.end(), 0);
     for (int64_t i = 0; i < np; ++i) parts[i].push_back((int32_t)i);
-    if (two_part)
-        for (const WfSplitDev &sp : ph->splits)
-            for (int32_t p : {sp.rev, sp.crev})
-                if (p >= 0) {
-                    parts[sp.job].push_back(p);
-                    owner[p] = sp.job;
-                }
+    for (const WfSplitDev &sp : ph->splits)
+        for (int32_t p : {sp.prob == WFK_SW ? sp.f0 : -1, sp.rev, sp.crev})
+            if (p >= 0) {
+                parts[sp.job].push_back(p);
+                owner[p] = sp.job;
+            }
     for (int64_t k = 0; k < np; ++k) {
         const int64_t i = owner[order[k]];
         if (parts[i].empty()) continue;  // with the part that came first
         ph->task_begin[i] = (int64_t)ph->tasks.size();
-        for (int32_t g = 0; g < ph->pairs[i].ngroups; ++g)
-            for (int32_t p : parts[i]) ph->tasks.push_back(WfTaskDev{p, g});
+        const int32_t ng = ph->pairs[i].ngroups;  // (the same in all parts)
+        if (two_part) {
+            for (int32_t g = 0; g < ng; ++g)
+                for (int32_t p : parts[i]) ph->tasks.push_back(WfTaskDev{p, g});
+        } else {
+            for (int32_t p : parts[i])
+                for (int32_t g = 0; g < ng; ++g) ph->tasks.push_back(WfTaskDev{p, g});
+        }
         ph->task_end[i] = (int64_t)ph->tasks.size();
         parts[i].clear();
     }

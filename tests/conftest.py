@@ -7,6 +7,7 @@ import pytest
 ROOT = Path(__file__).resolve().parent.parent
 sys.path.insert(0, str(ROOT))
 sys.path.insert(0, str(ROOT / "oracle"))
+sys.path.insert(0, str(ROOT / "tests"))
 
 
 def pytest_configure(config):
@@ -30,3 +31,10 @@ def ctx():
         raise
     yield c
     c.close()
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    """The host code on a HIP runtime without a GPU (tests/fake_device.py)."""
+    import fake_device
+    return fake_device.build(tmp_path_factory.mktemp("fake"))
