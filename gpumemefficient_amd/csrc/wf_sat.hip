@@ -200,7 +200,7 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
 
     // Row carries: lane l adds up row l % 16 over the tiles tc' = l / 16 mod 4
     // left of this one; carry: the inclusive prefix over the wave's rows.
-    int carry = 0;
+    uint32_t carry = 0;
     if (tc > 0) {
         const uint64_t *rp = a.rowsum + (int64_t)tr * a.ntc * kTR + wave * kRW + (lane & 15);
         for (int j = 0; j < tc; j += 16) {
@@ -231,13 +231,13 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                carry += (j + 4 * k + (lane >> 4) < tc) ? (int)(uint32_t)w[k] : 0;
+                carry += (j + 4 * k + (lane >> 4) < tc) ? (uint32_t)w[k] : 0u;
         }
-        carry = (int)((uint32_t)carry + (uint32_t)__shfl_xor(carry, 16));
-        carry = (int)((uint32_t)carry + (uint32_t)__shfl_xor(carry, 32));
-        carry = scan16(carry);
+        carry += (uint32_t)__shfl_xor((int)carry, 16);
+        carry += (uint32_t)__shfl_xor((int)carry, 32);
+        carry = (uint32_t)scan16((int)carry);
     }
-    if (lane == kRW - 1) sh.rows[wave] = carry;
+    if (lane == kRW - 1) sh.rows[wave] = (int)carry;
     __syncthreads();
 
     // What the waves above add to each column of this wave's rows.
@@ -282,7 +282,7 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
             for (int k = 0; k < kLC; ++k) top[k] = (uint32_t)w[k];
         }
         if (tr + 1 < a.ntr) {
-            const uint32_t all = (uint32_t)__builtin_amdgcn_readlane(carry, kRW - 1);
+            const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)carry, kRW - 1);
             uint64_t *d = a.bottom + ((int64_t)tr * a.ntc + tc) * kTC + lane;
 #pragma unroll
             for (int k = 0; k < kLC; ++k)
@@ -312,7 +312,7 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
     for (int h = 0; h < 2; ++h) soff[h] = c + 4 * h + 3 <= n1 ? voff[h] : kOut;
 #pragma unroll
     for (int r = 0; r < kRW; ++r) {
-        const uint32_t rc = (uint32_t)__builtin_amdgcn_readlane(carry, r);
+        const uint32_t rc = (uint32_t)__builtin_amdgcn_readlane((int)carry, r);
         uint32_t o[kLC];
 #pragma unroll
         for (int k = 0; k < kLC; ++k) o[k] = (uint32_t)v[r][k] + add[k] + rc;
