@@ -10,7 +10,7 @@
 //
 // so it needs no wavefront: addition mod 2^32 is associative and every order
 // gives the reference's bits.  Putting d(y) in place of the row's column-0
-// value makes p a plain row prefix and gives T'(y,0) = T(y,0) back.
+// value makes p a plain row prefix.
 //
 // Each workgroup takes one tile of 128 rows x 512 columns into registers
 // (wave w rows 16w.., lane l columns 8l..8l+7), scans its rows (seven adds in
@@ -305,11 +305,16 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
         add[6] += (uint32_t)s1.z;
         add[7] += (uint32_t)s1.w;
     }
-    // Vectors that lie within the columns <= n1 go out whole; the one that
-    // reaches past them (the table's right boundary columns) cell by cell.
+    // Vectors that lie within the columns 1..n1 go out whole; those that reach
+    // past them (the table's boundary columns, which are not written) cell by
+    // cell.
+    bool whole[2];
     uint32_t soff[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) soff[h] = c + 4 * h + 3 <= n1 ? voff[h] : kOut;
+    for (int h = 0; h < 2; ++h) {
+        whole[h] = c + 4 * h >= 1 && c + 4 * h + 3 <= n1;
+        soff[h] = whole[h] ? voff[h] : kOut;
+    }
 #pragma unroll
     for (int r = 0; r < kRW; ++r) {
         const uint32_t rc = (uint32_t)__builtin_amdgcn_readlane((int)carry, r);
@@ -322,15 +327,17 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
             const u4 q = {o[4 * h], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]};
             __builtin_amdgcn_raw_buffer_store_b128(q, rs, soff[h] + r * pitch, 0, 0);
         }
-        if (edge) {
+        if (edge || tc == 0) {
+            // (Three cells: column 0's vector starts at column 1.)
+            const int first = c == 0 ? 1 : 0;
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    const int x = c + 4 * h + k;
-                    const bool tail = c + 4 * h + 3 > n1 && x <= n1;
-                    __builtin_amdgcn_raw_buffer_store_b32(o[4 * h + k], rs, (tail ? (uint32_t)x * 4u : kOut) + r * pitch, 0,
-                                                           0);
+                    const int x = c + 4 * h + k + (h == 0 ? first : 0);
+                    const bool cell = !whole[h] && x <= n1;
+                    const uint32_t q = h == 0 && first ? o[k + 1] : o[4 * h + k];
+                    __builtin_amdgcn_raw_buffer_store_b32(q, rs, (cell ? (uint32_t)x * 4u : kOut) + r * pitch, 0, 0);
                 }
         }
     }
