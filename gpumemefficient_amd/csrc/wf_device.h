@@ -227,13 +227,15 @@ struct WfStencilArgs {
 
 // Kernel argument block of a summed-area table (wf_sat.hip): the table as
 // above, in ntr x ntc tiles.
-enum { WFS_SAT_TILE_ROWS = 128, WFS_SAT_TILE_COLS = 512 };
+enum { WFS_SAT_TILE_ROWS = 128, WFS_SAT_TILE_COLS = 512, WFS_SAT_BLOCK_TILES = 64 };
 struct WfSatArgs {
     int32_t *t;
     int64_t ld;
     int32_t n1, n2;
     int32_t ntr, ntc;
+    int32_t nblk;            // blocks of WFS_SAT_BLOCK_TILES tile columns
     uint64_t *rowsum;        // [ntr][ntc][WFS_SAT_TILE_ROWS] words (epoch << 32) | value: row sums of each tile
+    uint64_t *blksum;        // [ntr][nblk][WFS_SAT_TILE_ROWS] words: row sums up to a block's last tile
     uint64_t *bottom;        // [ntr][ntc][WFS_SAT_TILE_COLS] words: each tile's finished bottom row
     int32_t *counter;        // tile claim counter (zeroed by the reset kernel)
     WfResultDev *res;        // res[0].status: timeout flag

@@ -20,8 +20,14 @@
 // words with relaxed device-scope atomics, as the strip boundaries do:
 //
 //   rows     every tile publishes its 128 row sums as soon as it has them;
-//            a tile adds up those of all tiles to its left.  No chain: a
-//            tile's sums do not wait for anybody.
+//            a tile adds up those of the tiles to its left in its block of 64
+//            tile columns.  No chain: a tile's sums do not wait for anybody.
+//            A block's last tile publishes the sums of all columns up to its
+//            own instead, which the next block's tiles add: a chain of one hop
+//            per 32768 columns.  (With all tiles to the left read by each,
+//            what is read grows with the square of the width and passes the
+//            cells' traffic at 260 000 columns: 4M x 1024 30.3 ms against 6.8,
+//            13M x 512 139 against 10.9.  Blocks of 32 or 128 tiles: 6.7, 7.9.)
 //   columns  a tile's bottom row T'(y_end, x) needs the one of the tile above.
 //            This chain has n2 / 128 hops of about 1.3 us, so a tile forms its own part
 //            first and only adds the row above when it arrives, publishing
@@ -50,7 +56,8 @@ using wfk::now_ticks;
 constexpr int kRW = 16;    // rows of a wave
 constexpr int kLC = 8;     // columns of a lane
 constexpr int kW = 8;      // waves of a workgroup: two a SIMD, 256 VGPRs each, 128 of them the tile's cells
-constexpr int kTR = WFS_SAT_TILE_ROWS, kTC = WFS_SAT_TILE_COLS;
+constexpr int kTR = WFS_SAT_TILE_ROWS, kTC = WFS_SAT_TILE_COLS, kTB = WFS_SAT_BLOCK_TILES;
+static_assert(kTB % 16 == 0, "a block's tiles are read 16 at a time");
 static_assert(kTR == kW * kRW && kTC == 64 * kLC, "waves stack down the tile, a wave spans its columns");
 
 struct SatShared {
@@ -90,13 +97,11 @@ __device__ __forceinline__ void store_word(uint64_t *p, uint64_t v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// N words p[0], p[stride], ... polled until all carry the tag; false (and the
+// Polls the N loaded words w[k] = *at(k) until all carry the tag; false (and the
 // words as they are) once the wait exceeds the limit.
-template <int N>
-__device__ __forceinline__ bool wait_words(const uint64_t *p, int stride, uint32_t epoch, int64_t limit, uint64_t (&w)[N])
+template <int N, class At>
+__device__ __forceinline__ bool wait_words(At &&at, uint32_t epoch, int64_t limit, uint64_t (&w)[N])
 {
-#pragma unroll
-    for (int k = 0; k < N; ++k) w[k] = load_word(p + k * stride);
     int64_t t0 = 0;
     for (int spins = 0;; ++spins) {
         bool stale = false;
@@ -111,7 +116,7 @@ __device__ __forceinline__ bool wait_words(const uint64_t *p, int stride, uint32
         __builtin_amdgcn_s_sleep(1);
 #pragma unroll
         for (int k = 0; k < N; ++k)
-            if ((uint32_t)(w[k] >> 32) != epoch) w[k] = load_word(p + k * stride);
+            if ((uint32_t)(w[k] >> 32) != epoch) w[k] = load_word(at(k));
     }
 }
 
@@ -184,7 +189,9 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
         const int sum = __builtin_amdgcn_readlane(incl, 63);
         rowsum = lane == r ? sum : rowsum;
     }
-    if (tc + 1 < a.ntc && lane < kRW)
+    const int blk = tc / kTB;  // the tile's block of tile columns
+    const bool ends_blk = tc % kTB == kTB - 1;
+    if (tc + 1 < a.ntc && !ends_blk && lane < kRW)
         store_word(a.rowsum + ((int64_t)tr * a.ntc + tc) * kTR + wave * kRW + lane, tag | (uint32_t)rowsum);
 
     // Column prefixes of the wave's rows.
@@ -198,12 +205,15 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
         d[1] = make_int4(v[kRW - 1][4], v[kRW - 1][5], v[kRW - 1][6], v[kRW - 1][7]);
     }
 
-    // Row carries: lane l adds up row l % 16 over the tiles tc' = l / 16 mod 4
-    // left of this one; carry: the inclusive prefix over the wave's rows.
+    // Row carries: lane l adds up row l % 16 over the tiles l / 16 mod 4 of its
+    // block left of this one, and the blocks before; carry: the inclusive prefix
+    // over the wave's rows.
     uint32_t carry = 0;
     if (tc > 0) {
+        const uint64_t *bp = a.blksum + ((int64_t)tr * a.nblk + blk - 1) * kTR + wave * kRW + (lane & 15);
+        uint64_t wb[1] = {blk > 0 ? load_word(bp) : tag};
         const uint64_t *rp = a.rowsum + (int64_t)tr * a.ntc * kTR + wave * kRW + (lane & 15);
-        for (int j = 0; j < tc; j += 16) {
+        for (int j = blk * kTB; j < tc; j += 16) {
             uint64_t w[4];
             // Tiles past the last one left of this tile: its own first
             // predecessor again, added as zero.
@@ -212,31 +222,20 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
             for (int k = 0; k < 4; ++k) q[k] = rp + (int64_t)min(j + 4 * k + (lane >> 4), tc - 1) * kTR;
 #pragma unroll
             for (int k = 0; k < 4; ++k) w[k] = load_word(q[k]);
-            int64_t t0 = 0;
-            for (int spins = 0;; ++spins) {
-                bool stale = false;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) stale = stale || (uint32_t)(w[k] >> 32) != epoch;
-                if (__builtin_amdgcn_ballot_w64(stale) == 0) break;
-                const int64_t t = now_ticks();
-                if (spins == 0) t0 = t;
-                if (t - t0 > a.timeout_ticks) {
-                    if (lane == 0) atomicOr(&a.res->status, 1);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if ((uint32_t)(w[k] >> 32) != epoch) w[k] = load_word(q[k]);
-            }
+            if (!wait_words([&](int k) { return q[k]; }, epoch, a.timeout_ticks, w) && lane == 0)
+                atomicOr(&a.res->status, 1);
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 carry += (j + 4 * k + (lane >> 4) < tc) ? (uint32_t)w[k] : 0u;
         }
+        if (!wait_words([&](int) { return bp; }, epoch, a.timeout_ticks, wb) && lane == 0) atomicOr(&a.res->status, 1);
+        carry += lane < kRW ? (uint32_t)wb[0] : 0u;
         carry += (uint32_t)__shfl_xor((int)carry, 16);
         carry += (uint32_t)__shfl_xor((int)carry, 32);
-        carry = (uint32_t)scan16((int)carry);
     }
+    if (ends_blk && tc + 1 < a.ntc && lane < kRW)
+        store_word(a.blksum + ((int64_t)tr * a.nblk + blk) * kTR + wave * kRW + lane, tag | (carry + (uint32_t)rowsum));
+    carry = (uint32_t)scan16((int)carry);
     if (lane == kRW - 1) sh.rows[wave] = (int)carry;
     __syncthreads();
 
@@ -274,9 +273,11 @@ __device__ __forceinline__ void sat_tile(const WfSatArgs &a, int tr, int tc, Sat
 #pragma unroll
             for (int k = 0; k < kLC; ++k) top[k] = c + k <= n1 ? (uint32_t)a.t[c + k] : 0u;
         } else {
+            const uint64_t *q = a.bottom + ((int64_t)(tr - 1) * a.ntc + tc) * kTC + lane;
             uint64_t w[kLC];
-            if (!wait_words(a.bottom + ((int64_t)(tr - 1) * a.ntc + tc) * kTC + lane, 64, epoch, a.timeout_ticks, w) &&
-                lane == 0)
+#pragma unroll
+            for (int k = 0; k < kLC; ++k) w[k] = load_word(q + 64 * k);
+            if (!wait_words([&](int k) { return q + 64 * k; }, epoch, a.timeout_ticks, w) && lane == 0)
                 atomicOr(&a.res->status, 1);
 #pragma unroll
             for (int k = 0; k < kLC; ++k) top[k] = (uint32_t)w[k];

@@ -57,8 +57,11 @@ int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double
     const int cus = ctx->prop.multiProcessorCount;
     const int64_t ntc = (n1 + 1 + WFS_SAT_TILE_COLS - 1) / WFS_SAT_TILE_COLS;  // columns 0..n1
     const int64_t tr = WFS_SAT_TILE_ROWS, ntr = (n2 + tr - 1) / tr;
+    const int64_t nblk = (ntc + WFS_SAT_BLOCK_TILES - 1) / WFS_SAT_BLOCK_TILES;
     int st;
-    if ((st = ar->bnd.ensure((size_t)(ntr * ntc * (tr + WFS_SAT_TILE_COLS)) * sizeof(uint64_t), true)) != WF_OK) return st;
+    if ((st = ar->bnd.ensure((size_t)(ntr * ((ntc + nblk) * tr + ntc * WFS_SAT_TILE_COLS)) * sizeof(uint64_t), true)) !=
+        WF_OK)
+        return st;
     if ((st = ar->res.ensure(sizeof(WfResultDev))) != WF_OK) return st;
     if ((st = ar->counters.ensure(2 * sizeof(int32_t))) != WF_OK) return st;
     if ((st = ar->epoch.ensure(sizeof(uint32_t), true)) != WF_OK) return st;
@@ -69,8 +72,10 @@ int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double
     a.n2 = (int32_t)n2;
     a.ntr = (int32_t)ntr;
     a.ntc = (int32_t)ntc;
+    a.nblk = (int32_t)nblk;
     a.rowsum = (uint64_t *)ar->bnd.ptr;
-    a.bottom = a.rowsum + ntr * ntc * tr;
+    a.blksum = a.rowsum + ntr * ntc * tr;
+    a.bottom = a.blksum + ntr * nblk * tr;
     a.counter = (int32_t *)ar->counters.ptr;
     a.res = (WfResultDev *)ar->res.ptr;
     a.epoch = (const uint32_t *)ar->epoch.ptr;
