@@ -1136,7 +1136,7 @@ int wf_enqueue_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar, int mode, int max
 {
     const int64_t ncounters = ph->npairs + 1;
     if (reset && wf_launch_reset((WfResultDev *)ar->res.ptr, ph->npairs, (int32_t *)ar->counters.ptr, ncounters,
-                                 (uint32_t *)ar->epoch.ptr, stream) != hipSuccess)
+                                 (uint32_t *)ar->epoch.ptr, 1, stream) != hipSuccess)
         return WF_ERR_DEVICE;
     WfKernelArgs ka{};
     ka.pairs = (const WfPairDev *)ar->pairs.ptr;
@@ -1400,7 +1400,7 @@ int wf_align_table(wf_ctx *ctx, int problem, const int32_t *a, int64_t n1, const
     if ((st = dt.ensure((size_t)(n1 * n2) * sizeof(int32_t))) != WF_OK) return st;
     WfArenas *ar = &ctx->scratch;
     if (wf_launch_reset((WfResultDev *)ar->res.ptr, 1, (int32_t *)ar->counters.ptr, 2, (uint32_t *)ar->epoch.ptr,
-                        ctx->stream) != hipSuccess)
+                        1, ctx->stream) != hipSuccess)
         return WF_ERR_DEVICE;
     WfKernelArgs ka{};
     ka.pairs = (const WfPairDev *)ar->pairs.ptr;

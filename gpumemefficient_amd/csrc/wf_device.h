@@ -234,9 +234,10 @@ struct WfSatArgs {
     int32_t n1, n2;
     int32_t ntr, ntc;
     int32_t nblk;            // blocks of WFS_SAT_BLOCK_TILES tile columns
-    uint64_t *rowsum;        // [ntr][ntc][WFS_SAT_TILE_ROWS] words (epoch << 32) | value: row sums of each tile
-    uint64_t *blksum;        // [ntr][nblk][WFS_SAT_TILE_ROWS] words: row sums up to a block's last tile
-    uint64_t *bottom;        // [ntr][ntc][WFS_SAT_TILE_COLS] words: each tile's finished bottom row
+    int32_t ring, tags;      // rows of `bottom`; tags of the launch, the last of which is the epoch
+    uint64_t *rowsum;        // [ntr][ntc - 1][WFS_SAT_TILE_ROWS] words (epoch << 32) | value: row sums of each tile
+    uint64_t *blksum;        // [ntr][nblk - 1][WFS_SAT_TILE_ROWS] words: row sums up to a block's last tile
+    uint64_t *bottom;        // [ring][ntc][WFS_SAT_TILE_COLS] words, a tag per turn: each tile's finished bottom row
     int32_t *counter;        // tile claim counter (zeroed by the reset kernel)
     WfResultDev *res;        // res[0].status: timeout flag
     const uint32_t *epoch;

@@ -606,12 +606,14 @@ __global__ __launch_bounds__(64 * W, (lockstep_min_blocks<R, W>())) void wf_serv
 
 // Zero progress counters, results and claim counters before a launch (a
 // kernel rather than hipMemsetAsync so the sequence can be graph-captured).
-// Also advances the launch epoch that tags strip-boundary values.
-__global__ void wf_reset(WfResultDev *res, int64_t nres, int32_t *counters, int64_t ncounters, uint32_t *epoch)
+// Also advances the launch epoch that tags strip-boundary values, by the number
+// of tags the launch uses.
+__global__ void wf_reset(WfResultDev *res, int64_t nres, int32_t *counters, int64_t ncounters, uint32_t *epoch,
+                         uint32_t tags)
 {
     const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    if (i0 == 0) *epoch = *epoch + 1u;
+    if (i0 == 0) *epoch = *epoch + tags;
     for (int64_t i = i0; i < nres; i += stride) res[i] = WfResultDev{0, 0, 0, 0};
     for (int64_t i = i0; i < ncounters; i += stride) counters[i] = 0;
 }
@@ -637,14 +639,15 @@ extern "C" const WfVariant wf_variants_lockstep[] = {
 extern "C" const int wf_num_variants_lockstep = sizeof(wf_variants_lockstep) / sizeof(wf_variants_lockstep[0]);
 
 extern "C" hipError_t wf_launch_reset(WfResultDev *res, int64_t nres, int32_t *counters, int64_t ncounters,
-                                      uint32_t *epoch, hipStream_t stream)
+                                      uint32_t *epoch, uint32_t tags, hipStream_t stream)
 {
     int64_t n = nres;
     if (ncounters > n) n = ncounters;
     int blocks = (int)((n + 255) / 256);
     if (blocks < 1) blocks = 1;
     if (blocks > 1024) blocks = 1024;
-    hipLaunchKernelGGL(wfk::wf_reset, dim3(blocks), dim3(256), 0, stream, res, nres, counters, ncounters, epoch);
+    hipLaunchKernelGGL(wfk::wf_reset, dim3(blocks), dim3(256), 0, stream, res, nres, counters, ncounters, epoch,
+                       tags);
     return hipGetLastError();
 }
 

@@ -11,6 +11,17 @@
 
 namespace {
 
+// What a sweep may keep beside the table, in words: a row of the table for every
+// 256 rows (1/32 byte a cell), or 8 MiB.  A table near the device's memory leaves
+// no more.
+int64_t sweep_words(int64_t n1, int64_t n2)
+{
+    return std::max<int64_t>(((n2 + 255) / 256 - 1) * (n1 + 1), 1 << 20);
+}
+// Fewest rows of the ring that the workgroups of a sweep hand their bottom rows
+// down in.
+constexpr int64_t kSweepRing = 4;
+
 // A tile's strip height and rows per lane are checked and not used: both
 // kernels have one shape (every shape gives the same table).
 int check_tile(const wf_tile *tile)
@@ -23,9 +34,10 @@ int check_tile(const wf_tile *tile)
 
 // Reset and one launch of a sweep, timed with HIP events; the status and the
 // table's last interior cell come back behind it through the context's pinned
-// block, with one wait for everything.
+// block, with one wait for everything.  tags: of the words that the launch's
+// workgroups exchange.
 template <class Launch>
-int run_timed(wf_ctx *ctx, WfArenas *ar, const int32_t *cell, double *ms, int32_t *last, Launch &&launch)
+int run_timed(wf_ctx *ctx, WfArenas *ar, int64_t tags, const int32_t *cell, double *ms, int32_t *last, Launch &&launch)
 {
     int st;
     if ((st = wf_ensure_pinned(ctx, 256)) != WF_OK) return st;
@@ -33,7 +45,7 @@ int run_timed(wf_ctx *ctx, WfArenas *ar, const int32_t *cell, double *ms, int32_
     int32_t *l = reinterpret_cast<int32_t *>(ctx->pinned + 128);
     if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
     if (wf_launch_reset((WfResultDev *)ar->res.ptr, 1, (int32_t *)ar->counters.ptr, 2, (uint32_t *)ar->epoch.ptr,
-                        ctx->stream) != hipSuccess)
+                        (uint32_t)tags, ctx->stream) != hipSuccess)
         return WF_ERR_DEVICE;
     if (launch() != hipSuccess) return WF_ERR_DEVICE;
     if (hipEventRecord(ctx->ev1, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
@@ -58,10 +70,17 @@ int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double
     const int64_t ntc = (n1 + 1 + WFS_SAT_TILE_COLS - 1) / WFS_SAT_TILE_COLS;  // columns 0..n1
     const int64_t tr = WFS_SAT_TILE_ROWS, ntr = (n2 + tr - 1) / tr;
     const int64_t nblk = (ntc + WFS_SAT_BLOCK_TILES - 1) / WFS_SAT_BLOCK_TILES;
+    // The tiles' bottom rows go round a ring: a tile's is overwritten by the one
+    // `ring` tile rows below, which has had all those between, and a tag per turn
+    // tells them apart.  With the rows' sums that takes no more memory than a
+    // bottom row every 256 rows would (sweep_words; all tile rows: 1/13 byte a
+    // cell, and 40 a row in tables of one tile column).
+    const int64_t sums = ntr * tr * (ntc - 1 + nblk - 1), brow = ntc * WFS_SAT_TILE_COLS;
+    const int64_t rows = std::max<int64_t>(1, ntr - 1);
+    const int64_t ring = std::min(rows, std::max(kSweepRing, (sweep_words(n1, n2) - sums) / brow));
+    const int64_t tags = (rows - 1) / ring + 1;
     int st;
-    if ((st = ar->bnd.ensure((size_t)(ntr * ((ntc + nblk) * tr + ntc * WFS_SAT_TILE_COLS)) * sizeof(uint64_t), true)) !=
-        WF_OK)
-        return st;
+    if ((st = ar->bnd.ensure((size_t)(sums + ring * brow) * sizeof(uint64_t), true)) != WF_OK) return st;
     if ((st = ar->res.ensure(sizeof(WfResultDev))) != WF_OK) return st;
     if ((st = ar->counters.ensure(2 * sizeof(int32_t))) != WF_OK) return st;
     if ((st = ar->epoch.ensure(sizeof(uint32_t), true)) != WF_OK) return st;
@@ -74,14 +93,16 @@ int run_sat(wf_ctx *ctx, int64_t n1, int64_t n2, int32_t *dt, int64_t ld, double
     a.ntc = (int32_t)ntc;
     a.nblk = (int32_t)nblk;
     a.rowsum = (uint64_t *)ar->bnd.ptr;
-    a.blksum = a.rowsum + ntr * ntc * tr;
-    a.bottom = a.blksum + ntr * nblk * tr;
+    a.blksum = a.rowsum + ntr * (ntc - 1) * tr;
+    a.bottom = a.rowsum + sums;
+    a.ring = (int32_t)ring;
+    a.tags = (int32_t)tags;
     a.counter = (int32_t *)ar->counters.ptr;
     a.res = (WfResultDev *)ar->res.ptr;
     a.epoch = (const uint32_t *)ar->epoch.ptr;
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
     const int grid = (int)std::min<int64_t>(ntr * ntc, std::max(1, wf_sat_resident(cus)));
-    return run_timed(ctx, ar, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_sat(grid, &a, ctx->stream); });
+    return run_timed(ctx, ar, tags, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_sat(grid, &a, ctx->stream); });
 }
 
 // The sweep on a device table (pitch ld, ld % 4 == 0, 16-byte aligned); last:
@@ -115,7 +136,7 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
     const int lim = wf_stencil_resident(ctx->prop.multiProcessorCount);
     const int grid = (int)std::min<int64_t>(strips, std::max(1, lim));
-    return run_timed(ctx, ar, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
+    return run_timed(ctx, ar, 1, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
 }
 
 // Host table -> device copy of pitch ldd -> sweep -> host table (or only the

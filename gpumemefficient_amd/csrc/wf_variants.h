@@ -28,7 +28,7 @@ extern "C" const WfVariant wf_variants_bitpar[];
 extern "C" const int wf_num_variants_bitpar;
 
 extern "C" hipError_t wf_launch_reset(WfResultDev *res, int64_t nres, int32_t *counters, int64_t ncounters,
-                                      uint32_t *epoch, hipStream_t stream);
+                                      uint32_t *epoch, uint32_t tags, hipStream_t stream);
 // Lock-step <2,4,32> sweep that also writes every cell of pair 0 to ka->table.
 extern "C" hipError_t wf_launch_table(int grid, const WfKernelArgs *ka, hipStream_t stream);
 // Naive baselines (wf_naive.hip): method 0 one launch per cell

@@ -180,7 +180,10 @@ hipError_t wf_launch_engine(const WfVariant *v, int, const WfKernelArgs *ka, hip
     g_tasks += ka->task_end - ka->task_begin;
     return hipSuccess;
 }
-hipError_t wf_launch_reset(WfResultDev *, int64_t, int32_t *, int64_t, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t wf_launch_reset(WfResultDev *, int64_t, int32_t *, int64_t, uint32_t *, uint32_t, hipStream_t)
+{
+    return hipSuccess;
+}
 hipError_t wf_launch_table(int, const WfKernelArgs *, hipStream_t) { return hipSuccess; }
 hipError_t wf_launch_naive(int, int, int, int *, const int32_t *, const int32_t *, int, int, int *, hipStream_t)
 {
