@@ -218,7 +218,8 @@ struct WfStencilArgs {
     int64_t ld;
     int32_t n1, n2;
     int32_t nstrips;         // strips of WFS_SOR_STRIP_ROWS rows
-    uint64_t *bnd;           // (nstrips - 1) rows of n1 + 1 words: (epoch << 32) | value
+    int32_t ring, tags;      // rows of `bnd`; tags of the launch, the last of which is the epoch
+    uint64_t *bnd;           // [ring][n1 + 1] words (tag of the turn << 32) | value: the strips' bottom rows
     int32_t *counter;        // strip claim counter (zeroed by the reset kernel)
     WfResultDev *res;        // res[0].status: timeout flag
     const uint32_t *epoch;

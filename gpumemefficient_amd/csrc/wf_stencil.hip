@@ -37,7 +37,8 @@
 // stores finished chunks back.  The boundary wave stages the row above for
 // lane 0 and publishes the strip's bottom row for the next strip, through HBM
 // as (launch epoch << 32 | value) words written and polled at device scope, as
-// the alignment engines do.  The compute wave touches LDS only: about 12 issue
+// the alignment engines do; the rows go round a ring, each turn with a tag of
+// its own (run_device in wf_stencil_api.cpp).  The compute wave touches LDS only: about 12 issue
 // slots a step, of which the division's v_mul_hi is four.  The three meet at a
 // barrier per chunk.  Strips are claimed in order from an atomic counter, so a
 // strip only waits on one that a running workgroup holds.
@@ -166,8 +167,17 @@ __device__ __forceinline__ void sor_strip(const WfStencilArgs &a, int g, StShare
     const int nch = (n1 + 63 + kK * kAhead - 1) / (kK * kAhead) * kAhead;
     const bool has_prev = g > 0;
     const bool has_next = g + 1 < a.nstrips;
-    const uint64_t *bprev = a.bnd + (int64_t)(g - 1) * (n1 + 1);
-    uint64_t *bnext = a.bnd + (int64_t)g * (n1 + 1);
+    // Rows and tags of the ring of bottom rows: the strip's, the strip above's.
+    int rout = g;
+    uint32_t tout = epoch - (uint32_t)(a.tags - 1);
+    if (g >= a.ring) {
+        rout = g % a.ring;
+        tout += (uint32_t)(g / a.ring);
+    }
+    const int rin = rout > 0 ? rout - 1 : a.ring - 1;
+    const uint32_t tin = rout > 0 ? tout : tout - 1u;
+    const uint64_t *bprev = a.bnd + (int64_t)rin * (n1 + 1);
+    uint64_t *bnext = a.bnd + (int64_t)rout * (n1 + 1);
     int *win = sh.win;
 
     if (wave == 0) {
@@ -235,7 +245,7 @@ __device__ __forceinline__ void sor_strip(const WfStencilArgs &a, int g, StShare
         // chunks.
         auto need = [&](int c) __attribute__((always_inline)) { return min(n1, c * kK + kK + 1); };
         auto examine = [&](Poll &p, int c) __attribute__((always_inline)) {
-            const bool ready = p.x <= n1 && (!has_prev || p.v.y == epoch);
+            const bool ready = p.x <= n1 && (!has_prev || p.v.y == tin);
             const uint64_t late = ~__builtin_amdgcn_ballot_w64(ready);
             const int upto = min(__builtin_amdgcn_readfirstlane(p.x) - 1 + (late ? (int)__builtin_ctzll(late) : 64),
                                  need(c + 5));
@@ -260,7 +270,7 @@ __device__ __forceinline__ void sor_strip(const WfStencilArgs &a, int g, StShare
             rows_rsrc(has_next ? (const void *)bnext : (const void *)a.t, has_next ? (n1 + 1) * 8LL : 0);
         auto publish = [&](int c) __attribute__((always_inline)) {
             const int s = c * kK + (lane & (kK - 1)), x = s - 62;
-            const u2 v = {(uint32_t)win[63 * kTS + (s & (kTW - 1))], epoch};
+            const u2 v = {(uint32_t)win[63 * kTS + (s & (kTW - 1))], tout};
             __builtin_amdgcn_raw_buffer_store_b64(
                 v, pubr, (lane < kK && c >= 0 && x >= 1 && x <= n1) ? (uint32_t)x * 8u : kOut, 0, kCoherent);
         };

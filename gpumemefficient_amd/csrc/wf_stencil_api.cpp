@@ -116,10 +116,13 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     if (op == WF_SAT) return run_sat(ctx, n1, n2, dt, ld, ms, last);
     WfArenas *ar = &ctx->scratch;
     const int64_t strips = (n2 + WFS_SOR_STRIP_ROWS - 1) / WFS_SOR_STRIP_ROWS;
+    // The strips' bottom rows go round a ring, as the tiles' do: a strip publishes
+    // a column after the strip above has, and so on up to the one that read it.
+    const int64_t rows = std::max<int64_t>(1, strips - 1);
+    const int64_t ring = std::min(rows, std::max(kSweepRing, sweep_words(n1, n2) / (n1 + 1)));
+    const int64_t tags = (rows - 1) / ring + 1;
     int st;
-    if ((st = ar->bnd.ensure((size_t)std::max<int64_t>(1, (strips - 1) * (n1 + 1)) * sizeof(uint64_t), true)) !=
-        WF_OK)
-        return st;
+    if ((st = ar->bnd.ensure((size_t)(ring * (n1 + 1)) * sizeof(uint64_t), true)) != WF_OK) return st;
     if ((st = ar->res.ensure(sizeof(WfResultDev))) != WF_OK) return st;
     if ((st = ar->counters.ensure(2 * sizeof(int32_t))) != WF_OK) return st;
     if ((st = ar->epoch.ensure(sizeof(uint32_t), true)) != WF_OK) return st;
@@ -129,6 +132,8 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     a.n1 = (int32_t)n1;
     a.n2 = (int32_t)n2;
     a.nstrips = (int32_t)strips;
+    a.ring = (int32_t)ring;
+    a.tags = (int32_t)tags;
     a.bnd = (uint64_t *)ar->bnd.ptr;
     a.counter = (int32_t *)ar->counters.ptr;
     a.res = (WfResultDev *)ar->res.ptr;
@@ -136,7 +141,7 @@ int run_device(wf_ctx *ctx, int op, int64_t n1, int64_t n2, int32_t *dt, int64_t
     a.timeout_ticks = (int64_t)(ctx->timeout_s * 1.0e8);
     const int lim = wf_stencil_resident(ctx->prop.multiProcessorCount);
     const int grid = (int)std::min<int64_t>(strips, std::max(1, lim));
-    return run_timed(ctx, ar, 1, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
+    return run_timed(ctx, ar, tags, dt + n2 * ld + n1, ms, last, [&] { return wf_launch_stencil(grid, &a, ctx->stream); });
 }
 
 // Host table -> device copy of pitch ldd -> sweep -> host table (or only the

@@ -10,7 +10,7 @@ TABLES = [(1, 4_000_000), (13, 1_000_000), (100, 100_000), (511, 60_000), (512, 
           (32_768, 32_768), (1_000_000, 6_000), (13_990_000, 4_900)]
 
 
-@pytest.mark.parametrize("op", ["SAT"])
+@pytest.mark.parametrize("op", ["SAT", "SOR"])
 @pytest.mark.parametrize("n1,n2", TABLES)
 def test_sweep_memory_is_a_boundary_row_per_256_rows(fake, op, n1, n2):
     """A sweep keeps no more beside the table than a word a column for every 256
