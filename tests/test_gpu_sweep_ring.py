@@ -48,3 +48,16 @@ def test_sweeps_and_pairs_take_turns():
                 assert (r.last, r.max_score) == tuple(want)
                 _, t = c.align_table("LCS", a[:600], b[:1500])
                 assert np.array_equal(t, table)
+
+
+@pytest.mark.parametrize("op,n1,n2", [("SAT", 9000, 4000), ("SOR", 100, 0)])
+def test_workgroups_claim_more_than_once(ctx, op, n1, n2):
+    """More tiles (strips) than the launch has workgroups, so that some claim a
+    second one."""
+    from gpumemefficient_amd import _lib
+    lib, cus = _lib.load(), ctx.info()["compute_units"]
+    if op == "SAT":
+        assert -(-n2 // 128) * -(-(n1 + 1) // 512) > lib.wf_sat_resident(cus)
+    else:
+        n2 = 64 * (lib.wf_stencil_resident(cus) + 300) + 7
+    _sweep(ctx, op, n1, n2, 11)
