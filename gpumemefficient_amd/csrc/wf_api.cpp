@@ -539,7 +539,7 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
         for (int64_t i = 0; i < njobs; ++i)
             if (jobs[i].n1 > 0 && jobs[i].n2 > 0) strips += (jobs[i].n2 + strip - 1) / strip;
         const int64_t cus = ctx ? ctx->prop.multiProcessorCount : 256;
-        if (2 * strips <= cus)
+        if (2 * strips <= std::min(cus, max_groups > 0 ? max_groups : INT64_MAX))
             for (int64_t i = 0; i < njobs; ++i)
                 if (jobs[i].n1 >= (jobs[i].problem == WF_ED ? kSplitMinColsEd : kSplitMinColsLcs) && jobs[i].n2 > 0) {
                     mid[i] = jobs[i].n1 / 2;
@@ -1022,7 +1022,8 @@ namespace {
 // device block it is copied to: codes, splits and cuts, pairs, tasks, the
 // cleared results and claim counters, the launch epoch.
 struct BlockLayout {
-    size_t codes = 0, splits, pairs, tasks, res, counters, epoch, end;
+    size_t codes = 0, splits = 0, pairs = 0, tasks = 0, res = 0, counters = 0, epoch = 0, end = 0;
+    BlockLayout() = default;
     explicit BlockLayout(const WfPlanHost *ph)
     {
         WfPlanBytes nb;
@@ -1083,6 +1084,23 @@ int upload_block(wf_ctx *ctx, WfPlanHost *ph, const BlockLayout &L, WfArenas *ar
     ar->bnd = sc->bnd;
     ar->colw = sc->colw;
     return WF_OK;
+}
+
+// Plans the jobs and gives the plan device memory in `ar` (`place`); where there
+// is not enough for the column splits, which take up to twice the boundary rows,
+// plans and places them once more without.
+template <class Place>
+int plan_and_place(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile, WfPlanHost *ph, WfArenas *ar,
+                   Place &&place)
+{
+    int st = wf_build_plan(ctx, jobs, njobs, tile, ph);
+    if (st != WF_OK) return st;
+    st = place();
+    if (st != WF_ERR_NOMEM || ph->splits.empty()) return st;
+    ar->release();
+    *ph = WfPlanHost();
+    if ((st = wf_build_plan(ctx, jobs, njobs, tile, ph, 1)) != WF_OK) return st;
+    return place();
 }
 
 }  // namespace
@@ -1349,11 +1367,13 @@ int wf_align_batch(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile
     if (njobs == 0) return WF_OK;
     if (hipSetDevice(ctx->device) != hipSuccess) return WF_ERR_DEVICE;
     WfPlanHost ph;
-    int st = wf_build_plan(ctx, jobs, njobs, tile, &ph);
-    if (st != WF_OK) return st;
-    const BlockLayout L(&ph);
+    BlockLayout L;
     WfArenas ar;
-    if ((st = upload_block(ctx, &ph, L, &ar)) != WF_OK) return st;
+    int st = plan_and_place(ctx, jobs, njobs, tile, &ph, &ctx->scratch, [&] {
+        L = BlockLayout(&ph);
+        return upload_block(ctx, &ph, L, &ar);
+    });
+    if (st != WF_OK) return st;
     if (hipEventRecord(ctx->ev0, ctx->stream) != hipSuccess) return WF_ERR_DEVICE;
     if ((st = wf_enqueue_plan(ctx, &ph, &ar, WF_RUN_PERSISTENT, wf_max_resident_groups(ctx, ph.variant), ctx->stream,
                               false)) != WF_OK)
@@ -1487,8 +1507,8 @@ int wf_plan_create(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile
     if (hipSetDevice(ctx->device) != hipSuccess) return WF_ERR_DEVICE;
     wf_plan *p = new wf_plan();
     p->ctx = ctx;
-    int st = wf_build_plan(ctx, jobs, njobs, tile, &p->host);
-    if (st == WF_OK) st = wf_upload_plan(ctx, &p->host, &p->own);
+    int st = plan_and_place(ctx, jobs, njobs, tile, &p->host, &p->own,
+                            [&] { return wf_upload_plan(ctx, &p->host, &p->own); });
     if (st == WF_OK) st = wf_ensure_pinned(ctx, (size_t)p->host.npairs * sizeof(WfResultDev));
     if (st != WF_OK) {
         p->own.release();

@@ -154,8 +154,8 @@ bool wf_tune_lookup(const char *arch, int cus, int problem, int batch, int bucke
 int wf_default_waves(int64_t max_rows, int64_t total_cells, int npairs);
 int wf_default_rows_per_lane(int waves, int64_t max_rows, int64_t total_cells, int npairs);
 // max_groups > 0: the launch runs at most that many workgroups (a server
-// slot's share of the chip); an SW column split is planned only if all its
-// strips fit in them.
+// slot's share of the chip); a column split is planned only if all its strips
+// fit in them (1: none is).
 int wf_build_plan(struct wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile,
                   WfPlanHost *ph, int64_t max_groups = 0);
 // Bytes from the splits to the cuts behind them.

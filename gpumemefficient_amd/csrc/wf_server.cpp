@@ -281,26 +281,30 @@ static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
     // The variant's share bounds an SW column split (the split's strips must
     // fit in the launch's workgroups, or the launch would go to the lock-step
     // engine below).
-    sl.ph = WfPlanHost();
     sl.ar.retired = &s->retired;
-    int st = wf_build_plan(s->ctx, jobs.data(), (int64_t)jobs.size(), nullptr, &sl.ph);
-    if (st != WF_OK) return st;
-    if (sl.ph.variant->engine == WF_ENGINE_ASYNC && !sl.ph.splits.empty() &&
-        (int64_t)sl.ph.tasks.size() > share(sl.ph.variant)) {
-        const int64_t cap = share(sl.ph.variant);
+    auto build = [&](int64_t cap, const wf_tile *tile) {
         sl.ph = WfPlanHost();
-        if ((st = wf_build_plan(s->ctx, jobs.data(), (int64_t)jobs.size(), nullptr, &sl.ph, cap)) != WF_OK)
-            return st;
-    }
-    // The asynchronous engine only pays off when all strips of the launch are
-    // resident within the slot's share of the chip; otherwise the lock-step
-    // engine's higher occupancy wins.
-    if (sl.ph.variant->engine == WF_ENGINE_ASYNC && (int64_t)sl.ph.tasks.size() > share(sl.ph.variant)) {
+        return wf_build_plan(s->ctx, jobs.data(), (int64_t)jobs.size(), tile, &sl.ph, cap);
+    };
+    auto too_many = [&] {
+        return sl.ph.variant->engine == WF_ENGINE_ASYNC && (int64_t)sl.ph.tasks.size() > share(sl.ph.variant);
+    };
+    auto plan = [&](bool split) {
+        int st = build(split ? 0 : 1, nullptr);
+        if (st == WF_OK && too_many() && !sl.ph.splits.empty()) st = build(share(sl.ph.variant), nullptr);
+        // The asynchronous engine only pays off when all strips of the launch are
+        // resident within the slot's share of the chip; otherwise the lock-step
+        // engine's higher occupancy wins.
         const wf_tile lock{0, 0, 0, WF_TILE_LOCKSTEP};
-        sl.ph = WfPlanHost();
-        if ((st = wf_build_plan(s->ctx, jobs.data(), (int64_t)jobs.size(), &lock, &sl.ph)) != WF_OK) return st;
+        if (st == WF_OK && too_many()) st = build(0, &lock);
+        return st == WF_OK ? wf_upload_plan_async(s->ctx, &sl.ph, &sl.ar, sl.stream, false) : st;
+    };
+    int st = plan(true);
+    if (st == WF_ERR_NOMEM && !sl.ph.splits.empty()) {  // (as plan_and_place in wf_api.cpp)
+        sl.ar.release();
+        st = plan(false);
     }
-    if ((st = wf_upload_plan_async(s->ctx, &sl.ph, &sl.ar, sl.stream, false)) != WF_OK) return st;
+    if (st != WF_OK) return st;
     const int maxg = share(sl.ph.variant);
     if ((st = wf_enqueue_plan(s->ctx, &sl.ph, &sl.ar, WF_RUN_PERSISTENT, maxg, sl.stream)) != WF_OK) return st;
     const int64_t n = sl.ph.npairs;

@@ -3,7 +3,8 @@ import ctypes as C
 
 import pytest
 
-from gpumemefficient_amd import _lib
+from fake_device import pair
+from gpumemefficient_amd import _lib, _server_abi
 
 # (n1, n2): narrow, wide and square tables.
 TABLES = [(1, 4_000_000), (13, 1_000_000), (100, 100_000), (511, 60_000), (512, 60_000), (600, 50_000), (4096, 65_536),
@@ -29,3 +30,44 @@ def test_sweep_memory_is_a_boundary_row_per_256_rows(fake, op, n1, n2):
     lib.wf_ctx_destroy(ctx)
     lib.fake_set_memory(1 << 40)
     assert st == _lib.WF_OK
+
+
+# (problem, n1, n2, symbols), the bytes that the pair needs unsplit and a little
+# more (a column split takes twice the rows, or half the codes again).
+SPLIT = [("SW", 20_000, 4000, 4, 7 * 20_000 * 8 + 300_000), ("SW", 20_000, 4000, 20, 7 * 20_000 * 8 + 300_000),
+         ("SW", 20_000, 80_000, 4, 156 * 20_000 * 8 + 1_000_000), ("LCS", 2_000_000, 3000, 4, 3_200_000)]
+
+
+@pytest.mark.parametrize("prob,n1,n2,k,room", SPLIT)
+def test_a_split_that_does_not_fit_is_left_out(fake, prob, n1, n2, k, room):
+    """A pair whose column split needs more memory than there is runs unsplit: a
+    call, a plan and a server's request that the unsplit pair fits succeed."""
+    lib = fake.c
+    job = pair(prob, n1, n2, k)
+    strips = -(-n2 // (512 if prob == "SW" else 2048))
+    tasks = C.c_int64()
+    for memory in (1 << 40, room):
+        ctx = C.c_void_p()
+        assert lib.wf_ctx_create(0, C.byref(ctx)) == 0
+        lib.fake_set_memory(memory)
+        out = _lib.wf_result()
+        lib.fake_tasks()
+        assert lib.wf_align_batch(ctx, fake.jobs([job]), 1, None, C.byref(out)) == _lib.WF_OK
+        n = lib.fake_tasks()
+        assert n == strips if memory == room else n > strips
+        lib.wf_ctx_destroy(ctx)
+        h = C.c_void_p()
+        assert lib.wf_plan_create(fake.ctx, fake.jobs([job]), 1, None, C.byref(h)) == _lib.WF_OK
+        lib.wf_plan_describe(h, None, None, None, None, C.byref(tasks), None)
+        assert tasks.value == n
+        lib.wf_plan_destroy(h)
+        opts = _server_abi.wf_server_opts(hbm_budget=1 << 30)
+        srv = C.c_void_p()
+        assert lib.wf_server_create(0, C.byref(opts), C.byref(srv)) == 0
+        assert lib.wf_server_submit(srv, fake.jobs([job]), None) == 0
+        assert lib.wf_server_wait_idle(srv, 20.0) == 0
+        done, got = (_server_abi.wf_completion * 1)(), C.c_int()
+        assert lib.wf_server_poll(srv, done, 1, C.byref(got)) == 0
+        lib.wf_server_destroy(srv)
+        assert got.value == 1 and done[0].status == _lib.WF_OK
+    lib.fake_set_memory(1 << 40)
