@@ -88,9 +88,10 @@ extern "C" int wf_align_noalloc(wf_ctx *ctx, int problem, const int32_t *a, int6
         return b.bnd <= kBndBytes && small <= kBndOff;
     };
     // A column-split SW pair needs 1.5 to 2 times the boundary rows of the
-    // pair: where the split does not fit and the pair does, it runs unsplit
-    // (a launch of one workgroup leaves no room for a split).
-    if (!fits_scratch(nb) && ph.variant->engine == WF_ENGINE_ASYNC && !ph.splits.empty()) {
+    // pair, and every split reversed codes: where the split does not fit and the
+    // pair does, it runs unsplit (a launch of one workgroup leaves no room for a
+    // split).
+    if (!fits_scratch(nb) && !ph.splits.empty()) {
         ph = WfPlanHost();
         if ((st = wf_build_plan(ctx, &j, 1, tile, &ph, 1)) != WF_OK) return st;
         wf_plan_bytes(&ph, &nb);

@@ -1,9 +1,10 @@
 """Device memory that the host code asks for, on a HIP runtime without a GPU."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
-from fake_device import pair
+from fake_device import i32, pair
 from gpumemefficient_amd import _lib, _server_abi
 
 # (n1, n2): narrow, wide and square tables.
@@ -71,3 +72,28 @@ def test_a_split_that_does_not_fit_is_left_out(fake, prob, n1, n2, k, room):
         lib.wf_server_destroy(srv)
         assert got.value == 1 and done[0].status == _lib.WF_OK
     lib.fake_set_memory(1 << 40)
+
+
+@pytest.mark.parametrize("prob", ["ED", "LCS"])
+def test_noalloc_takes_the_longest_pairs(fake, prob):
+    """Pairs up to the size whose codes, and those of a half of their columns
+    again, fill the 8 MiB of the scratch area: a half cut along a staircase is
+    longer, and then the pair runs unsplit."""
+    lib, n2 = fake.c, 2049
+
+    def small(n1):  # descriptors, last columns, codes of a pair cut at its middle
+        codes = sum((x + 15) // 16 * 16 for x in (n1, n2, n1 - n1 // 2, n2))
+        return 256 * 6 + 2 * 2 * 64 * 8 + (codes + 255) // 256 * 256
+
+    n1 = 5_000_000
+    while small(n1 + 1) <= 8 << 20:
+        n1 += 1
+    for n in (n1, n1 - 1500, 4000):
+        _, a, b, _ = pair(prob, n, n2)
+        out = _lib.wf_result()
+        st = lib.wf_align_noalloc(fake.ctx, _lib.PROBLEMS[prob], i32(a), a.size, i32(b), b.size, None, C.byref(out))
+        assert st == _lib.WF_OK, n
+    # (8 MiB of codes never fit.)
+    a = np.zeros(8 << 20, np.int32)
+    st = lib.wf_align_noalloc(fake.ctx, _lib.PROBLEMS[prob], i32(a), a.size, i32(b), b.size, None, C.byref(out))
+    assert st == _lib.WF_ERR_SCRATCH
