@@ -158,6 +158,7 @@ struct wf_server {
     wf_server_opts opts{};
     std::vector<Slot> slots;
     RetiredMem retired;                    // arenas the slots have outgrown, freed while no slot runs
+    int64_t retired_bytes = 0;             // their size, part of the budget
     std::thread sched;
     std::mutex mu;
     std::condition_variable cv;
@@ -327,10 +328,21 @@ static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
     return WF_OK;
 }
 
+// Frees what the slots have outgrown (`free_all`: no slot runs) and charges the
+// rest to the budget.
+static void charge_retired(wf_server *s, bool free_all)
+{
+    if (free_all && !s->retired.mem.empty()) s->retired.release();
+    if (s->retired_bytes == (int64_t)s->retired.bytes) return;  // (only the scheduler writes either)
+    std::lock_guard<std::mutex> lk(s->mu);
+    s->retired_bytes = (int64_t)s->retired.bytes;
+}
+
 static void scheduler(wf_server *s)
 {
     (void)hipSetDevice(s->ctx->device);
     const int strip_rows = 512;
+    auto running = [s] { return std::count_if(s->slots.begin(), s->slots.end(), [](const Slot &x) { return x.busy; }); };
     while (true) {
         bool did = false;
         // 1. completions
@@ -338,6 +350,7 @@ static void scheduler(wf_server *s)
             if (!sl.busy) continue;
             const hipError_t q = hipEventQuery(sl.done);
             if (q == hipSuccess) {
+                if (!s->retired.mem.empty() && running() == 1) charge_retired(s, true);
                 finish_slot(s, sl);
                 did = true;
             } else if (q != hipErrorNotReady) {
@@ -345,9 +358,7 @@ static void scheduler(wf_server *s)
                 s->error = WF_ERR_DEVICE;
             }
         }
-        if (!s->retired.mem.empty() &&
-            std::none_of(s->slots.begin(), s->slots.end(), [](const Slot &x) { return x.busy; }))
-            s->retired.release();
+        if (!s->retired.mem.empty() && running() == 0) charge_retired(s, true);
         // 2. admission by HBM budget, in arrival order
         {
             std::lock_guard<std::mutex> lk(s->mu);
@@ -366,7 +377,7 @@ static void scheduler(wf_server *s)
                     did = true;
                     continue;
                 }
-                if (s->used + r.bytes > s->budget) break;
+                if (s->used + s->retired_bytes + r.bytes > s->budget) break;
                 s->used += r.bytes;
                 s->admitted.push_back(std::move(r));
                 s->pending.pop_front();
@@ -402,7 +413,7 @@ static void scheduler(wf_server *s)
                 sl.alone = false;
                 if (first != s->admitted.end() && apart(*first)) {
                     // A split needs up to twice the boundary rows.
-                    sl.alone = s->used + first->bytes <= s->budget;
+                    sl.alone = s->used + s->retired_bytes + first->bytes <= s->budget;
                     if (sl.alone) {
                         s->used += first->bytes;
                         first->bytes *= 2;
@@ -425,6 +436,7 @@ static void scheduler(wf_server *s)
             const double t = s->now();
             for (Request &r : batch) r.t_start = t;
             const int st = launch_slot(s, sl, std::move(batch));
+            charge_retired(s, st != WF_OK && running() == 0);
             if (st != WF_OK) {
                 // The launch's requests fail with its status; only a HIP
                 // runtime error stops the server (requests are validated at
@@ -875,7 +887,7 @@ int wf_server_stats(wf_server *s, wf_server_stats_t *st)
     st->completed = s->completed;
     st->cells = s->cells;
     st->hbm_budget = s->budget;
-    st->hbm_used = s->used;
+    st->hbm_used = s->used + s->retired_bytes;
     st->pending = (int64_t)s->pending.size();
     return WF_OK;
 }

@@ -21,6 +21,7 @@ std::mutex g_mu;
 std::map<void *, size_t> g_mem;
 size_t g_live = 0, g_peak = 0, g_free = (size_t)288 << 30;
 std::atomic<bool> g_hold{false};
+std::atomic<int> g_release{0};  // counts fake_release() calls
 std::atomic<int> g_launches{0};
 std::atomic<int64_t> g_tasks{0};
 std::atomic<int> g_engine{-1};
@@ -38,8 +39,9 @@ void fake_set_memory(size_t bytes)
 }
 size_t fake_live() { return g_live; }
 size_t fake_peak() { return g_peak; }
-// While set, launches do not end.
+// While set, launches begin that do not end before fake_release().
 void fake_hold(int on) { g_hold = on != 0; }
+void fake_release() { ++g_release; }
 // Engine launches so far; the last one's engine, and the tasks of all.
 int fake_launches() { return g_launches; }
 int fake_last_engine() { return g_engine; }
@@ -141,17 +143,21 @@ hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e)
 {
-    *e = (hipEvent_t)::operator new(1);
+    *e = (hipEvent_t) new int(-1);
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e)
 {
-    ::operator delete((void *)e);
+    delete (int *)e;
     return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventQuery(hipEvent_t) { return g_hold ? hipErrorNotReady : hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t)
+{
+    *(int *)e = g_hold ? g_release.load() : -1;
+    return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) { return *(int *)e == g_release ? hipErrorNotReady : hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {
     *ms = 0.f;

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes as C
 import subprocess
+import time
 from pathlib import Path
 
 import numpy as np
@@ -35,7 +36,7 @@ class Fake:
         self.c = lib = C.CDLL(str(so))
         for name, res, args in [
                 ("fake_set_memory", None, [size]), ("fake_live", size, []), ("fake_peak", size, []),
-                ("fake_hold", None, [C.c_int]), ("fake_launches", C.c_int, []), ("fake_last_engine", C.c_int, []),
+                ("fake_hold", None, [C.c_int]), ("fake_release", None, []), ("fake_launches", C.c_int, []), ("fake_last_engine", C.c_int, []),
                 ("fake_tasks", i64, []), ("hipMalloc", C.c_int, [C.POINTER(P), size]), ("hipFree", C.c_int, [P]),
                 ("wf_ctx_create", C.c_int, [C.c_int, C.POINTER(P)]), ("wf_ctx_destroy", None, [P]),
                 ("wf_align_batch", C.c_int, [P, P, i64, P, P]),
@@ -57,6 +58,29 @@ class Fake:
             j.a, j.n1, j.b, j.n2 = i32(a), a.size, i32(b), b.size
         arr.keep = pairs
         return arr
+
+    def server(self, **opts):
+        h = C.c_void_p()
+        o = _server_abi.wf_server_opts(**opts)
+        assert self.c.wf_server_create(0, C.byref(o), C.byref(h)) == 0
+        return h
+
+    def submit(self, srv, job):
+        assert self.c.wf_server_submit(srv, self.jobs([job]), None) == 0
+
+    def stats(self, srv):
+        st = _server_abi.wf_server_stats_t()
+        assert self.c.wf_server_stats(srv, C.byref(st)) == 0
+        return st
+
+    def done(self, srv, n, limit=20.0):
+        """Statuses of n completions (fewer after `limit` seconds)."""
+        out, got, k, end = (_server_abi.wf_completion * n)(), [], C.c_int(), time.monotonic() + limit
+        while len(got) < n and time.monotonic() < end:
+            assert self.c.wf_server_poll(srv, out, n - len(got), C.byref(k)) == 0
+            got += [out[i].status for i in range(k.value)]
+            time.sleep(0.0005)
+        return got
 
     def plan(self, pairs):
         """(status, plan handle, tasks)."""
