@@ -265,6 +265,23 @@ static void finish_slot(wf_server *s, Slot &sl)
     s->cv.notify_all();
 }
 
+// Charges what the slot's split plan needs beyond the bytes of its requests (up to
+// as many boundary rows again, and its last columns) to the budget, until the
+// requests are done; false where that is more than is left.
+static bool charge_split(wf_server *s, Slot &sl)
+{
+    WfPlanBytes b;
+    wf_plan_bytes(&sl.ph, &b);
+    int64_t more = (int64_t)(b.codes + b.pairs + b.tasks + b.bnd + b.res + b.counters + b.epoch + b.colw + b.splits);
+    for (const Request &r : sl.reqs) more -= r.bytes;
+    if (more <= 0) return true;
+    std::lock_guard<std::mutex> lk(s->mu);
+    if (s->used + s->retired_bytes + more > s->budget) return false;
+    s->used += more;
+    sl.reqs[0].bytes += more;
+    return true;
+}
+
 static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
 {
     sl.reqs = std::move(batch);
@@ -297,13 +314,16 @@ static int launch_slot(wf_server *s, Slot &sl, std::vector<Request> &&batch)
         // resident within the slot's share of the chip; otherwise the lock-step
         // engine's higher occupancy wins.
         const wf_tile lock{0, 0, 0, WF_TILE_LOCKSTEP};
-        if (st == WF_OK && too_many()) st = build(0, &lock);
-        return st == WF_OK ? wf_upload_plan_async(s->ctx, &sl.ph, &sl.ar, sl.stream, false) : st;
+        return st == WF_OK && too_many() ? build(0, &lock) : st;
     };
+    auto upload = [&] { return wf_upload_plan_async(s->ctx, &sl.ph, &sl.ar, sl.stream, false); };
+    // A split runs where the budget and the device have the memory for it.
     int st = plan(true);
+    if (st == WF_OK && !sl.ph.splits.empty() && !charge_split(s, sl)) st = plan(false);
+    if (st == WF_OK) st = upload();
     if (st == WF_ERR_NOMEM && !sl.ph.splits.empty()) {  // (as plan_and_place in wf_api.cpp)
         sl.ar.release();
-        st = plan(false);
+        if ((st = plan(false)) == WF_OK) st = upload();
     }
     if (st != WF_OK) return st;
     const int maxg = share(sl.ph.variant);
@@ -412,12 +432,7 @@ static void scheduler(wf_server *s)
                 while (first != s->admitted.end() && apart(*first) && alone + 1 >= (int)s->slots.size()) ++first;
                 sl.alone = false;
                 if (first != s->admitted.end() && apart(*first)) {
-                    // A split needs up to twice the boundary rows.
-                    sl.alone = s->used + s->retired_bytes + first->bytes <= s->budget;
-                    if (sl.alone) {
-                        s->used += first->bytes;
-                        first->bytes *= 2;
-                    }
+                    sl.alone = true;
                     batch.push_back(std::move(*first));
                     s->admitted.erase(first);
                 } else if (first != s->admitted.end()) {
