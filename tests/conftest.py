@@ -15,6 +15,17 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: long-running")
 
 
+def pytest_collection_modifyitems(items):
+    # These compile driver sources of the reference, whose directory may be there
+    # and empty.
+    for item in items:
+        if getattr(item, "originalname", "") == "test_reference_driver_sources_link_against_compat_libs":
+            p = item.callspec.params
+            src = item.module.REF / p["pdir"] / f"GPU_Hyperlane_{p['kind']}.cpp"
+            if not src.is_file():
+                item.add_marker(pytest.mark.skip(reason=f"{src.name} of {p['pdir']} is not on this host"))
+
+
 @pytest.fixture(scope="session")
 def ctx():
     """One libwfdp context for the whole GPU session.  A missing library is an
