@@ -286,9 +286,10 @@ static const WfVariant *find_variant(int E, int R, int W, int K)
 // the WFDP_VARIANT environment override ("engine,R,W,K"), the autotuned
 // table (wf_tune.cpp) for this workload and device, built-in defaults.
 // strip_rows = 64 * waves * rows_per_lane; tile_w maps to the chunk (the
-// lock-step barrier interval, or the async progress interval).
-const WfVariant *wf_pick_variant(wf_ctx *ctx, const wf_tile *tile, const wf_job *jobs, int64_t njobs,
-                                 int64_t max_rows, int64_t total_cells)
+// lock-step barrier interval, or the async progress interval).  tuned: may take
+// the table's.
+static const WfVariant *pick_variant(wf_ctx *ctx, const wf_tile *tile, const wf_job *jobs, int64_t njobs,
+                                     int64_t max_rows, int64_t total_cells, bool tuned)
 {
     int E = WF_ENGINE_LOCKSTEP, R = 0, W = 0, K = 0;
     if (const char *env = std::getenv("WFDP_VARIANT")) {
@@ -311,7 +312,7 @@ const WfVariant *wf_pick_variant(wf_ctx *ctx, const wf_tile *tile, const wf_job 
     const int32_t engine_flags = WF_TILE_LOCKSTEP | WF_TILE_ASYNC | WF_TILE_BITPAR | WF_TILE_BITPAR_STAGED;
     const bool explicit_tile = tile && (tile->tile_w > 0 || tile->strip_rows > 0 || tile->rows_per_lane > 0 ||
                                         (tile->flags & engine_flags));
-    if (!explicit_tile && !cache && ctx) {
+    if (tuned && !explicit_tile && !cache && ctx) {
         int p, b, bk, te, tr, tw, tk;
         wf_tune_key(jobs, njobs, &p, &b, &bk);
         if (wf_tune_lookup(ctx->prop.gcnArchName, ctx->prop.multiProcessorCount, p, b, bk, &te, &tr, &tw, &tk)) {
@@ -504,8 +505,8 @@ static std::vector<int32_t> bitpar_cuts(int64_t n1, int64_t n2, int64_t strip)
     return c;
 }
 
-int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile,
-                  WfPlanHost *ph, int64_t max_groups)
+static int build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile, WfPlanHost *ph,
+                      int64_t max_groups, bool tuned)
 {
     int64_t max_rows = 0, total_cells = 0;
     for (int64_t i = 0; i < njobs; ++i) {
@@ -516,7 +517,7 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
         if (j.n1 > 0 && j.n2 > 0) max_rows = std::max(max_rows, j.n2);
         total_cells += j.n1 * j.n2;
     }
-    const WfVariant *v = wf_pick_variant(ctx, tile, jobs, njobs, max_rows, total_cells);
+    const WfVariant *v = pick_variant(ctx, tile, jobs, njobs, max_rows, total_cells, tuned);
     if (!v) return WF_ERR_NOKERNEL;
     ph->variant = v;
     const int64_t strip = 64LL * v->waves * v->rows_per_lane;
@@ -920,6 +921,17 @@ int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile 
     ph->bnd_ints = bnd_ints;
     ph->order = order;
     return WF_OK;
+}
+
+// The tuned table knows a pair's size, not its symbols: LCS and ED pairs of more
+// than 32, which its bit-parallel variants cannot run, take the built-in choice.
+int wf_build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_tile *tile, WfPlanHost *ph,
+                  int64_t max_groups)
+{
+    const int st = build_plan(ctx, jobs, njobs, tile, ph, max_groups, true);
+    if (st != WF_ERR_NOKERNEL) return st;
+    *ph = WfPlanHost();
+    return build_plan(ctx, jobs, njobs, tile, ph, max_groups, false);
 }
 
 int wf_upload_plan(wf_ctx *ctx, WfPlanHost *ph, WfArenas *ar)

@@ -144,8 +144,6 @@ int wf_encode_job(const wf_job &j, int32_t tile_flags, bool perm4, uint8_t *a_ou
 int32_t wf_empty_score(int problem, int64_t n1, int64_t n2, int flags);
 // Byte row tables for SW on cell engines with two rows per lane (WFDP_PERM=0: off).
 bool wf_perm4_enabled();
-const WfVariant *wf_pick_variant(struct wf_ctx *ctx, const wf_tile *tile, const wf_job *jobs, int64_t njobs,
-                                 int64_t max_rows, int64_t total_cells);
 void wf_tune_key(const wf_job *jobs, int64_t njobs, int *problem, int *batch, int *bucket);
 // Load the autotune table shipped with the library (once per process).
 void wf_tune_autoload();

@@ -8,7 +8,7 @@
 //   class "batch":  several pairs, bucket = floor(log2(mean cells per pair))
 // The table is a small text file (one entry per line, '#' comments):
 //   <arch> <cus> <problem> <class> <bucket> <engine> <rows_per_lane> <waves> <chunk> <ms>
-// wf_pick_variant() consults it before the built-in defaults.
+// The planner consults it before the built-in defaults.
 #include <dlfcn.h>
 #include <hip/hip_runtime.h>
 

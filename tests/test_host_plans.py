@@ -27,3 +27,22 @@ def test_a_pairs_parts_share_its_launch(fake, prob, n1, n2, k, parts):
         assert fake.c.fake_launches() - before == len(todo) + 1
         assert fake.c.fake_tasks() == tasks
         fake.c.wf_plan_destroy(plan)
+
+
+@pytest.mark.parametrize("prob,n1,n2", [("LCS", 3000, 4096), ("ED", 2000, 20_000), ("ED", 1000, 1000)])
+def test_large_alphabets_beside_a_tuned_bit_parallel_entry(fake, tmp_path, prob, n1, n2):
+    """A tuned entry is looked up by size: a pair of more symbols than its engine
+    takes runs on the built-in choice, as a pair without an entry does."""
+    table = tmp_path / "tune.txt"
+    table.write_text("none 256 1 single 14 3 32 1 64 1.0\nnone 256 0 single 12 3 32 1 64 0.1\n"
+                     "none 256 1 single 9 2 32 1 64 1.0\n")
+    job = pair(prob, n1, n2, k=33)
+    for _ in range(2):  # without the entries, with them
+        st, plan, tasks = fake.plan([job])
+        assert st == 0 and tasks == -(-n2 // 512)
+        fake.c.wf_plan_destroy(plan)
+        assert fake.c.wf_tune_load(str(table).encode()) == 0
+    st, plan, tasks = fake.plan([pair(prob, n1, n2, k=32)])
+    assert st == 0 and tasks <= 2 * -(-n2 // 2048)
+    fake.c.wf_plan_destroy(plan)
+    fake.c.wf_tune_clear()
