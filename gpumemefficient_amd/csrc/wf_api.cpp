@@ -468,12 +468,8 @@ constexpr int64_t kSplitMinColsEd = 576, kSplitMinColsLcs = 832;
 // SW pairs narrower than this are not split (measured gains of the split:
 // 13% at 1024 x 1024, 17% at 2048 x 2048, 30% at 3000 x 600).
 constexpr int64_t kSwSplitMinCols = 1024;
-// Narrowest pair without the maximum that is split in two parts (without f0,
-// WfSplitDev) and not in three where three have more strips than the chip has CUs
-// (ms in two / three parts: 90 strips, 24000 columns 1.02 / 0.99, 98304 1.89 /
-// 1.86; 128 strips, 16384 columns 1.14 / 1.13, 65536 1.77 / 1.73, 98304 2.20 /
-// 2.27, 131072 2.60 / 2.98; 170 strips, 10000 columns 1.41 / 1.38, 49152 1.86 /
-// 1.81, 65536 2.07 / 2.23, 98304 2.60 / 3.46: within 4% up to 65536 columns).
+// Narrowest pair that is split in two or three parts (without f0, WfSplitDev)
+// where three or four have more strips than the chip has CUs.
 constexpr int64_t kSwTwoPartMinCols = 16384;
 
 // Columns where the strips of a column-split SW pair are cut (WfSplitDev):
@@ -583,29 +579,26 @@ static int build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_t
             extra += cand[i] * si;
         }
         // Three or four parts while every strip has a CU of its own.  Beyond
-        // that, a launch of one pair takes two or three parts, whose strips
-        // share CUs only towards the end, at any width that is split at all
-        // (no maximum: 131072^2 4.74 ms, unsplit 6.55; 2000 columns x 180
-        // strips 1.50, unsplit 2.84; 1024 x 256 strips 1.83, unsplit 3.41; with
-        // it: 65536^2 2.02, unsplit 3.62; 10000 x 90 strips 0.90, unsplit 1.72;
-        // 1024 x 65 strips 0.53, unsplit 1.01, x 170 strips 1.33 and 2.59; 20
-        // symbols likewise), and one without the maximum three parts while they
-        // fit and it is not wide (kSwTwoPartMinCols).  A batch, whose strips all
-        // run at once, is not split beyond a strip per CU (16 pairs of 4096^2,
-        // 384 strips: 0.27 ms against 0.21 unsplit).
+        // that, a launch of one wide pair takes two or three parts, whose
+        // strips share CUs only towards the end (no maximum: 131072 x 65536
+        // 2.60 ms against 2.98 in three parts and 4.47 with a straight cut;
+        // 131072^2 4.74 against 6.55 unsplit; with it: 65536^2 2.02 against
+        // 3.62 unsplit), and a narrow one without the maximum three parts
+        // (4096 x 44032, 258 strips: 0.66 ms, unsplit 1.24).  A batch, whose
+        // strips all run at once, is not split beyond a strip per CU (16 pairs
+        // of 4096^2, 384 strips: 0.27 ms against 0.21 unsplit).
         const bool four = std::find(cand.begin(), cand.end(), 3) != cand.end();
         const int64_t cus = ctx ? ctx->prop.multiProcessorCount : 256;
         const int64_t resident = std::min(ctx ? (int64_t)wf_max_resident_groups(ctx, v) : 256,
                                           max_groups > 0 ? max_groups : INT64_MAX);
-        const bool one = njobs == 1 && cand[0];
-        const bool wide = one && jobs[0].n1 >= kSwTwoPartMinCols;
+        const bool wide = njobs == 1 && cand[0] && jobs[0].n1 >= kSwTwoPartMinCols;
         if (extra > 0 && strips + extra <= std::min(resident, (four || njobs > 1 || wide) ? cus : INT64_MAX)) {
             for (int64_t i = 0; i < njobs; ++i)
                 if (cand[i]) {
                     swsplit[i] = cand[i];
                     nextra += cand[i];
                 }
-        } else if (one && cand[0] * strips <= resident) {
+        } else if (wide && cand[0] * strips <= resident) {
             swsplit[0] = cand[0];
             two_part = true;
             nextra = cand[0] - 1;
