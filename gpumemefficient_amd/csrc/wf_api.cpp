@@ -469,7 +469,16 @@ constexpr int64_t kSplitMinColsEd = 576, kSplitMinColsLcs = 832;
 // 13% at 1024 x 1024, 17% at 2048 x 2048, 30% at 3000 x 600).
 constexpr int64_t kSwSplitMinCols = 1024;
 // Narrowest pair that is split in two or three parts (without f0, WfSplitDev)
-// where three or four have more strips than the chip has CUs.
+// where three or four have more strips than the chip has CUs.  With the maximum
+// the line does not lie where the gain ends: three parts halve the time of narrower
+// pairs too (ms in one part / three: 1024 x 65 strips 1.01 / 0.53, 10000 x 90
+// 1.72 / 0.90, 16384 x 130 2.38 / 1.25), which stay in one part, as test_sw_split_*
+// has it.  Without it (ms in three parts / two) two are the better ones from
+// about 65536 columns on and within 4% below: 128 strips, 16384 columns 1.13 / 1.14,
+// 65536 1.73 / 1.77, 98304 2.27 / 2.20, 131072 2.98 / 2.60; 170 strips, 16384
+// columns 1.38 / 1.43, 49152 1.81 / 1.86, 65536 2.23 / 2.07, 98304 3.46 / 2.60.
+// Narrower ones of more strips than three parts have room for stay in one part
+// too (2000 x 180 strips 2.84 ms, in two 1.50).
 constexpr int64_t kSwTwoPartMinCols = 16384;
 
 // Columns where the strips of a column-split SW pair are cut (WfSplitDev):
