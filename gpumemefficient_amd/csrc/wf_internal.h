@@ -117,7 +117,7 @@ struct WfPlanHost {
     int64_t njobs = 0;   // result slots 0..njobs-1
     int64_t npairs = 0;  // njobs plus the reverse halves of split pairs
     std::vector<WfSplitDev> splits;
-    std::vector<WfCutDev> cuts;  // columns of the strips of SW splits' pairs; device: behind the splits
+    std::vector<WfCutDev> cuts;  // columns of the strips of pairs cut along a staircase; device: behind the splits
     int64_t colw_entries = 0;
     const WfVariant *variant = nullptr;
     std::vector<WfPairDev> pairs;

@@ -14,7 +14,9 @@
 // Requests that arrive while others run are admitted and launched on the
 // next free slot, so their work overlaps on the device with the launches
 // already running.  Each launch's grid is capped at 1/S of the resident
-// capacity so a large request cannot starve the other slots.
+// capacity so a large request cannot starve the other slots, except a launch
+// of one long request (is_long), which may take the chip: its strips run
+// beside the other slots' (at least one slot is left to them).
 //
 // Resident mode (wf_server_opts.resident) replaces the slots with one
 // persistent launch of the lock-step engine that lives as long as the
@@ -217,11 +219,17 @@ static bool alphabet_fits(const wf_job *job)
 // runs on the asynchronous (LCS, ED: staged bit-parallel) engine, while the
 // other slots run the rest.  The lines lie where the chain costs about 2.5 ms
 // in a shared launch (lock-step SW 35 ns for each of n1 + 1.5 n2 steps, plain
-// bit-parallel 45 ns a column).
-static bool is_long(const Request &r)
+// bit-parallel 45 ns a column).  Not LCS and ED over more than 32 symbols: the
+// cell engines do not split them, and one alone takes what the shared launch
+// does (65536^2, 64 letters, 3.8 ms either way; three of them 5.9 and 7.3).  Nor
+// pairs of more 512-row strips than CUs: SW then runs in one part with two
+// strips on a CU, and several are in each other's way (with 150 short ones, apart
+// / shared: one 20000 x 200000 7.2 / 9.3 ms, three 10.8 / 12.2; one 4000 x 250000 9.0
+// / 10.7, three 13.4 / 11.8).
+static bool is_long(const Request &r, int cus)
 {
     const int64_t n1 = (int64_t)r.a.size(), n2 = (int64_t)r.b.size();
-    if (n2 == 0 || n2 > 512 * 256) return false;  // more strips than the asynchronous engine is chosen for
+    if (n2 == 0 || n2 > 512LL * cus) return false;
     return r.bitpar ? n1 >= 49152 : r.problem == WF_SW && n1 + n2 + n2 / 2 >= 65536;
 }
 // Long requests, waiting or running, up to which each runs alone; with more of
@@ -861,7 +869,7 @@ int wf_server_submit(wf_server *s, const wf_job *job, uint64_t *ticket)
     r.b.assign(job->b, job->b + job->n2);
     r.bytes = request_bytes(job->n1, job->n2, 512);
     r.bitpar = wf_bitpar_eligible(job, 1);
-    r.is_long = is_long(r);
+    r.is_long = is_long(r, s->ctx->prop.multiProcessorCount);
     std::lock_guard<std::mutex> lk(s->mu);
     if ((int64_t)s->pending.size() >= s->opts.queue_capacity) return WF_ERR_AGAIN;
     r.ticket = s->next_ticket++;

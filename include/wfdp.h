@@ -156,11 +156,11 @@ int wf_align(wf_ctx *ctx, int problem, const int32_t *a, int64_t n1, const int32
  * process ends; the caller passes the same host inputs and output as to
  * wf_align().  Pairs whose strip boundaries or codes do not fit return
  * WF_ERR_SCRATCH (roughly: (n2 / strip_rows - 1) * n1 * 8 bytes of boundary
- * rows, a sixteenth of it for bit-parallel pairs, within 56 MiB, and n1 + n2
- * bytes of codes within 8 MiB; 16384 x 16384
- * SW fits; a pair whose column split would not fit runs unsplit).  All calls on one GPU share that GPU's array, and calls that
- * overlap on one GPU (several threads or contexts) race: the caller
- * serialises them. */
+ * rows, a sixteenth of it on the staged bit-parallel engine, within 56 MiB,
+ * and n1 + n2 bytes of codes within 8 MiB; 16384 x 16384 SW fits; a pair whose
+ * column split would not fit runs unsplit).  All calls on one GPU share that
+ * GPU's array, and calls that overlap on one GPU (several threads or contexts)
+ * race: the caller serialises them. */
 #define WF_NOALLOC_SCRATCH_BYTES (64LL << 20)
 int wf_align_noalloc(wf_ctx *ctx, int problem, const int32_t *a, int64_t n1, const int32_t *b,
                      int64_t n2, const wf_tile *tile, wf_result *out);
@@ -288,7 +288,8 @@ typedef struct wf_server wf_server;
 typedef struct {
     int32_t streams;        /* concurrent launches (HIP streams); 0 = 4 */
     int32_t max_batch;      /* requests per launch; 0 = 512 */
-    int64_t hbm_budget;     /* device bytes the server may hold; 0 = half of free memory */
+    int64_t hbm_budget;     /* device bytes that requests from their admission to their completion, and
+                             * buffers outgrown meanwhile, may take; 0 = half of free memory */
     int32_t queue_capacity; /* queued requests before submit returns WF_ERR_AGAIN; 0 = 2^20 */
     int32_t per_request;    /* 1: one launch per request on one stream (baseline) */
     int32_t resident;       /* 1: one persistent launch for the server's lifetime: requests
