@@ -902,30 +902,37 @@ static int build_plan(wf_ctx *ctx, const wf_job *jobs, int64_t njobs, const wf_t
     // 131072^2, 512 strips: 4.74 ms, part by part 5.88).  The other splits' go
     // part by part: their f0 strips all start at once (65536^2, 384 strips:
     // 1.74 ms part by part, 2.94 strip by strip).
-    std::vector<std::vector<int32_t>> parts(np);
-    std::vector<int64_t> owner(np);
-    std::iota(owner.begin(), owner.end(), 0);
-    for (int64_t i = 0; i < np; ++i) parts[i].push_back((int32_t)i);
-    for (const WfSplitDev &sp : ph->splits)
-        for (int32_t p : {sp.prob == WFK_SW ? sp.f0 : -1, sp.rev, sp.crev})
-            if (p >= 0) {
-                parts[sp.job].push_back(p);
-                owner[p] = sp.job;
-            }
+    std::vector<int32_t> split_of(ph->splits.empty() ? 0 : np, -1);  // -2: in the list with the part that came first
+    for (size_t k = 0; k < ph->splits.size(); ++k) {
+        const WfSplitDev &sp = ph->splits[k];
+        for (int32_t p : {sp.job, sp.prob == WFK_SW ? sp.f0 : -1, sp.rev, sp.crev})
+            if (p >= 0) split_of[p] = (int32_t)k;
+    }
     for (int64_t k = 0; k < np; ++k) {
-        const int64_t i = owner[order[k]];
-        if (parts[i].empty()) continue;  // with the part that came first
+        int64_t i = order[k];
+        int32_t part[4] = {(int32_t)i};
+        int parts = 1;
+        if (!split_of.empty() && split_of[i] != -1) {
+            if (split_of[i] == -2) continue;
+            const WfSplitDev &sp = ph->splits[split_of[i]];
+            parts = 0;
+            for (int32_t p : {sp.job, sp.prob == WFK_SW ? sp.f0 : -1, sp.rev, sp.crev})
+                if (p >= 0) {
+                    split_of[p] = -2;
+                    part[parts++] = p;
+                }
+            i = sp.job;
+        }
         ph->task_begin[i] = (int64_t)ph->tasks.size();
         const int32_t ng = ph->pairs[i].ngroups;  // (the same in all parts)
         if (two_part) {
             for (int32_t g = 0; g < ng; ++g)
-                for (int32_t p : parts[i]) ph->tasks.push_back(WfTaskDev{p, g});
+                for (int p = 0; p < parts; ++p) ph->tasks.push_back(WfTaskDev{part[p], g});
         } else {
-            for (int32_t p : parts[i])
-                for (int32_t g = 0; g < ng; ++g) ph->tasks.push_back(WfTaskDev{p, g});
+            for (int p = 0; p < parts; ++p)
+                for (int32_t g = 0; g < ng; ++g) ph->tasks.push_back(WfTaskDev{part[p], g});
         }
         ph->task_end[i] = (int64_t)ph->tasks.size();
-        parts[i].clear();
     }
     ph->bnd_ints = bnd_ints;
     ph->order = order;
