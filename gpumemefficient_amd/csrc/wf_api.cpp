@@ -974,14 +974,16 @@ int wf_copy_plan(WfPlanHost *ph, WfArenas *ar, hipStream_t stream)
     if (hipMemcpyAsync(ar->codes.ptr, ph->codes.data(), ph->codes.size(), hipMemcpyHostToDevice,
                        stream) != hipSuccess)
         return WF_ERR_DEVICE;
-    if (!ph->splits.empty() &&
-        hipMemcpyAsync(ar->splits.ptr, ph->splits.data(), ph->splits.size() * sizeof(WfSplitDev),
-                       hipMemcpyHostToDevice, stream) != hipSuccess)
-        return WF_ERR_DEVICE;
-    if (!ph->cuts.empty() &&
-        hipMemcpyAsync((uint8_t *)ar->splits.ptr + wf_cuts_offset(ph), ph->cuts.data(),
-                       ph->cuts.size() * sizeof(WfCutDev), hipMemcpyHostToDevice, stream) != hipSuccess)
-        return WF_ERR_DEVICE;
+    // Splits and cuts in one copy (a copy is about 8 us of a request's latency).
+    if (!ph->splits.empty()) {
+        const size_t at = wf_cuts_offset(ph), cuts = ph->cuts.size() * sizeof(WfCutDev);
+        ph->split_block.assign(at + cuts, 0);
+        std::memcpy(ph->split_block.data(), ph->splits.data(), ph->splits.size() * sizeof(WfSplitDev));
+        if (cuts) std::memcpy(ph->split_block.data() + at, ph->cuts.data(), cuts);
+        if (hipMemcpyAsync(ar->splits.ptr, ph->split_block.data(), at + cuts, hipMemcpyHostToDevice, stream) !=
+            hipSuccess)
+            return WF_ERR_DEVICE;
+    }
     if (!ph->pairs.empty() &&
         hipMemcpyAsync(ar->pairs.ptr, ph->pairs.data(), ph->pairs.size() * sizeof(WfPairDev),
                        hipMemcpyHostToDevice, stream) != hipSuccess)

@@ -118,6 +118,7 @@ struct WfPlanHost {
     int64_t npairs = 0;  // njobs plus the reverse halves of split pairs
     std::vector<WfSplitDev> splits;
     std::vector<WfCutDev> cuts;  // columns of the strips of pairs cut along a staircase; device: behind the splits
+    std::vector<uint8_t> split_block;  // both as wf_copy_plan lays them out
     int64_t colw_entries = 0;
     const WfVariant *variant = nullptr;
     std::vector<WfPairDev> pairs;
