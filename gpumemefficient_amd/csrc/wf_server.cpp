@@ -238,7 +238,10 @@ static bool is_long(const Request &r, int cus)
 // for one in a shared launch; ED 65536^2: 1.3 ms alone, 3.2 in a shared one).
 constexpr int kFewLongSw = 3, kFewLongBitpar = 6;
 
-static void finish_slot(wf_server *s, Slot &sl)
+// last: no other slot runs, so what the slots have outgrown is freed next, before
+// anything is admitted: it counts no longer (freeing takes longer than many
+// launches, so the completions do not wait for it).
+static void finish_slot(wf_server *s, Slot &sl, bool last)
 {
     std::vector<wf_completion> out;
     out.reserve(sl.reqs.size());
@@ -264,6 +267,7 @@ static void finish_slot(wf_server *s, Slot &sl)
         s->used -= sl.reqs[i].bytes;
         s->cells += (uint64_t)(sl.reqs[i].a.size() * sl.reqs[i].b.size());
     }
+    if (last) s->retired_bytes = 0;
     s->inflight -= (int64_t)sl.reqs.size();
     s->completed += sl.reqs.size();
     s->done.insert(s->done.end(), out.begin(), out.end());
@@ -378,8 +382,7 @@ static void scheduler(wf_server *s)
             if (!sl.busy) continue;
             const hipError_t q = hipEventQuery(sl.done);
             if (q == hipSuccess) {
-                if (!s->retired.mem.empty() && running() == 1) charge_retired(s, true);
-                finish_slot(s, sl);
+                finish_slot(s, sl, running() == 1);
                 did = true;
             } else if (q != hipErrorNotReady) {
                 std::lock_guard<std::mutex> lk(s->mu);

@@ -4,6 +4,7 @@
 // records its engine and its tasks and computes nothing; allocations can be made
 // to fail and launches to last.
 #include <hip/hip_runtime.h>
+#include <sched.h>
 #include <sys/mman.h>
 
 #include <algorithm>
@@ -22,6 +23,7 @@ std::map<void *, size_t> g_mem;
 size_t g_live = 0, g_peak = 0, g_free = (size_t)288 << 30;
 std::atomic<bool> g_hold{false};
 std::atomic<int> g_release{0};  // counts fake_release() calls
+std::atomic<bool> g_free_hold{false};
 std::atomic<int> g_launches{0};
 std::atomic<int64_t> g_tasks{0};
 std::atomic<int> g_engine{-1};
@@ -42,6 +44,8 @@ size_t fake_peak() { return g_peak; }
 // While set, launches begin that do not end before fake_release().
 void fake_hold(int on) { g_hold = on != 0; }
 void fake_release() { ++g_release; }
+// While set, hipFree does not return.
+void fake_free_hold(int on) { g_free_hold = on != 0; }
 // Engine launches so far; the last one's engine, and the tasks of all.
 int fake_launches() { return g_launches; }
 int fake_last_engine() { return g_engine; }
@@ -62,6 +66,7 @@ hipError_t hipMalloc(void **p, size_t n)
 }
 hipError_t hipFree(void *p)
 {
+    while (g_free_hold) sched_yield();
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_mem.find(p);
     if (it == g_mem.end()) return hipErrorInvalidValue;

@@ -36,7 +36,7 @@ class Fake:
         self.c = lib = C.CDLL(str(so))
         for name, res, args in [
                 ("fake_set_memory", None, [size]), ("fake_live", size, []), ("fake_peak", size, []),
-                ("fake_hold", None, [C.c_int]), ("fake_release", None, []), ("fake_launches", C.c_int, []), ("fake_last_engine", C.c_int, []),
+                ("fake_hold", None, [C.c_int]), ("fake_free_hold", None, [C.c_int]), ("fake_release", None, []), ("fake_launches", C.c_int, []), ("fake_last_engine", C.c_int, []),
                 ("fake_tasks", i64, []), ("hipMalloc", C.c_int, [C.POINTER(P), size]), ("hipFree", C.c_int, [P]),
                 ("wf_ctx_create", C.c_int, [C.c_int, C.POINTER(P)]), ("wf_ctx_destroy", None, [P]),
                 ("wf_align_batch", C.c_int, [P, P, i64, P, P]),

@@ -87,3 +87,31 @@ def test_long_bit_parallel_requests_are_charged_once(fake):
     assert tasks == 2 * 5
     assert used <= _rows(50_000, 10_000) + 100_000
     fake.c.wf_server_destroy(srv)
+
+
+def test_completions_do_not_wait_for_outgrown_arenas_to_be_freed(fake):
+    """Freeing what slots have outgrown waits for the device: the last launch's
+    requests are done before it begins (and count no longer), and nothing is
+    admitted until it has ended."""
+    lib = fake.c
+    srv = fake.server(streams=2, hbm_budget=1 << 30)
+    lib.fake_hold(1)
+    fake.submit(srv, pair("SW", 300, 200))
+    while fake.stats(srv).launches < 1:
+        pass
+    lib.fake_hold(0)
+    for n1, n2 in [(900, 20_000), (900, 40_000)]:
+        fake.submit(srv, pair("SW", n1, n2))
+        assert fake.done(srv, 1) == [OK]
+    assert fake.stats(srv).hbm_used > _rows(900, 20_000)
+    lib.fake_free_hold(1)
+    lib.fake_release()
+    assert fake.done(srv, 1, 5.0) == [OK]
+    assert lib.wf_server_wait_idle(srv, 5.0) == OK
+    assert fake.stats(srv).hbm_used == 0
+    fake.submit(srv, pair("SW", 900, 700))
+    time.sleep(0.05)
+    assert fake.stats(srv).launches == 3
+    lib.fake_free_hold(0)
+    assert fake.done(srv, 1) == [OK]
+    lib.wf_server_destroy(srv)
