@@ -321,8 +321,8 @@ static const WfVariant *pick_variant(wf_ctx *ctx, const wf_tile *tile, const wf_
     }
     // LCS and ED pairs with at most 32 symbols go to the bit-parallel engine
     // (32 rows per lane word) unless a cell engine is asked for: its chain of
-    // waves down a pair is 32 times shorter and a column step costs about
-    // 20 VALU operations for 32 cells.
+    // waves down a pair is 32 times shorter and a column step costs 7 (LCS) to
+    // 15 (ED) VALU operations for 32 cells.
     const bool cell_flags = tile && (tile->flags & (WF_TILE_LOCKSTEP | WF_TILE_ASYNC | WF_TILE_CACHE));
     const int32_t bp_flags = WF_TILE_BITPAR | WF_TILE_BITPAR_STAGED;
     const bool want_bitpar = (tile && ((tile->flags & bp_flags) || tile->rows_per_lane == 32)) ||
@@ -345,9 +345,10 @@ static const WfVariant *pick_variant(wf_ctx *ctx, const wf_tile *tile, const wf_
                 if (jobs[i].n1 > 0 && jobs[i].n2 > 0) strips += (jobs[i].n2 + 2047) / 2048;
             staged = strips <= (ctx ? ctx->prop.multiProcessorCount : 256);
         }
-        // Strip height, measured on ED 65536^2: staged, one compute wave
-        // (2.75 ms; W = 2 3.14); plain, two waves (3.23 ms; W = 1 3.68,
-        // W = 4 3.32; K = 128 3.39).  Likewise for LCS 8192^2.
+        // Strip height, measured on ED 65536^2, unsplit: staged, one compute
+        // wave (2.30 ms; W = 2 2.46); plain, two waves (3.29 ms; W = 1 3.46,
+        // W = 4 3.34; K = 128 3.30).  LCS 8192^2: 0.162 (0.249); 0.297 (0.345,
+        // 0.331; 0.299).
         if (Wb == 0) Wb = staged ? 1 : (max_rows > 2048 ? 2 : 1);
         const int Eb = staged ? WF_ENGINE_BITPAR_STAGED : WF_ENGINE_BITPAR;
         const WfVariant *best = nullptr;

@@ -12,7 +12,7 @@
 //        matching based on dynamic programming", J. ACM 46(3), section 4:
 //        state Pv/Mv (vertical +1/-1), horizontal deltas Ph/Mh; the word
 //        above passes its last row's horizontal delta (hin) down, and a -1
-//        enters the carry chain of the addition as Eq | 1.
+//        enters the carry chain of the addition (in place of Eq | 1).
 //   LCS  the bit-vector LCS of Crochemore, Iliopoulos, Pinzon and Reid (2001)
 //        "A fast and practical bit-vector algorithm for the longest common
 //        subsequence problem", IPL 80(6): V' = (V + (V & Eq)) | (V & ~Eq);
@@ -23,8 +23,8 @@
 // start.  The words of a wave form the same 64-lane systolic array as the
 // cell engines (lane l handles column s - l at step s; the word above's
 // output reaches lane l through one DPP wave_shr:1), so a wave covers 2048
-// rows and a column step costs about 20 VALU operations for 32 cells instead
-// of 3-4 per cell.  The chain of waves down a pair is 32 times shorter than
+// rows and a column step costs 7 (LCS, staged) to 15 (ED) VALU operations for
+// 32 cells instead of 3-4 per cell.  The chain of waves down a pair is 32 times shorter than
 // the cell engines' (one wave per 2048 rows instead of per 128), which is
 // where a single large pair spends half its time there.
 //
